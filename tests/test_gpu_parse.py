@@ -82,3 +82,27 @@ def test_parse_golden_inputs_and_rmat20(dev):
 def test_parse_refuses_malformed(dev, bad):
     with pytest.raises(dev.GchiError, match="FORMAT|format|fields"):
         dev.parse_edgelist(bad)
+
+
+@pytest.mark.parametrize("shift", [0, 1, 15])
+@pytest.mark.parametrize("length", [4, 127, 128, 129, 130, 1000, 1022])
+def test_parse_lines_across_chunk_ends(dev, length, shift):
+    """A line of each length starting 1..130 bytes before a 4 KiB chunk's end
+    (its LDS window ends 128 bytes past the chunk), an edge line and a comment,
+    the text at an unaligned device address, ended with and without a newline."""
+    import torch
+    for back in (1, 2, 63, 64, 65, 130):
+        for head in ("1 2", "#  "):
+            fill = 4096 - back
+            lead = "10 11\n" * (fill // 6 - 1)
+            lead += "7 8" + " " * (fill - len(lead) - 4) + "\n"
+            line = head + " " * (length - 3)
+            body = lead + line + "\n" + "3 4\n" * 2000 + line
+            for tail in ("", "\n"):
+                text = (body + tail).encode()
+                buf = torch.from_numpy(np.frombuffer(b"\n" * shift + text, np.uint8).copy()).to("cuda")
+                s, d, n, mx = dev.parse_edgelist(buf[shift:])
+                ws, wd = oracle.parse_edgelist(text)
+                assert n == len(ws) and mx == 11
+                np.testing.assert_array_equal(dev.to_host_u32(s, n), ws)
+                np.testing.assert_array_equal(dev.to_host_u32(d, n), wd)
