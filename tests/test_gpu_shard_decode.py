@@ -121,3 +121,59 @@ def test_decode_many_streams_in_one_call(dev):
     bad = d[:2] + [(to_dev_u8(dev, streams[0][:-1]), len(streams[0]) - 1)]
     with pytest.raises(dev.GchiError):
         dev.shard_decode_many(bad)
+
+
+def _stream(rng, nbytes, kinds):
+    """A valid stream of about nbytes bytes whose record lengths are drawn from
+    `kinds` (0 = a zero run), with words that look like headers at any phase."""
+    out, size = [], 0
+    while size < nbytes:
+        c = int(rng.choice(kinds))
+        if c == 0:
+            out.append(bytes([0, int(rng.integers(0, 255))]))
+        else:
+            words = rng.integers(0, 1 << 32, c, dtype=np.uint64).astype(np.uint32)
+            words[rng.random(c) < 0.3] &= np.uint32(0x0000ff00)
+            words[rng.random(c) < 0.1] = np.uint32(0xff)
+            head = bytes([c]) if c < 255 else b"\xff" + int(c).to_bytes(4, "little")
+            out.append(head + words.tobytes())
+        size += len(out[-1])
+    return b"".join(out)
+
+
+@pytest.mark.parametrize("kinds", [(0,), (1,), (254,), (0, 1, 2, 3, 254), (0, 3, 255, 300, 5000, 70000), (200000, 1)],
+                         ids=["zeros", "ones", "longest_short", "short", "mixed", "huge"])
+@pytest.mark.parametrize("size", [1, 63, 255, 16383, 16385, 700_001, 2_500_003])
+def test_decode_lengths_and_phases(dev, size, kinds):
+    """Streams around the sub-block (64), block (256), chunk (16 KB) and
+    superchunk (8 chunks and more) lengths, records that cross, cover and skip
+    them, at an unaligned device address too."""
+    rng = np.random.default_rng(size + len(kinds))
+    adj = _stream(rng, size, kinds)
+    want = oracle.shard_decode(adj)
+    torch = dev._torch()
+    for shift in (0, 3):
+        d = torch.from_numpy(np.frombuffer(b"\0" * shift + adj, np.uint8).copy()).to("cuda")[shift:]
+        s, t, vend = dev.shard_decode(d, len(adj))
+        np.testing.assert_array_equal(dev.to_host_u32(s, len(want[0])), want[0])
+        np.testing.assert_array_equal(dev.to_host_u32(t, len(want[0])), want[1])
+
+
+def test_decode_far_list_overflow(dev):
+    """More four-byte-count look-alikes than a superchunk's far list holds: a
+    long record whose words hold, at every offset, counts that end far inside
+    the superchunks behind, so the true far entry may be missing from the list
+    and the chain walks that superchunk chunk by chunk."""
+    span = 8 * 16384  # superchunk of a stream of at most 128 chunks
+    n = span // 4 - 200
+    words = np.empty(n, np.uint32)
+    words[0::2] = 0xff000000  # 0xff, then the next word as the count
+    words[1::2] = (span // 4) + np.arange(len(words[1::2])) % 3000 + 400
+    first = b"\xff" + int(n).to_bytes(4, "little") + words.tobytes()
+    second = b"\xff" + int(span // 4 + 2000).to_bytes(4, "little") + bytes(4 * (span // 4 + 2000))
+    tail = (b"\x02" + bytes(8)) * 30000
+    adj = first + second + tail
+    want = oracle.shard_decode(adj)
+    s, t, vend = dev.shard_decode(to_dev_u8(dev, adj), len(adj))
+    np.testing.assert_array_equal(dev.to_host_u32(s, len(want[0])), want[0])
+    np.testing.assert_array_equal(dev.to_host_u32(t, len(want[0])), want[1])
