@@ -12,13 +12,15 @@
 //       oriented CSR (N+(v): the higher-ranked neighbours of v, ascending).
 //   gchi_tc_count   : every triangle a<b<w is found once, at vertex a, as
 //       w in N+(a) n N+(b) for b in N+(a).  One wavefront per vertex a.
-//       |N+(a)| <= 1024 (the hash form, tc_count_hash_kernel): N+(a) goes
-//       into an LDS hash table and every w of N+(b) is looked up lane-wide.
-//       Longer N+(a) (tc_count_kernel): the (b, w in N+(b)) pairs of 64
-//       consecutive b are flattened over the 64 lanes and each lane
-//       binary-searches its w in N+(a) in global memory.  Counts: a, b and w
-//       each get +1 per triangle, gathered per wavefront and flushed with
-//       uint64 atomics, converted to uint32 with an overflow flag.
+//       w among the 4096 highest ranks (the core; nearly all wedges of a skewed
+//       graph end there): tc_count_core_kernel, rows as bitmaps.
+//       The other w, |N+(a)| <= 1024 of them (the hash form,
+//       tc_count_hash_kernel): N+(a) goes into an LDS hash table and every w of
+//       N+(b) is looked up lane-wide.  Longer N+(a) (tc_count_kernel): the
+//       (b, w in N+(b)) pairs of 64 consecutive b are flattened over the 64
+//       lanes and each lane binary-searches its w in N+(a) in global memory.
+//       Counts: a, b and w each get +1 per triangle, gathered per wavefront or
+//       workgroup and converted to uint32 with an overflow flag.
 #include <mutex>
 
 #include "common.hpp"
@@ -132,7 +134,10 @@ GCHI_DEV int bsearch_u32(const uint32_t *a, uint32_t lo, uint32_t hi, uint32_t x
     return -1;
 }
 
+// end[v] = where the row ends for the hash and search kernels: off[v + 1], or the
+// row's first core entry.
 __global__ __launch_bounds__(kTcWaves *kWave) void tc_count_kernel(const uint32_t *__restrict__ off,
+                                                                   const uint32_t *__restrict__ end,
                                                                    const uint32_t *__restrict__ adj, uint32_t n,
                                                                    uint32_t min_da, unsigned long long *cnt,
                                                                    unsigned long long *total) {
@@ -147,12 +152,12 @@ __global__ __launch_bounds__(kTcWaves *kWave) void tc_count_kernel(const uint32_
     const uint64_t step = (uint64_t)gridDim.x * kTcWaves * kWave;
     for (uint64_t base = ((uint64_t)blockIdx.x * kTcWaves + wave) * kWave; base < n; base += step) {
         const uint64_t v = base + lane;
-        const uint32_t dv = v < n ? off[v + 1] - off[v] : 0u;
+        const uint32_t dv = v < n ? end[v] - off[v] : 0u;
         uint64_t todo = __ballot(dv >= 2 && dv > min_da);
         while (todo) {
         const uint32_t a = (uint32_t)base + (uint32_t)__builtin_ctzll(todo);
         todo &= todo - 1;
-        const uint32_t ab = off[a], da = off[a + 1] - ab;
+        const uint32_t ab = off[a], da = end[a] - ab;
         const uint32_t *A = adj + ab;
         const bool lds = da <= (uint32_t)kTcLds;
         if (lds)
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(kTcWaves *kWave) void tc_count_kernel(const uint32_
             const bool valid = k < da;
             uint32_t b = valid ? As[k] : 0u;
             uint32_t bb = valid ? off[b] : 0u;
-            uint32_t lb = valid ? off[b + 1] - bb : 0u;
+            uint32_t lb = valid ? end[b] - bb : 0u;
             uint32_t pre = lb;
 #pragma unroll
             for (int o = 1; o < kWave; o <<= 1) {
@@ -245,12 +250,14 @@ constexpr uint32_t kTcHashSlots = 2048;
 constexpr uint32_t kTcHashMax = kTcHashSlots / 2;
 constexpr uint32_t kTcEmpty = 0xffffffffu;
 // Vertex tickets come from kTcStripes counters, each in its own 128-byte line:
-// stripe k hands out the ranks n-1-k, n-1-k-kTcStripes, ...  Atomics on one
-// address complete one after another (about 10 ns each here), so a single
-// counter would cap the kernel at ~10^8 vertices per second.
+// stripe k hands out groups k, k + kTcStripes, ... of kTcTicket ranks from the
+// highest down.  Atomics on one address complete one after another (about 10 ns
+// each here), so a single counter would cap the kernel at ~10^8 vertices per
+// second.
 constexpr uint32_t kTcStripes = 32;
 constexpr int kTcInflight = 8;  // w loads per lane in flight (one memory round trip per 512 w)
 constexpr uint32_t kTcStripeGap = 32;
+constexpr uint32_t kTcTicket = 16;  // vertices per ticket
 
 GCHI_DEV uint32_t tc_slot(uint32_t w, int sh) { return (w * 2654435761u) >> sh; }
 
@@ -315,6 +322,7 @@ GCHI_DEV uint32_t tc_count_b(const uint32_t *adj, const uint32_t *keys, uint32_t
 }
 
 __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(const uint32_t *__restrict__ off,
+                                                                            const uint32_t *__restrict__ end,
                                                                             const uint32_t *__restrict__ adj,
                                                                             uint32_t n, unsigned long long *cnt,
                                                                             unsigned long long *total,
@@ -330,15 +338,21 @@ __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(cons
         uint32_t t = 0;
         if (lane == 0) t = atomicAdd(&work[stripe * kTcStripeGap], 1u);
         t = __shfl(t, 0, kWave);
-        const uint64_t idx = stripe + (uint64_t)kTcStripes * t;
-        if (idx >= n) {  // this stripe is drained: move on, stop after all of them
+        const uint64_t top = (stripe + (uint64_t)kTcStripes * t) * kTcTicket;
+        if (top >= n) {  // this stripe is drained: move on, stop after all of them
             if (++spent == kTcStripes) break;
             stripe = (stripe + 1) % kTcStripes;
             continue;
         }
-        const uint32_t a = n - 1 - (uint32_t)idx;  // highest rank (most work) first
-        const uint32_t ab = off[a], da = off[a + 1] - ab;
-        if (da < 2 || da > kTcHashMax) continue;
+        // highest rank (most work) first; vertices without two neighbours to hash are passed over together
+        const uint64_t mine = top + lane;
+        const bool in = lane < (int)kTcTicket && mine < n;
+        const uint32_t dmine = in ? end[n - 1 - (uint32_t)mine] - off[n - 1 - (uint32_t)mine] : 0u;
+        uint64_t todo = __ballot(dmine >= 2 && dmine <= kTcHashMax);
+        while (todo) {
+        const uint32_t a = n - 1 - (uint32_t)top - (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        const uint32_t ab = off[a], da = end[a] - ab;
         const uint32_t want = 4 * da;  // slots: pow2 >= 4 da, at most kTcHashSlots
         const int lg = min(32 - __clz((int)(want - 1)), 11);
         const uint32_t S = 1u << lg, mask = S - 1;
@@ -362,7 +376,7 @@ __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(cons
             const bool valid = k + 1 < da;
             const uint32_t b = valid ? A[k] : 0u;
             const uint32_t bb = valid ? off[b] : 0u;
-            const uint32_t lb = valid ? off[b + 1] - bb : 0u;
+            const uint32_t lb = valid ? end[b] - bb : 0u;
             const uint32_t nb = min((uint32_t)kWave, da - 1 - bc);
             // The first 64 entries of N+(b_j) are loaded one b ahead (slots w2[0],
             // w2[1] in turn), so that b_j's probes overlap b_{j+1}'s loads.
@@ -386,8 +400,275 @@ __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(cons
         acc_total += acc_a;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        }
     }
     if (lane == 0 && acc_total) atomicAdd(total, acc_total);
+}
+
+// ---- the core: triangles whose highest vertex w is among the kTcCore highest ranks ----
+// In a skewed graph nearly all wedges end there (96% at R-MAT scale 19), and the
+// rows that make them are dense in it, so a row's core entries are a bitmap of
+// kTcCore bits, 64 per lane: the w of (a, b) are one AND, their number one
+// popcount, and the credits of w vertical counters in registers (bit planes
+// summed with carry-save adders, flushed every 2^kTcPlanes bitmaps).  Bitmaps
+// are kept for the rows with more than kTcList core entries (below that the
+// list is shorter than the bitmap) of the highest ranks; the entries of other
+// rows are tested one by one against N+(a)'s bitmap in LDS.
+// Bound: vector instructions (about 25 per bitmap) and the L2 reads of the
+// bitmaps.  @@
+constexpr uint32_t kTcCore = 4096;
+constexpr uint32_t kTcCoreWords = kTcCore / 32;
+constexpr uint32_t kTcList = 128;
+constexpr uint32_t kTcMapRows = 1u << 18;   // at most 128 MiB of bitmaps
+constexpr uint32_t kTcNear = 16384;         // ranks whose b and w credits are counted in LDS
+constexpr int kTcCoreThreads = 512;
+constexpr int kTcCoreWaves = kTcCoreThreads / kWave;
+constexpr int kTcPlanes = 12;
+constexpr uint32_t kTcTicketCore = 8;       // vertices per ticket
+
+// end[v] = first entry of v's row in the core (rank >= base).
+__global__ void tc_core_split(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, uint32_t n,
+                              uint32_t base, uint32_t *__restrict__ end) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
+        uint32_t lo = off[v], hi = off[v + 1];
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (adj[mid] >= base) hi = mid;
+            else lo = mid + 1;
+        }
+        end[v] = lo;
+    }
+}
+
+// One wavefront per row v = first + r with more than kTcList core entries: its bitmap.
+__global__ __launch_bounds__(256) void tc_core_maps(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj,
+                                                    const uint32_t *__restrict__ end, uint32_t first, uint32_t rows,
+                                                    uint32_t base, uint2 *__restrict__ maps) {
+    __shared__ uint32_t s_bits[256 / kWave][kTcCoreWords];
+    const int lane = threadIdx.x & (kWave - 1);
+    uint32_t *bits = s_bits[threadIdx.x / kWave];
+    const uint32_t nw = gridDim.x * (256 / kWave);
+    for (uint32_t r = blockIdx.x * (256 / kWave) + threadIdx.x / kWave; r < rows; r += nw) {
+        const uint32_t b = end[first + r], e = off[first + r + 1];
+        if (e - b <= kTcList) continue;
+        bits[lane] = bits[lane + kWave] = 0u;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t k = b + lane; k < e; k += kWave) {
+            const uint32_t c = adj[k] - base;
+            atomicOr(&bits[c >> 5], 1u << (c & 31));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        maps[(uint64_t)r * kWave + lane] = make_uint2(bits[2 * lane], bits[2 * lane + 1]);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// sum and carry of three words
+GCHI_DEV void tc_csa(uint32_t &s, uint32_t &c, uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t u = x ^ y;
+    c = (x & y) | (u & z);
+    s = u ^ z;
+}
+
+// Adds eight words to the bit planes.
+GCHI_DEV void tc_planes_add(uint32_t (&p)[kTcPlanes], const uint32_t (&x)[8]) {
+    uint32_t a, b, c, d, e;
+    tc_csa(p[0], a, p[0], x[0], x[1]);
+    tc_csa(p[0], b, p[0], x[2], x[3]);
+    tc_csa(p[1], c, p[1], a, b);
+    tc_csa(p[0], a, p[0], x[4], x[5]);
+    tc_csa(p[0], b, p[0], x[6], x[7]);
+    tc_csa(p[1], d, p[1], a, b);
+    tc_csa(p[2], e, p[2], c, d);
+#pragma unroll
+    for (int k = 3; k < kTcPlanes; k++) {
+        const uint32_t t = p[k] & e;
+        p[k] ^= e;
+        e = t;
+    }
+}
+
+// Sum over the wavefront, in lane 63.
+GCHI_DEV uint32_t tc_sum63(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
+__global__ __launch_bounds__(kTcCoreThreads, 4) void tc_count_core_kernel(
+    const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, const uint32_t *__restrict__ end, uint32_t n,
+    uint32_t base, uint32_t near, uint32_t first, const uint2 *__restrict__ maps, unsigned long long *cnt,
+    unsigned long long *total, uint32_t *work, uint32_t *__restrict__ slab) {
+    __shared__ uint32_t s_near[kTcNear];  // credits of the ranks from near
+    __shared__ uint32_t s_bits[kTcCoreWaves][kTcCoreWords];
+    __shared__ unsigned long long s_total;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    uint32_t *bits = s_bits[wave];
+    uint32_t *core = s_near + (base - near);
+    for (uint32_t k = threadIdx.x; k < kTcNear; k += kTcCoreThreads) s_near[k] = 0u;
+    if (threadIdx.x == 0) s_total = 0;
+    __syncthreads();
+    uint32_t p0[kTcPlanes], p1[kTcPlanes];
+#pragma unroll
+    for (int k = 0; k < kTcPlanes; k++) p0[k] = p1[k] = 0u;
+    uint32_t held = 0;  // bitmaps in the planes
+    auto flush = [&]() {
+        for (uint32_t i = 0; i < 32; i++) {
+            uint32_t c0 = 0, c1 = 0;
+#pragma unroll
+            for (int k = 0; k < kTcPlanes; k++) {
+                c0 |= ((p0[k] >> i) & 1u) << k;
+                c1 |= ((p1[k] >> i) & 1u) << k;
+            }
+            if (c0) atomicAdd(&core[lane * 64 + i], c0);
+            if (c1) atomicAdd(&core[lane * 64 + 32 + i], c1);
+        }
+#pragma unroll
+        for (int k = 0; k < kTcPlanes; k++) p0[k] = p1[k] = 0u;
+        held = 0;
+    };
+    unsigned long long acc_total = 0;
+    uint32_t stripe = (blockIdx.x * kTcCoreWaves + wave) % kTcStripes, spent = 0;
+    for (;;) {
+        uint32_t t = 0;
+        if (lane == 0) t = atomicAdd(&work[stripe * kTcStripeGap], 1u);
+        t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+        const uint64_t top = (stripe + (uint64_t)kTcStripes * t) * kTcTicketCore;
+        if (top >= n) {
+            if (++spent == kTcStripes) break;
+            stripe = (stripe + 1) % kTcStripes;
+            continue;
+        }
+        const uint32_t many = (uint32_t)min<uint64_t>(kTcTicketCore, n - top);
+        for (uint32_t q = 0; q < many; q++) {
+            const uint32_t a = n - 1 - (uint32_t)top - q;
+            const uint32_t ab = off[a], ac = end[a], ae = off[a + 1];
+            if (ae - ab < 2 || ac == ae) continue;
+            bits[lane] = bits[lane + kWave] = 0u;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t k = ac + lane; k < ae; k += kWave) {
+                const uint32_t c = adj[k] - base;
+                atomicOr(&bits[c >> 5], 1u << (c & 31));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t a0 = bits[2 * lane], a1 = bits[2 * lane + 1];
+            uint32_t acc_a = 0;  // per lane; a has at most 2^31 triangles here (at most E pairs of a lane's b)
+            for (uint32_t bc = ab; bc + 1 < ae; bc += kWave) {  // the last neighbour has no w above it
+                const bool valid = bc + lane + 1 < ae;
+                const uint32_t b = valid ? adj[bc + lane] : 0u;
+                const uint32_t bs = valid ? end[b] : 0u;
+                const uint32_t lb = valid ? off[b + 1] - bs : 0u;
+                const bool mapped = lb > kTcList && b >= first;
+                uint32_t tb = 0;  // triangles (a, b of this lane, w)
+                uint64_t m = __ballot(mapped);
+                while (m) {
+                    uint32_t x0[8], x1[8], j[8], sum[4];
+                    const uint32_t some = (uint32_t)__popcll(m);
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const bool on = (uint32_t)u < some;  // wavefront-uniform
+                        j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
+                        m &= m - (on ? 1ull : 0ull);
+                        x0[u] = x1[u] = 0u;
+                        if (on) {
+                            const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)j[u]) - first;
+                            const uint2 w = maps[(uint64_t)r * kWave + lane];
+                            x0[u] = w.x;
+                            x1[u] = w.y;
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        x0[u] &= a0;
+                        x1[u] &= a1;
+                    }
+                    tc_planes_add(p0, x0);
+                    tc_planes_add(p1, x1);
+#pragma unroll
+                    for (int u = 0; u < 4; u++)  // two counts (at most kTcCore each) per sum
+                        sum[u] = tc_sum63((uint32_t)(__popc(x0[2 * u]) + __popc(x1[2 * u])) +
+                                          ((uint32_t)(__popc(x0[2 * u + 1]) + __popc(x1[2 * u + 1])) << 16));
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const uint32_t both = (uint32_t)__builtin_amdgcn_readlane((int)sum[u / 2], kWave - 1);
+                        const uint32_t c = u & 1 ? both >> 16 : both & 0xffffu;
+                        if ((uint32_t)u < some) tb = (uint32_t)lane == j[u] ? c : tb;
+                    }
+                    held += 8;
+                    if (held > (1u << kTcPlanes) - 16) flush();
+                }
+                // short rows: four at a time, the first 64 entries of each in flight together
+                m = __ballot(valid && !mapped && lb != 0);
+                while (m) {
+                    uint32_t w[4], j[4], beg[4], len[4];
+                    const uint32_t some = (uint32_t)__popcll(m);
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const bool on = (uint32_t)u < some;
+                        j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
+                        m &= m - (on ? 1ull : 0ull);
+                        beg[u] = (uint32_t)__builtin_amdgcn_readlane((int)bs, (int)j[u]);
+                        len[u] = on ? (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j[u]) : 0u;
+                        w[u] = (uint32_t)lane < len[u] ? adj[beg[u] + lane] : n;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        uint32_t hits = 0;
+                        for (uint32_t k = 0; k < len[u]; k += kWave) {
+                            if (k) w[u] = k + lane < len[u] ? adj[beg[u] + k + lane] : n;
+                            bool hit = false;
+                            if (w[u] < n) {
+                                const uint32_t c = w[u] - base;
+                                hit = (bits[c >> 5] >> (c & 31)) & 1u;
+                                if (hit) atomicAdd(&core[c], 1u);
+                            }
+                            hits += (uint32_t)__popcll(__ballot(hit));
+                        }
+                        if ((uint32_t)u < some) tb = (uint32_t)lane == j[u] ? hits : tb;
+                    }
+                }
+                if (tb) {
+                    if (b >= near) atomicAdd(&s_near[b - near], tb);
+                    else atomicAdd(&cnt[b], (unsigned long long)tb);
+                }
+                acc_a += tb;
+            }
+            const unsigned long long found = wave_sum((unsigned long long)acc_a);
+            if (lane == 0 && found) atomicAdd(&cnt[a], found);
+            acc_total += found;
+        }
+    }
+    flush();
+    if (lane == 0 && acc_total) atomicAdd(&s_total, acc_total);
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < kTcNear; k += kTcCoreThreads)
+        slab[(uint64_t)blockIdx.x * kTcNear + k] = s_near[k];
+    if (threadIdx.x == 0 && s_total) atomicAdd(total, s_total);
+}
+
+// cnt[near + k] += the workgroups' credits (the only writer at this point of the stream).
+__global__ void tc_core_sum(const uint32_t *__restrict__ slab, uint32_t nwg, uint32_t near, uint32_t n,
+                            unsigned long long *cnt) {
+    __shared__ unsigned long long s_part[4][kWave];
+    const uint32_t lane = threadIdx.x & (kWave - 1), part = threadIdx.x / kWave;
+    const uint32_t k = blockIdx.x * kWave + lane;
+    unsigned long long c = 0;
+    for (uint32_t g = part; g < nwg; g += 4) c += slab[(uint64_t)g * kTcNear + k];
+    s_part[part][lane] = c;
+    __syncthreads();
+    if (part == 0 && near + k < n) {
+        c = s_part[0][lane] + s_part[1][lane] + s_part[2][lane] + s_part[3][lane];
+        if (c) cnt[near + k] += c;
+    }
 }
 
 __global__ void tc_to_u32(const unsigned long long *cnt, uint32_t n, uint32_t *out, uint32_t *overflow) {
@@ -513,38 +794,76 @@ extern "C" int gchi_tc_prepare(const uint32_t *d_src, const uint32_t *d_dst, uin
 
 namespace gchi {
 
-// The counting launches, over counters cnt[n+1] / tot[1] / ticket stripes wk
-// (all cleared here first).
+// Scratch of one count.  rows = 0: no core kernel (only cnt, tot and wk are there).
+struct TcCount {
+    unsigned long long *cnt, *tot;  // [n + 1], [1]
+    uint32_t *wk, *wk2;             // ticket stripes of the hash and the core kernel
+    uint32_t *end, *slab;
+    uint2 *maps;
+    uint32_t rows, nwg;
+};
+
+static int tc_ncu() {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+        return v;
+    return 256;
+}
+
+// The counting launches (the counters are cleared here first).
 static int tc_count_impl(const uint32_t *d_off, const uint32_t *d_adj, uint32_t nvertices, uint32_t *d_per_vertex,
-                         uint64_t *d_total, uint32_t *d_overflow, unsigned long long *cnt, unsigned long long *tot,
-                         uint32_t *wk, hipStream_t s) {
-    launch_fill_u64(reinterpret_cast<uint64_t *>(cnt), 0ull, nvertices, s);
-    launch_fill_u64(reinterpret_cast<uint64_t *>(tot), 0ull, 1, s);
-    launch_fill_u32(wk, 0u, kTcStripes * kTcStripeGap, s);
+                         uint64_t *d_total, uint32_t *d_overflow, const TcCount &w, hipStream_t s) {
+    const uint32_t n = nvertices;
+    launch_fill_u64(reinterpret_cast<uint64_t *>(w.cnt), 0ull, n, s);
+    launch_fill_u64(reinterpret_cast<uint64_t *>(w.tot), 0ull, 1, s);
+    launch_fill_u32(w.wk, 0u, kTcStripes * kTcStripeGap, s);
     launch_fill_u32(d_overflow, 0u, 1, s);
-    int ncu = 256;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ncu = v;
+    const int ncu = tc_ncu();
+    const uint32_t *end = d_off + 1;
+    if (w.rows) {
+        const uint32_t base = n > kTcCore ? n - kTcCore : 0u, near = n > kTcNear ? n - kTcNear : 0u;
+        const uint32_t first = n - w.rows;
+        launch_fill_u32(w.wk2, 0u, kTcStripes * kTcStripeGap, s);
+        hipLaunchKernelGGL(tc_core_split, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, d_off, d_adj, n, base, w.end);
+        hipLaunchKernelGGL(tc_core_maps, dim3(grid_for(w.rows, 4, 8192)), dim3(256), 0, s, d_off, d_adj, w.end, first,
+                           w.rows, base, w.maps);
+        hipLaunchKernelGGL(tc_count_core_kernel, dim3(w.nwg), dim3(kTcCoreThreads), 0, s, d_off, d_adj, w.end, n, base,
+                           near, first, w.maps, w.cnt, w.tot, w.wk2, w.slab);
+        hipLaunchKernelGGL(tc_core_sum, dim3(kTcNear / kWave), dim3(256), 0, s, w.slab, w.nwg, near, n, w.cnt);
+        end = w.end;
     }
-    hipLaunchKernelGGL(tc_count_hash_kernel, dim3(ncu * 6), dim3(kTcHashWaves * kWave), 0, s, d_off, d_adj,
-                       nvertices, cnt, tot, wk);
-    hipLaunchKernelGGL(tc_count_kernel, dim3(ncu * 8), dim3(kTcWaves * kWave), 0, s, d_off, d_adj, nvertices,
-                       kTcHashMax, cnt, tot);
-    hipLaunchKernelGGL(tc_to_u32, dim3(grid_for(nvertices, 256, 65536)), dim3(256), 0, s, cnt, nvertices,
-                       d_per_vertex, d_overflow);
-    GCHI_HIP(hipMemcpyAsync(d_total, tot, 8, hipMemcpyDeviceToDevice, s));
+    if (!w.rows || n > kTcCore) {
+        hipLaunchKernelGGL(tc_count_hash_kernel, dim3(ncu * 6), dim3(kTcHashWaves * kWave), 0, s, d_off, end, d_adj, n,
+                           w.cnt, w.tot, w.wk);
+        hipLaunchKernelGGL(tc_count_kernel, dim3(ncu * 8), dim3(kTcWaves * kWave), 0, s, d_off, end, d_adj, n,
+                           kTcHashMax, w.cnt, w.tot);
+    }
+    hipLaunchKernelGGL(tc_to_u32, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, w.cnt, n, d_per_vertex, d_overflow);
+    GCHI_HIP(hipMemcpyAsync(d_total, w.tot, 8, hipMemcpyDeviceToDevice, s));
     GCHI_LAUNCH_CHECK();
     return GCHI_OK;
 }
 
 template <typename C>
-static void tc_count_layout(C &c, uint32_t nvertices, unsigned long long **cnt, unsigned long long **tot,
-                            uint32_t **wk) {
-    *cnt = c.template take<unsigned long long>((size_t)nvertices + 1);
-    *tot = c.template take<unsigned long long>(1);
-    *wk = c.template take<uint32_t>(kTcStripes * kTcStripeGap);
+static void tc_count_layout(C &c, uint32_t nvertices, TcCount *w) {
+    w->cnt = c.template take<unsigned long long>((size_t)nvertices + 1);
+    w->tot = c.template take<unsigned long long>(1);
+    w->wk = c.template take<uint32_t>(kTcStripes * kTcStripeGap);
+    w->rows = 0;
+}
+
+// The core kernel's scratch after it: bitmaps for the highest n / 8 ranks (at
+// least 16384, at most kTcMapRows: rows of more than kTcList core entries are
+// among them in a skewed graph, 64 bytes per vertex), two workgroups per CU.
+template <typename C>
+static void tc_core_layout(C &c, uint32_t nvertices, TcCount *w) {
+    w->rows = std::min(nvertices, std::min(kTcMapRows, std::max(nvertices / 8, kTcNear)));
+    w->nwg = std::min<uint32_t>(2 * 256, std::max(1u, nvertices / 64));
+    w->wk2 = c.template take<uint32_t>(kTcStripes * kTcStripeGap);
+    w->end = c.template take<uint32_t>(nvertices);
+    w->slab = c.template take<uint32_t>((size_t)w->nwg * kTcNear);
+    w->maps = c.template take<uint2>((size_t)w->rows * kWave);
 }
 
 // ---- allocation-free counting: scratch in a file-scope device array ----
@@ -579,9 +898,9 @@ using namespace gchi;
 extern "C" int gchi_tc_count_workspace(uint32_t nvertices, size_t *bytes) {
     GCHI_CHECK(bytes, GCHI_ERR_INVALID, "null bytes");
     SizerAdapter a;
-    unsigned long long *cnt, *tot;
-    uint32_t *wk;
-    tc_count_layout(a, nvertices, &cnt, &tot, &wk);
+    TcCount w;
+    tc_count_layout(a, nvertices, &w);
+    tc_core_layout(a, nvertices, &w);
     *bytes = a.z.off;
     return GCHI_OK;
 }
@@ -595,11 +914,10 @@ extern "C" int gchi_tc_count(const uint32_t *d_off, const uint32_t *d_adj, uint3
     gchi_tc_count_workspace(nvertices, &need);
     GCHI_CHECK(d_work && work_bytes >= need, GCHI_ERR_WORKSPACE, "tc_count: workspace too small");
     Carver c(d_work, work_bytes);
-    unsigned long long *cnt, *tot;
-    uint32_t *wk;
-    tc_count_layout(c, nvertices, &cnt, &tot, &wk);
-    return tc_count_impl(d_off, d_adj, nvertices, d_per_vertex, d_total, d_overflow, cnt, tot, wk,
-                         as_stream(stream));
+    TcCount w;
+    tc_count_layout(c, nvertices, &w);
+    tc_core_layout(c, nvertices, &w);
+    return tc_count_impl(d_off, d_adj, nvertices, d_per_vertex, d_total, d_overflow, w, as_stream(stream));
 }
 
 extern "C" int gchi_tc_count_noalloc(const uint32_t *d_off, const uint32_t *d_adj, uint32_t nvertices,
@@ -613,12 +931,10 @@ extern "C" int gchi_tc_count_noalloc(const uint32_t *d_off, const uint32_t *d_ad
     GCHI_HIP(hipGetDevice(&dev));
     GCHI_TRY(tc_scratch_setup(dev));
     Carver c(g_scratch_ptr[dev], kTcScratchBytes);
-    unsigned long long *cnt, *tot;
-    uint32_t *wk;
-    tc_count_layout(c, nvertices, &cnt, &tot, &wk);
+    TcCount w;
+    tc_count_layout(c, nvertices, &w);  // no bitmaps: the hash and search kernels alone
     GCHI_CHECK(c.ok(), GCHI_ERR_INVALID, "tc_count_noalloc: scratch layout exceeds its array");
-    return tc_count_impl(d_off, d_adj, nvertices, d_per_vertex, d_total, d_overflow, cnt, tot, wk,
-                         as_stream(stream));
+    return tc_count_impl(d_off, d_adj, nvertices, d_per_vertex, d_total, d_overflow, w, as_stream(stream));
 }
 
 __global__ void relabel_kernel(const uint32_t *src, const uint32_t *dst, uint64_t e, uint32_t n, const uint32_t *map,

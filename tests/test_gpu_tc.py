@@ -57,3 +57,46 @@ def test_tc_scale21_vs_oracle(dev):
     assert tot == otot
     np.testing.assert_array_equal(dev.to_host_u32(prep.vertexmap, n), vm)
     np.testing.assert_array_equal(pv, opv)
+
+
+@pytest.mark.parametrize("n", [3, 129, 131, 1500, 4097, 4200])
+def test_tc_complete_graphs(dev, n):
+    """K_n around the sizes of the counting kernels: rows of 128 and 129 core
+    entries (list / bitmap), a core smaller than, equal to and larger than the
+    4096 highest ranks, more bitmaps per wavefront than its bit planes hold."""
+    a, b = np.triu_indices(n, 1)
+    prep, pv, tot, ovf = run_tc(dev, a.astype(np.uint32), b.astype(np.uint32), n)
+    assert ovf == 0 and tot == n * (n - 1) * (n - 2) // 6
+    assert (pv == (n - 1) * (n - 2) // 2).all()
+
+
+@pytest.mark.parametrize("n,hubs,p,extra", [(5000, 200, 0.9, 40000), (17000, 700, 0.5, 60000),
+                                            (40000, 4200, 0.05, 200000), (150000, 300, 0.7, 500000)])
+def test_tc_core_and_tail_vs_oracle(dev, n, hubs, p, extra):
+    """Dense hubs, random edges to them and a sparse rest: triangles with none,
+    one, two and all vertices in the core, bitmapped and listed rows, credits
+    counted in LDS and in global memory; the same counts from the form without
+    a workspace (no core kernel)."""
+    import torch
+    rng = np.random.default_rng(n)
+    a, b = np.triu_indices(hubs, 1)
+    k = rng.random(len(a)) < p
+    s = [a[k], rng.integers(0, hubs, extra), rng.integers(0, n, extra)]
+    d = [b[k], rng.integers(0, n, extra), rng.integers(0, n, extra)]
+    base = rng.integers(0, n - 3, 5000)  # triangles of the tail
+    s += [base, base, base + 1]
+    d += [base + 1, base + 2, base + 2]
+    ids = rng.permutation(n)
+    s, d = ids[np.concatenate(s)], ids[np.concatenate(d)]
+    src, dst = graphs.preprocess(s, d, simple=True)
+    prep, pv, tot, ovf = run_tc(dev, src, dst, n)
+    vm, opv, otot = oracle.triangles(n, src, dst)
+    assert tot == otot and ovf == 0
+    np.testing.assert_array_equal(pv, opv)
+    q = dev.empty_u32(n)
+    t2 = torch.zeros(1, dtype=torch.int64, device="cuda")
+    o2 = torch.zeros(1, dtype=torch.int32, device="cuda")
+    dev.check(dev.lib().gchi_tc_count_noalloc(dev.dptr(prep.off), dev.dptr(prep.adj), n, dev.dptr(q), dev.dptr(t2),
+                                              dev.dptr(o2), dev.stream()), "tc_count_noalloc")
+    assert int(t2.item()) == otot
+    np.testing.assert_array_equal(dev.to_host_u32(q, n), opv)
