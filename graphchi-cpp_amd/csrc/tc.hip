@@ -14,11 +14,11 @@
 //       w in N+(a) n N+(b) for b in N+(a).  One wavefront per vertex a.
 //       w among the 4096 highest ranks (the core; nearly all wedges of a skewed
 //       graph end there): tc_count_core_kernel, rows as bitmaps.
-//       The other w, |N+(a)| <= 1024 of them (the hash form,
-//       tc_count_hash_kernel): N+(a) goes into an LDS hash table and every w of
-//       N+(b) is looked up lane-wide.  Longer N+(a) (tc_count_kernel): the
+//       The other w, |N+(a)| <= 512 of them (tc_count_tail_kernel): the
 //       (b, w in N+(b)) pairs of 64 consecutive b are flattened over the 64
-//       lanes and each lane binary-searches its w in N+(a) in global memory.
+//       lanes, and each w passes a 4096-bit filter of N+(a) in LDS before it is
+//       searched there.  Longer N+(a) (tc_count_kernel): the same pairs, each
+//       lane binary-searching its w in N+(a).
 //       Counts: a, b and w each get +1 per triangle, gathered per wavefront or
 //       workgroup and converted to uint32 with an overflow flag.
 #include <mutex>
@@ -134,8 +134,8 @@ GCHI_DEV int bsearch_u32(const uint32_t *a, uint32_t lo, uint32_t hi, uint32_t x
     return -1;
 }
 
-// end[v] = where the row ends for the hash and search kernels: off[v + 1], or the
-// row's first core entry.
+// end[v] = where the row ends for this kernel and the tail kernel: off[v + 1], or
+// the row's first core entry.
 __global__ __launch_bounds__(kTcWaves *kWave) void tc_count_kernel(const uint32_t *__restrict__ off,
                                                                    const uint32_t *__restrict__ end,
                                                                    const uint32_t *__restrict__ adj, uint32_t n,
@@ -235,174 +235,153 @@ __global__ __launch_bounds__(kTcWaves *kWave) void tc_count_kernel(const uint32_
     }
 }
 
-// Hash form, for |N+(a)| <= kTcHashMax (every vertex of a degree-ordered
-// graph with up to ~500K edges, and nearly all of larger ones).  Vertices are
-// taken from the highest rank down: the work per vertex grows with its rank,
-// so the longest ones start first.  One wavefront per vertex a puts N+(a) into
-// an LDS hash table (open addressing, linear probing, at most half full, a
-// quarter when |N+(a)| <= kTcHashSlots / 4), then walks b in N+(a) one at a
-// time and looks up every w in N+(b) lane-wide, kTcInflight w per lane in
-// flight.  A hit is the triangle a < b < w.  Counts: w's and b's credits go to
-// their slots (16-bit halves of LDS words: at most 2|N+(a)| per slot) and are
-// added to the global counts once per vertex a.
-constexpr int kTcHashWaves = 4;
-constexpr uint32_t kTcHashSlots = 2048;
-constexpr uint32_t kTcHashMax = kTcHashSlots / 2;
-constexpr uint32_t kTcEmpty = 0xffffffffu;
-// Vertex tickets come from kTcStripes counters, each in its own 128-byte line:
-// stripe k hands out groups k, k + kTcStripes, ... of kTcTicket ranks from the
-// highest down.  Atomics on one address complete one after another (about 10 ns
-// each here), so a single counter would cap the kernel at ~10^8 vertices per
-// second.
-constexpr uint32_t kTcStripes = 32;
-constexpr int kTcInflight = 8;  // w loads per lane in flight (one memory round trip per 512 w)
-constexpr uint32_t kTcStripeGap = 32;
-constexpr uint32_t kTcTicket = 16;  // vertices per ticket
-
-GCHI_DEV uint32_t tc_slot(uint32_t w, int sh) { return (w * 2654435761u) >> sh; }
-
-GCHI_DEV int tc_find(const uint32_t *keys, uint32_t mask, int sh, uint32_t w) {
-    uint32_t h = tc_slot(w, sh);
-    for (;;) {
-        const uint32_t k = keys[h];
-        if (k == w) return (int)h;
-        if (k == kTcEmpty) return -1;
-        h = (h + 1) & mask;
-    }
+// Inclusive scans over the wavefront (sum; maximum), in six steps.
+template <int CTRL, int ROWS>
+GCHI_DEV uint32_t tc_dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+GCHI_DEV uint32_t tc_scan_sum(uint32_t v) {
+    v += tc_dpp<0x111, 0xf>(v);  // row_shr:1
+    v += tc_dpp<0x112, 0xf>(v);  // row_shr:2
+    v += tc_dpp<0x114, 0xf>(v);  // row_shr:4
+    v += tc_dpp<0x118, 0xf>(v);  // row_shr:8
+    v += tc_dpp<0x142, 0xa>(v);  // row_bcast:15
+    v += tc_dpp<0x143, 0xc>(v);  // row_bcast:31
+    return v;
+}
+GCHI_DEV uint32_t tc_scan_max(uint32_t v) {
+    v = max(v, tc_dpp<0x111, 0xf>(v));
+    v = max(v, tc_dpp<0x112, 0xf>(v));
+    v = max(v, tc_dpp<0x114, 0xf>(v));
+    v = max(v, tc_dpp<0x118, 0xf>(v));
+    v = max(v, tc_dpp<0x142, 0xa>(v));
+    v = max(v, tc_dpp<0x143, 0xc>(v));
+    return v;
 }
 
-GCHI_DEV void tc_credit(uint32_t *cw, uint32_t slot, uint32_t c) { atomicAdd(&cw[slot >> 1], c << ((slot & 1) * 16)); }
-
-// Entry `lane` of N+(b_j) (b_j, its start and length in lane j of b/bb/lb), or
-// kTcEmpty past the list; the load is issued at an in-bounds address either way.
-GCHI_DEV uint32_t tc_first_w(const uint32_t *adj, uint32_t bb, uint32_t lb, uint32_t j, int lane) {
-    const uint32_t bbj = (uint32_t)__builtin_amdgcn_readlane((int)bb, (int)j);
-    const uint32_t lbj = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j);
-    const uint32_t v = adj[lbj ? bbj + min((uint32_t)lane, lbj - 1) : 0u];
-    return (uint32_t)lane < lbj ? v : kTcEmpty;
+GCHI_DEV void tc_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Triangles (a, b_j, w) for w in N+(b_j): w0 holds the list's first 64
-// entries, the rest are loaded here; each w found in the table is credited,
-// and b_j once with the wavefront's total.  Returns that total.
-GCHI_DEV uint32_t tc_count_b(const uint32_t *adj, const uint32_t *keys, uint32_t *cw, uint32_t mask, int sh,
-                             uint32_t b, uint32_t bb, uint32_t lb, uint32_t j, uint32_t w0, int lane) {
-    const uint32_t bj = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)j);
-    const uint32_t bbj = (uint32_t)__builtin_amdgcn_readlane((int)bb, (int)j);
-    const uint32_t lbj = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j);
-    const uint32_t *B = adj + bbj;
-    uint32_t hits = 0;
-    if (w0 != kTcEmpty) {
-        const int h = tc_find(keys, mask, sh, w0);
-        if (h >= 0) {
-            tc_credit(cw, (uint32_t)h, 1u);
-            hits++;
-        }
-    }
-    for (uint32_t t = kWave + lane; t < lbj; t += kTcInflight * kWave) {
-        uint32_t w[kTcInflight];
-#pragma unroll
-        for (int q = 0; q < kTcInflight; q++) {
-            const uint32_t tq = t + q * kWave;
-            w[q] = tq < lbj ? B[tq] : kTcEmpty;
-        }
-#pragma unroll
-        for (int q = 0; q < kTcInflight; q++) {
-            if (w[q] == kTcEmpty) continue;
-            const int h = tc_find(keys, mask, sh, w[q]);
-            if (h >= 0) {
-                tc_credit(cw, (uint32_t)h, 1u);
-                hits++;
-            }
-        }
-    }
-    hits = wave_sum(hits);
-    if (hits && lane == 0) tc_credit(cw, (uint32_t)tc_find(keys, mask, sh, bj), hits);
-    return hits;
-}
+// The vertices of wavefront w are n-1-w, n-1-w-nw, ... (nw wavefronts): the work
+// per vertex changes slowly with its rank, so every wavefront gets a like share
+// without tickets (which took 146 of 1105 us per wavefront in the core kernel).
+// Lane l holds the row bounds of the l-th of the next 64 vertices.
 
-__global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(const uint32_t *__restrict__ off,
+// |N+(a)| in [2, kTcTailMax]: N+(a) in LDS with a bit filter of its ids, the
+// pairs of 64 b at a time in flattened order, kTcTailStep pairs per lane in
+// flight.  A pair's b comes from marks in LDS at the first pair of every b and a
+// maximum scan.  Bound: vector instructions (about 30 per 64 pairs) and, in
+// sparse graphs, the three dependent loads per vertex (row, b's bounds, w).
+// Short rows keep all lanes busy this way: the form before it, one b at a time
+// against a hash table, took 882 us for the tails of R-MAT scale 19 (75M pairs),
+// this one 172 us.
+constexpr int kTcTailWaves = 4;
+constexpr uint32_t kTcTailMax = 512;
+constexpr int kTcTailStep = 4;
+
+GCHI_DEV uint32_t tc_filter(uint32_t x) { return (x ^ (x >> 12)) & 4095u; }
+
+__global__ __launch_bounds__(kTcTailWaves *kWave) void tc_count_tail_kernel(const uint32_t *__restrict__ off,
                                                                             const uint32_t *__restrict__ end,
                                                                             const uint32_t *__restrict__ adj,
                                                                             uint32_t n, unsigned long long *cnt,
-                                                                            unsigned long long *total,
-                                                                            uint32_t *work) {
-    __shared__ uint32_t sKey[kTcHashWaves][kTcHashSlots];
-    __shared__ uint32_t sCw[kTcHashWaves][kTcHashSlots / 2];
+                                                                            unsigned long long *total) {
+    __shared__ uint32_t s_a[kTcTailWaves][kTcTailMax];    // N+(a), ascending
+    __shared__ uint32_t s_c[kTcTailWaves][kTcTailMax];    // credits of its entries
+    __shared__ uint32_t s_bits[kTcTailWaves][4096 / 32];
+    __shared__ uint32_t s_mark[kTcTailWaves][kTcTailStep * kWave];
+    __shared__ uint32_t s_hit[kTcTailWaves][kWave];
+    __shared__ unsigned long long s_total;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    uint32_t *keys = sKey[wave];
-    uint32_t *cw = sCw[wave];
+    uint32_t *A = s_a[wave], *C = s_c[wave], *bits = s_bits[wave], *mark = s_mark[wave], *hitc = s_hit[wave];
+    if (threadIdx.x == 0) s_total = 0;
+    __syncthreads();
     unsigned long long acc_total = 0;
-    uint32_t stripe = (blockIdx.x * kTcHashWaves + wave) % kTcStripes, spent = 0;
-    for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(&work[stripe * kTcStripeGap], 1u);
-        t = __shfl(t, 0, kWave);
-        const uint64_t top = (stripe + (uint64_t)kTcStripes * t) * kTcTicket;
-        if (top >= n) {  // this stripe is drained: move on, stop after all of them
-            if (++spent == kTcStripes) break;
-            stripe = (stripe + 1) % kTcStripes;
-            continue;
-        }
-        // highest rank (most work) first; vertices without two neighbours to hash are passed over together
-        const uint64_t mine = top + lane;
-        const bool in = lane < (int)kTcTicket && mine < n;
-        const uint32_t dmine = in ? end[n - 1 - (uint32_t)mine] - off[n - 1 - (uint32_t)mine] : 0u;
-        uint64_t todo = __ballot(dmine >= 2 && dmine <= kTcHashMax);
+    const uint64_t nw = (uint64_t)gridDim.x * kTcTailWaves;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * kTcTailWaves + wave; i0 < n; i0 += nw * kWave) {
+        const uint64_t mine = i0 + nw * lane;
+        const uint32_t va = mine < n ? n - 1 - (uint32_t)mine : 0u;
+        const uint32_t vb = mine < n ? off[va] : 0u, ve = mine < n ? end[va] : 0u;
+        uint64_t todo = __ballot(ve - vb >= 2 && ve - vb <= kTcTailMax);
         while (todo) {
-        const uint32_t a = n - 1 - (uint32_t)top - (uint32_t)__builtin_ctzll(todo);
-        todo &= todo - 1;
-        const uint32_t ab = off[a], da = end[a] - ab;
-        const uint32_t want = 4 * da;  // slots: pow2 >= 4 da, at most kTcHashSlots
-        const int lg = min(32 - __clz((int)(want - 1)), 11);
-        const uint32_t S = 1u << lg, mask = S - 1;
-        const int sh = 32 - lg;
-        for (uint32_t k = lane; k < S; k += kWave) keys[k] = kTcEmpty;
-        for (uint32_t k = lane; k < S / 2; k += kWave) cw[k] = 0u;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t *A = adj + ab;
-        for (uint32_t k = lane; k < da; k += kWave) {
-            const uint32_t x = A[k];
-            uint32_t h = tc_slot(x, sh);
-            while (atomicCAS(&keys[h], kTcEmpty, x) != kTcEmpty) h = (h + 1) & mask;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        uint32_t acc_a = 0;
-        // the last element of N+(a) closes no triangle here (no w above it)
-        for (uint32_t bc = 0; bc + 1 < da; bc += kWave) {
-            const uint32_t k = bc + lane;
-            const bool valid = k + 1 < da;
-            const uint32_t b = valid ? A[k] : 0u;
-            const uint32_t bb = valid ? off[b] : 0u;
-            const uint32_t lb = valid ? end[b] - bb : 0u;
-            const uint32_t nb = min((uint32_t)kWave, da - 1 - bc);
-            // The first 64 entries of N+(b_j) are loaded one b ahead (slots w2[0],
-            // w2[1] in turn), so that b_j's probes overlap b_{j+1}'s loads.
-            uint32_t w2[2];
-            w2[0] = tc_first_w(adj, bb, lb, 0, lane);
-            for (uint32_t j0 = 0; j0 < nb; j0 += 2) {  // loads unconditional (clamped j), uses not
-                w2[1] = tc_first_w(adj, bb, lb, min(j0 + 1, nb - 1), lane);
-                acc_a += tc_count_b(adj, keys, cw, mask, sh, b, bb, lb, j0, w2[0], lane);
-                w2[0] = tc_first_w(adj, bb, lb, min(j0 + 2, nb - 1), lane);
-                if (j0 + 1 < nb) acc_a += tc_count_b(adj, keys, cw, mask, sh, b, bb, lb, j0 + 1, w2[1], lane);
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)va, l);
+            const uint32_t ab = (uint32_t)__builtin_amdgcn_readlane((int)vb, l);
+            const uint32_t da = (uint32_t)__builtin_amdgcn_readlane((int)ve, l) - ab;
+            bits[lane] = bits[lane + kWave] = 0u;
+            tc_lds_sync();
+            for (uint32_t k = lane; k < da; k += kWave) {
+                const uint32_t x = adj[ab + k], h = tc_filter(x);
+                A[k] = x;
+                C[k] = 0u;
+                atomicOr(&bits[h >> 5], 1u << (h & 31));
             }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t k = lane; k < S; k += kWave) {
-            const uint32_t key = keys[k];
-            const uint32_t c = (cw[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-            if (key != kTcEmpty && c) atomicAdd(&cnt[key], (unsigned long long)c);
-        }
-        if (lane == 0 && acc_a) atomicAdd(&cnt[a], (unsigned long long)acc_a);
-        acc_total += acc_a;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+            tc_lds_sync();
+            uint32_t acc_a = 0;
+            for (uint32_t bc = 0; bc + 1 < da; bc += kWave) {  // the last neighbour has no w above it
+                const bool valid = bc + lane + 1 < da;
+                const uint32_t b = valid ? A[bc + lane] : 0u;
+                const uint32_t bb = valid ? off[b] : 0u;
+                const uint32_t lb = valid ? end[b] - bb : 0u;
+                const uint32_t pre = tc_scan_sum(lb);
+                const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)pre, kWave - 1);
+                const uint32_t first = pre - lb;  // b's first pair
+                const uint32_t shift = bb - first;
+                hitc[lane] = 0u;
+                uint32_t carry = 0;  // 1 + lane of the b that the last pair so far belongs to
+                for (uint32_t p0 = 0; p0 < tot; p0 += kTcTailStep * kWave) {
+#pragma unroll
+                    for (int u = 0; u < kTcTailStep; u++) mark[u * kWave + lane] = 0u;
+                    tc_lds_sync();
+                    if (lb && first - p0 < (uint32_t)(kTcTailStep * kWave)) mark[first - p0] = (uint32_t)lane + 1;
+                    tc_lds_sync();
+                    uint32_t w[kTcTailStep], j[kTcTailStep];
+#pragma unroll
+                    for (int u = 0; u < kTcTailStep; u++) {
+                        const uint32_t m = max(tc_scan_max(mark[u * kWave + lane]), carry);
+                        carry = (uint32_t)__builtin_amdgcn_readlane((int)m, kWave - 1);
+                        j[u] = m - 1;
+                        const uint32_t p = p0 + u * kWave + lane;
+                        const uint32_t at = (uint32_t)__shfl((int)shift, (int)j[u], kWave) + p;
+                        w[u] = p < tot ? adj[at] : n;
+                    }
+#pragma unroll
+                    for (int u = 0; u < kTcTailStep; u++) {
+                        const uint32_t h = tc_filter(w[u]);
+                        if (w[u] < n && ((bits[h >> 5] >> (h & 31)) & 1u)) {
+                            // w > b, which is entry bc + j of N+(a)
+                            const int k = bsearch_u32(A, bc + j[u] + 1, da, w[u]);
+                            if (k >= 0) {
+                                atomicAdd(&C[k], 1u);
+                                atomicAdd(&hitc[j[u]], 1u);
+                            }
+                        }
+                    }
+                    tc_lds_sync();
+                }
+                tc_lds_sync();
+                const uint32_t c = hitc[lane];
+                if (c) atomicAdd(&C[bc + lane], c);
+                acc_a += c;
+                tc_lds_sync();
+            }
+            for (uint32_t k = lane; k < da; k += kWave) {
+                const uint32_t c = C[k];
+                if (c) atomicAdd(&cnt[A[k]], (unsigned long long)c);
+            }
+            acc_a = wave_sum(acc_a);  // at most kTcTailMax^2 / 2
+            if (lane == 0 && acc_a) atomicAdd(&cnt[a], (unsigned long long)acc_a);
+            acc_total += acc_a;
+            tc_lds_sync();
         }
     }
-    if (lane == 0 && acc_total) atomicAdd(total, acc_total);
+    if (lane == 0 && acc_total) atomicAdd(&s_total, acc_total);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_total) atomicAdd(total, s_total);
 }
 
 // ---- the core: triangles whose highest vertex w is among the kTcCore highest ranks ----
@@ -411,20 +390,21 @@ __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(cons
 // kTcCore bits, 64 per lane: the w of (a, b) are one AND, their number one
 // popcount, and the credits of w vertical counters in registers (bit planes
 // summed with carry-save adders, flushed every 2^kTcPlanes bitmaps).  Bitmaps
-// are kept for the rows with more than kTcList core entries (below that the
-// list is shorter than the bitmap) of the highest ranks; the entries of other
+// are kept for the rows with more than kTcList core entries (one per lane: 762 us
+// at R-MAT scale 19, 811 with 128) of the highest ranks; the entries of other
 // rows are tested one by one against N+(a)'s bitmap in LDS.
 // Bound: vector instructions (about 25 per bitmap) and the L2 reads of the
-// bitmaps.  @@
+// bitmaps (512 bytes each; two sets of eight rows take turns so that one is in
+// flight).  R-MAT scale 19, 7.7M edges, 1.71G wedges: 752 us, and 34 for the
+// workgroups' credits; the hash table that looked up every wedge took 6312 us.
 constexpr uint32_t kTcCore = 4096;
 constexpr uint32_t kTcCoreWords = kTcCore / 32;
-constexpr uint32_t kTcList = 128;
+constexpr uint32_t kTcList = 64;
 constexpr uint32_t kTcMapRows = 1u << 18;   // at most 128 MiB of bitmaps
 constexpr uint32_t kTcNear = 16384;         // ranks whose b and w credits are counted in LDS
 constexpr int kTcCoreThreads = 512;
 constexpr int kTcCoreWaves = kTcCoreThreads / kWave;
 constexpr int kTcPlanes = 12;
-constexpr uint32_t kTcTicketCore = 8;       // vertices per ticket
 
 // end[v] = first entry of v's row in the core (rank >= base).
 __global__ void tc_core_split(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, uint32_t n,
@@ -491,21 +471,92 @@ GCHI_DEV void tc_planes_add(uint32_t (&p)[kTcPlanes], const uint32_t (&x)[8]) {
     }
 }
 
-// Sum over the wavefront, in lane 63.
-GCHI_DEV uint32_t tc_sum63(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
+// Eight bitmap rows in flight: rows of lanes j (of their b), `some` of them.
+struct TcRows {
+    uint32_t x0[8], x1[8], j[8], some;
+};
+
+GCHI_DEV void tc_rows_load(TcRows &g, uint64_t &m, uint32_t b, uint32_t first, const uint2 *__restrict__ maps,
+                           int lane) {
+    g.some = (uint32_t)__popcll(m);
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const bool on = (uint32_t)u < g.some;  // wavefront-uniform
+        g.j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
+        m &= m - (on ? 1ull : 0ull);
+        g.x0[u] = g.x1[u] = 0u;
+        if (on) {
+            const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)g.j[u]) - first;
+            const uint2 w = maps[(uint64_t)r * kWave + lane];
+            g.x0[u] = w.x;
+            g.x1[u] = w.y;
+        }
+    }
+}
+
+// ANDs the rows with N+(a) (a0, a1), adds them to the planes, and gives lane
+// j[u] the number of common bits of its row in tb.
+GCHI_DEV void tc_rows_count(TcRows &g, uint32_t a0, uint32_t a1, uint32_t (&p0)[kTcPlanes], uint32_t (&p1)[kTcPlanes],
+                            uint32_t &tb, int lane) {
+    uint32_t sum[4];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        g.x0[u] &= a0;
+        g.x1[u] &= a1;
+    }
+    tc_planes_add(p0, g.x0);
+    tc_planes_add(p1, g.x1);
+#pragma unroll
+    for (int u = 0; u < 4; u++)  // two counts (at most kTcCore each) per sum
+        sum[u] = tc_scan_sum((uint32_t)(__popc(g.x0[2 * u]) + __popc(g.x1[2 * u])) +
+                             ((uint32_t)(__popc(g.x0[2 * u + 1]) + __popc(g.x1[2 * u + 1])) << 16));
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const uint32_t both = (uint32_t)__builtin_amdgcn_readlane((int)sum[u / 2], kWave - 1);
+        const uint32_t c = u & 1 ? both >> 16 : both & 0xffffu;
+        if ((uint32_t)u < g.some) tb = (uint32_t)lane == g.j[u] ? c : tb;
+    }
+}
+
+// Eight short rows in flight, up to kTcList entries each.
+struct TcLists {
+    uint32_t w[8], j[8], some;
+};
+static_assert(kTcList <= kWave, "one entry per lane");
+
+GCHI_DEV void tc_lists_load(TcLists &g, uint64_t &m, uint32_t bs, uint32_t lb, const uint32_t *__restrict__ adj,
+                            uint32_t n, int lane) {
+    g.some = (uint32_t)__popcll(m);
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const bool on = (uint32_t)u < g.some;
+        g.j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
+        m &= m - (on ? 1ull : 0ull);
+        const uint32_t beg = (uint32_t)__builtin_amdgcn_readlane((int)bs, (int)g.j[u]);
+        const uint32_t len = on ? (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)g.j[u]) : 0u;
+        g.w[u] = (uint32_t)lane < len ? adj[beg + lane] : n;
+    }
+}
+
+GCHI_DEV void tc_lists_count(const TcLists &g, const uint32_t *bits, uint32_t *core, uint32_t base, uint32_t n,
+                             uint32_t &tb, int lane) {
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        bool hit = false;
+        if (g.w[u] < n) {
+            const uint32_t c = g.w[u] - base;
+            hit = (bits[c >> 5] >> (c & 31)) & 1u;
+            if (hit) atomicAdd(&core[c], 1u);
+        }
+        const uint32_t hits = (uint32_t)__popcll(__ballot(hit));
+        if ((uint32_t)u < g.some) tb = (uint32_t)lane == g.j[u] ? hits : tb;
+    }
 }
 
 __global__ __launch_bounds__(kTcCoreThreads, 4) void tc_count_core_kernel(
     const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, const uint32_t *__restrict__ end, uint32_t n,
     uint32_t base, uint32_t near, uint32_t first, const uint2 *__restrict__ maps, unsigned long long *cnt,
-    unsigned long long *total, uint32_t *work, uint32_t *__restrict__ slab) {
+    unsigned long long *total, uint32_t *__restrict__ slab) {
     __shared__ uint32_t s_near[kTcNear];  // credits of the ranks from near
     __shared__ uint32_t s_bits[kTcCoreWaves][kTcCoreWords];
     __shared__ unsigned long long s_total;
@@ -535,106 +586,83 @@ __global__ __launch_bounds__(kTcCoreThreads, 4) void tc_count_core_kernel(
         held = 0;
     };
     unsigned long long acc_total = 0;
-    uint32_t stripe = (blockIdx.x * kTcCoreWaves + wave) % kTcStripes, spent = 0;
-    for (;;) {
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(&work[stripe * kTcStripeGap], 1u);
-        t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
-        const uint64_t top = (stripe + (uint64_t)kTcStripes * t) * kTcTicketCore;
-        if (top >= n) {
-            if (++spent == kTcStripes) break;
-            stripe = (stripe + 1) % kTcStripes;
-            continue;
-        }
-        const uint32_t many = (uint32_t)min<uint64_t>(kTcTicketCore, n - top);
-        for (uint32_t q = 0; q < many; q++) {
-            const uint32_t a = n - 1 - (uint32_t)top - q;
-            const uint32_t ab = off[a], ac = end[a], ae = off[a + 1];
-            if (ae - ab < 2 || ac == ae) continue;
+    const uint64_t nw = (uint64_t)gridDim.x * kTcCoreWaves;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * kTcCoreWaves + wave; i0 < n; i0 += nw * kWave) {
+        const uint64_t mine = i0 + nw * lane;
+        const uint32_t va = mine < n ? n - 1 - (uint32_t)mine : 0u;
+        const uint32_t vb = mine < n ? off[va] : 0u, vc = mine < n ? end[va] : 0u, ve = mine < n ? off[va + 1] : 0u;
+        uint64_t todo = __ballot(ve - vb >= 2 && vc != ve);
+        while (todo) {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)va, l);
+            const uint32_t ab = (uint32_t)__builtin_amdgcn_readlane((int)vb, l);
+            const uint32_t ac = (uint32_t)__builtin_amdgcn_readlane((int)vc, l);
+            const uint32_t ae = (uint32_t)__builtin_amdgcn_readlane((int)ve, l);
+            uint32_t bnext = ab + lane + 1 < ae ? adj[ab + lane] : 0u;
             bits[lane] = bits[lane + kWave] = 0u;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            tc_lds_sync();
             for (uint32_t k = ac + lane; k < ae; k += kWave) {
                 const uint32_t c = adj[k] - base;
                 atomicOr(&bits[c >> 5], 1u << (c & 31));
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            tc_lds_sync();
             const uint32_t a0 = bits[2 * lane], a1 = bits[2 * lane + 1];
-            uint32_t acc_a = 0;  // per lane; a has at most 2^31 triangles here (at most E pairs of a lane's b)
+            uint32_t acc_a = 0;  // per lane: at most kTcCore per 64 neighbours of a
             for (uint32_t bc = ab; bc + 1 < ae; bc += kWave) {  // the last neighbour has no w above it
                 const bool valid = bc + lane + 1 < ae;
-                const uint32_t b = valid ? adj[bc + lane] : 0u;
+                const uint32_t b = bnext;
                 const uint32_t bs = valid ? end[b] : 0u;
                 const uint32_t lb = valid ? off[b + 1] - bs : 0u;
+                bnext = bc + kWave + lane + 1 < ae ? adj[bc + kWave + lane] : 0u;
                 const bool mapped = lb > kTcList && b >= first;
                 uint32_t tb = 0;  // triangles (a, b of this lane, w)
                 uint64_t m = __ballot(mapped);
-                while (m) {
-                    uint32_t x0[8], x1[8], j[8], sum[4];
-                    const uint32_t some = (uint32_t)__popcll(m);
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const bool on = (uint32_t)u < some;  // wavefront-uniform
-                        j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
-                        m &= m - (on ? 1ull : 0ull);
-                        x0[u] = x1[u] = 0u;
-                        if (on) {
-                            const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)j[u]) - first;
-                            const uint2 w = maps[(uint64_t)r * kWave + lane];
-                            x0[u] = w.x;
-                            x1[u] = w.y;
-                        }
+                if (m) {  // two sets of rows take turns: one loads while the other is counted
+                    TcRows ga, gb;
+                    tc_rows_load(ga, m, b, first, maps, lane);
+                    for (;;) {
+                        tc_rows_load(gb, m, b, first, maps, lane);
+                        tc_rows_count(ga, a0, a1, p0, p1, tb, lane);
+                        held += 8;
+                        if (!gb.some) break;
+                        tc_rows_load(ga, m, b, first, maps, lane);
+                        tc_rows_count(gb, a0, a1, p0, p1, tb, lane);
+                        held += 8;
+                        if (!ga.some) break;
                     }
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        x0[u] &= a0;
-                        x1[u] &= a1;
-                    }
-                    tc_planes_add(p0, x0);
-                    tc_planes_add(p1, x1);
-#pragma unroll
-                    for (int u = 0; u < 4; u++)  // two counts (at most kTcCore each) per sum
-                        sum[u] = tc_sum63((uint32_t)(__popc(x0[2 * u]) + __popc(x1[2 * u])) +
-                                          ((uint32_t)(__popc(x0[2 * u + 1]) + __popc(x1[2 * u + 1])) << 16));
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const uint32_t both = (uint32_t)__builtin_amdgcn_readlane((int)sum[u / 2], kWave - 1);
-                        const uint32_t c = u & 1 ? both >> 16 : both & 0xffffu;
-                        if ((uint32_t)u < some) tb = (uint32_t)lane == j[u] ? c : tb;
-                    }
-                    held += 8;
-                    if (held > (1u << kTcPlanes) - 16) flush();
+                    if (held > (1u << kTcPlanes) - 1 - kWave - 8) flush();  // room for the next 64 neighbours
                 }
-                // short rows: four at a time, the first 64 entries of each in flight together
-                m = __ballot(valid && !mapped && lb != 0);
+                m = __ballot(valid && !mapped && lb != 0 && lb <= kTcList);
+                if (m) {
+                    TcLists ga, gb;
+                    tc_lists_load(ga, m, bs, lb, adj, n, lane);
+                    for (;;) {
+                        tc_lists_load(gb, m, bs, lb, adj, n, lane);
+                        tc_lists_count(ga, bits, core, base, n, tb, lane);
+                        if (!gb.some) break;
+                        tc_lists_load(ga, m, bs, lb, adj, n, lane);
+                        tc_lists_count(gb, bits, core, base, n, tb, lane);
+                        if (!ga.some) break;
+                    }
+                }
+                m = __ballot(valid && !mapped && lb > kTcList);  // long rows below the bitmapped ranks
                 while (m) {
-                    uint32_t w[4], j[4], beg[4], len[4];
-                    const uint32_t some = (uint32_t)__popcll(m);
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const bool on = (uint32_t)u < some;
-                        j[u] = on ? (uint32_t)__builtin_ctzll(m) : 0u;
-                        m &= m - (on ? 1ull : 0ull);
-                        beg[u] = (uint32_t)__builtin_amdgcn_readlane((int)bs, (int)j[u]);
-                        len[u] = on ? (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j[u]) : 0u;
-                        w[u] = (uint32_t)lane < len[u] ? adj[beg[u] + lane] : n;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        uint32_t hits = 0;
-                        for (uint32_t k = 0; k < len[u]; k += kWave) {
-                            if (k) w[u] = k + lane < len[u] ? adj[beg[u] + k + lane] : n;
-                            bool hit = false;
-                            if (w[u] < n) {
-                                const uint32_t c = w[u] - base;
-                                hit = (bits[c >> 5] >> (c & 31)) & 1u;
-                                if (hit) atomicAdd(&core[c], 1u);
-                            }
-                            hits += (uint32_t)__popcll(__ballot(hit));
+                    const int j = __builtin_ctzll(m);
+                    m &= m - 1;
+                    const uint32_t beg = (uint32_t)__builtin_amdgcn_readlane((int)bs, j);
+                    const uint32_t len = (uint32_t)__builtin_amdgcn_readlane((int)lb, j);
+                    uint32_t hits = 0;
+                    for (uint32_t k = lane; k - lane < len; k += kWave) {
+                        bool hit = false;
+                        if (k < len) {
+                            const uint32_t c = adj[beg + k] - base;
+                            hit = (bits[c >> 5] >> (c & 31)) & 1u;
+                            if (hit) atomicAdd(&core[c], 1u);
                         }
-                        if ((uint32_t)u < some) tb = (uint32_t)lane == j[u] ? hits : tb;
+                        hits += (uint32_t)__popcll(__ballot(hit));
                     }
+                    tb = lane == j ? hits : tb;
                 }
                 if (tb) {
                     if (b >= near) atomicAdd(&s_near[b - near], tb);
@@ -645,6 +673,7 @@ __global__ __launch_bounds__(kTcCoreThreads, 4) void tc_count_core_kernel(
             const unsigned long long found = wave_sum((unsigned long long)acc_a);
             if (lane == 0 && found) atomicAdd(&cnt[a], found);
             acc_total += found;
+            tc_lds_sync();
         }
     }
     flush();
@@ -794,10 +823,9 @@ extern "C" int gchi_tc_prepare(const uint32_t *d_src, const uint32_t *d_dst, uin
 
 namespace gchi {
 
-// Scratch of one count.  rows = 0: no core kernel (only cnt, tot and wk are there).
+// Scratch of one count.  rows = 0: no core kernel (only cnt and tot are there).
 struct TcCount {
     unsigned long long *cnt, *tot;  // [n + 1], [1]
-    uint32_t *wk, *wk2;             // ticket stripes of the hash and the core kernel
     uint32_t *end, *slab;
     uint2 *maps;
     uint32_t rows, nwg;
@@ -817,27 +845,25 @@ static int tc_count_impl(const uint32_t *d_off, const uint32_t *d_adj, uint32_t 
     const uint32_t n = nvertices;
     launch_fill_u64(reinterpret_cast<uint64_t *>(w.cnt), 0ull, n, s);
     launch_fill_u64(reinterpret_cast<uint64_t *>(w.tot), 0ull, 1, s);
-    launch_fill_u32(w.wk, 0u, kTcStripes * kTcStripeGap, s);
     launch_fill_u32(d_overflow, 0u, 1, s);
     const int ncu = tc_ncu();
     const uint32_t *end = d_off + 1;
     if (w.rows) {
         const uint32_t base = n > kTcCore ? n - kTcCore : 0u, near = n > kTcNear ? n - kTcNear : 0u;
         const uint32_t first = n - w.rows;
-        launch_fill_u32(w.wk2, 0u, kTcStripes * kTcStripeGap, s);
         hipLaunchKernelGGL(tc_core_split, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, d_off, d_adj, n, base, w.end);
         hipLaunchKernelGGL(tc_core_maps, dim3(grid_for(w.rows, 4, 8192)), dim3(256), 0, s, d_off, d_adj, w.end, first,
                            w.rows, base, w.maps);
         hipLaunchKernelGGL(tc_count_core_kernel, dim3(w.nwg), dim3(kTcCoreThreads), 0, s, d_off, d_adj, w.end, n, base,
-                           near, first, w.maps, w.cnt, w.tot, w.wk2, w.slab);
+                           near, first, w.maps, w.cnt, w.tot, w.slab);
         hipLaunchKernelGGL(tc_core_sum, dim3(kTcNear / kWave), dim3(256), 0, s, w.slab, w.nwg, near, n, w.cnt);
         end = w.end;
     }
     if (!w.rows || n > kTcCore) {
-        hipLaunchKernelGGL(tc_count_hash_kernel, dim3(ncu * 6), dim3(kTcHashWaves * kWave), 0, s, d_off, end, d_adj, n,
-                           w.cnt, w.tot, w.wk);
+        hipLaunchKernelGGL(tc_count_tail_kernel, dim3(ncu * 6), dim3(kTcTailWaves * kWave), 0, s, d_off, end, d_adj, n,
+                           w.cnt, w.tot);
         hipLaunchKernelGGL(tc_count_kernel, dim3(ncu * 8), dim3(kTcWaves * kWave), 0, s, d_off, end, d_adj, n,
-                           kTcHashMax, w.cnt, w.tot);
+                           kTcTailMax, w.cnt, w.tot);
     }
     hipLaunchKernelGGL(tc_to_u32, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, w.cnt, n, d_per_vertex, d_overflow);
     GCHI_HIP(hipMemcpyAsync(d_total, w.tot, 8, hipMemcpyDeviceToDevice, s));
@@ -849,7 +875,6 @@ template <typename C>
 static void tc_count_layout(C &c, uint32_t nvertices, TcCount *w) {
     w->cnt = c.template take<unsigned long long>((size_t)nvertices + 1);
     w->tot = c.template take<unsigned long long>(1);
-    w->wk = c.template take<uint32_t>(kTcStripes * kTcStripeGap);
     w->rows = 0;
 }
 
@@ -860,7 +885,6 @@ template <typename C>
 static void tc_core_layout(C &c, uint32_t nvertices, TcCount *w) {
     w->rows = std::min(nvertices, std::min(kTcMapRows, std::max(nvertices / 8, kTcNear)));
     w->nwg = std::min<uint32_t>(2 * 256, std::max(1u, nvertices / 64));
-    w->wk2 = c.template take<uint32_t>(kTcStripes * kTcStripeGap);
     w->end = c.template take<uint32_t>(nvertices);
     w->slab = c.template take<uint32_t>((size_t)w->nwg * kTcNear);
     w->maps = c.template take<uint2>((size_t)w->rows * kWave);
@@ -870,7 +894,7 @@ static void tc_core_layout(C &c, uint32_t nvertices, TcCount *w) {
 // Counters for up to GCHI_TC_NOALLOC_MAX_VERTICES vertices, laid out as
 // tc_count_layout carves them (256-byte aligned pieces).
 constexpr size_t kTcScratchCounts = (((size_t)GCHI_TC_NOALLOC_MAX_VERTICES + 1) * 8 + 255) / 256 * 256;
-constexpr size_t kTcScratchBytes = kTcScratchCounts + 256 + (size_t)kTcStripes * kTcStripeGap * 4;
+constexpr size_t kTcScratchBytes = kTcScratchCounts + 256;
 static __device__ __align__(256) unsigned char scratch[kTcScratchBytes];
 
 // Device address of each device's copy of scratch (the array's name in host
@@ -932,7 +956,7 @@ extern "C" int gchi_tc_count_noalloc(const uint32_t *d_off, const uint32_t *d_ad
     GCHI_TRY(tc_scratch_setup(dev));
     Carver c(g_scratch_ptr[dev], kTcScratchBytes);
     TcCount w;
-    tc_count_layout(c, nvertices, &w);  // no bitmaps: the hash and search kernels alone
+    tc_count_layout(c, nvertices, &w);  // no bitmaps: the tail and search kernels alone
     GCHI_CHECK(c.ok(), GCHI_ERR_INVALID, "tc_count_noalloc: scratch layout exceeds its array");
     return tc_count_impl(d_off, d_adj, nvertices, d_per_vertex, d_total, d_overflow, w, as_stream(stream));
 }
