@@ -1672,8 +1672,9 @@ int pr_sweep_rank_space(const gchi_pr_plan *p, const gchi_pr_op *op, int src, in
 }
 
 struct PlanView {
-    uint32_t N, nblk, nhub, nchunk, npersist;
-    const uint32_t *reg_off, *reg_src, *blk_row, *hub_bits, *hub_v, *hub_chunk_off;
+    uint32_t N, nhub, nchunk;
+    uint64_t nedges;
+    const uint32_t *reg_off, *reg_src, *hub_bits, *hub_v, *hub_chunk_off;
     const uint64_t *chunk_beg;
     const uint32_t *chunk_len, *hub_src, *outdeg;
 };
@@ -1687,8 +1688,8 @@ int pr_plan_view(const gchi_pr_plan *p, PlanView *v) {
                                               "plan with persistent 0-3");
     GCHI_CHECK(!p->hot, GCHI_ERR_UNSUPPORTED, "plan view: the plan's edges hold gather-layout positions "
                                               "(hot_vertices != 0); build it with hot_vertices = 0");
-    *v = PlanView{p->N, p->nblk, p->nhub, p->nchunk, p->npersist, p->reg_off, p->reg_src, p->blk_row, p->hub_bits,
-                  p->hub_v, p->hub_chunk_off, p->chunk_beg, p->chunk_len, p->hub_src, p->outdeg};
+    *v = PlanView{p->N, p->nhub, p->nchunk, p->e_reg + p->e_hub, p->reg_off, p->reg_src, p->hub_bits, p->hub_v,
+                  p->hub_chunk_off, p->chunk_beg, p->chunk_len, p->hub_src, p->outdeg};
     return GCHI_OK;
 }
 

@@ -8,23 +8,29 @@
 // res_k = ||r_k - r_{k-1}||_1 the remaining error is at most
 // res_k * d / (1 - d); a query is converged when that bound is <= tol.
 //
-// Layout: 64 queries form a block; ranks are stored vertex-major, 64 values
-// per vertex (128 B in BF16, 256 B in FP32), so a wavefront owning one
-// destination row (lane = query) turns every in-edge into one coalesced row
-// gather shared by the 64 queries; the in-edge index stream is read once per
-// query block instead of once per query.  Rows come from the PageRank plan
-// (regular blocks of < 2W edges, hub rows cut into 512-edge chunks whose
-// 64-wide partials are combined in chunk order).  A persistent kernel pulls
-// (query block, tile) items, query-block-major, from kPpStripes device work
-// counters (stripe s hands out items s, s + kPpStripes, ...; each counter in
-// its own 128-byte line, since atomics on one address complete one after
-// another).
+// Layout: 64 queries form a block; ranks are stored row-major, 64 values per
+// vertex (128 B in BF16, 256 B in FP32), so every in-edge is one coalesced row
+// gather shared by the 64 queries and the in-edge stream is read once per query
+// block instead of once per query.  A last block of at most 32 queries has rows
+// of 4, 8, 16 or 32 values.  Vertices with in-edges come first, in id order,
+// then the others: a row without in-edges keeps its teleport value, written once.
+//
+// Work: the batch keeps the in-edges as one stream in row order (source
+// position, 1/outdeg), a bit per edge that ends its row, and cuts it into items
+// of S edges.  Every item is the same work whatever the row lengths are: a
+// wavefront walks an item's edges with 16 gathers in flight and 16 more behind
+// them, across row ends, and writes the rows that lie inside; the rows that
+// cross items are summed from their parts by ppr_split_kernel.  (The form
+// before took rows of up to 2W edges one at a time, a chain of five dependent
+// loads each, from tiles too coarse to fill the chip with a small graph.)
+// Bound: L2 and Infinity Cache reads of the rows in FP32, the wavefronts' issue
+// rate in BF16.  R-MAT scale 17, 2.1M edges, 130 queries (64 + 64 + 2), one
+// sweep: FP32 559 -> 107 us (1.07 GB of rows, 10 TB/s), BF16 501 -> 97 us, and
+// 14 for the rows that cross items.
 //
 // Precision: phase 1 stores ranks in BF16 with FP32 accumulation; phase 2
 // converts to FP32 and refines with FP32 sweeps until every query meets the
 // tolerance.  The per-query L1 residuals are FP64 sums.
-#include <type_traits>
-
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -35,30 +41,48 @@
 namespace gchi {
 // plan internals shared with pagerank.hip
 struct PlanView {
-    uint32_t N, nblk, nhub, nchunk, npersist;
-    const uint32_t *reg_off, *reg_src, *blk_row, *hub_bits, *hub_v, *hub_chunk_off;
+    uint32_t N, nhub, nchunk;
+    uint64_t nedges;
+    const uint32_t *reg_off, *reg_src, *hub_bits, *hub_v, *hub_chunk_off;
     const uint64_t *chunk_beg;
     const uint32_t *chunk_len, *hub_src, *outdeg;
 };
 int pr_plan_view(const gchi_pr_plan *p, PlanView *v);
+
+// Kernel arguments: the batch's stream and tables.
+struct PpArgs {
+    const uint32_t *src;       // [E, padded] position of each edge's source
+    const float *w;            // [E, padded] 1 / outdeg of the source (0 in the padding)
+    const uint64_t *ends;      // bit e: edge e is the last of its row
+    const uint32_t *item;      // [nitems] position of the row of the item's first edge, | kPpMid when the row began before
+    const uint32_t *split;     // [nitems] row that begins in the item and goes on in the next; kPpNone
+    const uint32_t *rstart;    // [K + 1] first edge of row k
+    const uint32_t *pos, *vert;  // vertex -> position, position -> vertex
+    const uint32_t *seedk;     // [nqb][kwords] bit k: row k is a seed of the block
+    const uint32_t *seed_v, *seed_q, *seed_n;
+    const float *tele;
+    float *part;               // [nqb][nitems][2][64] head and tail sums of the rows that cross items
+    double *res;
+    const uint32_t *active;    // query blocks still swept; active[nqb] = their count
+    uint32_t N, K, S, nitems, kwords, nqb;
+    int lq;                    // the last block's rows have 2^lq values (6: like the others)
+    uint64_t E;
+    float damping;
+};
 }  // namespace gchi
 
 struct gchi_ppr_batch {
-    gchi::PlanView pv;
-    uint32_t nq = 0, nqb = 0;
-    float *inv_outdeg = nullptr;   // [N]
+    gchi::PpArgs a{};
+    uint32_t nq = 0, nqb = 0, N = 0;
     void *r16[2] = {nullptr, nullptr};  // [nqb][N][64] bf16
     float *r32[2] = {nullptr, nullptr};  // [nqb][N][64] fp32
-    float *hub_part = nullptr;     // [nqb][nchunk][64]
     double *res = nullptr;         // [nqb*64]
-    uint32_t *seed_bits = nullptr; // [nqb][words]
+    uint32_t *seedk = nullptr;
     uint32_t *seed_v = nullptr;    // [nqb][64*64] sorted (vertex, query)
     uint32_t *seed_q = nullptr;
     uint32_t *seed_n = nullptr;    // [nqb]
     float *tele = nullptr;         // [nqb*64] restart mass per seed
-    uint32_t *counter = nullptr;
     uint32_t *active = nullptr;    // [nqb] query blocks still swept, then their count at [nqb]
-    size_t words = 0;
     int cur = 0;                   // buffer holding the current ranks
     int ncu = 256;
     bool fp32 = false;
@@ -76,10 +100,10 @@ namespace gchi {
 constexpr int kPpThreads = 256;
 constexpr int kPpWaves = kPpThreads / kWave;
 constexpr int kQ = 64;                 // queries per block (one per lane)
-constexpr uint32_t kPpStripes = 16;    // work counters of the persistent sweep
-constexpr uint32_t kPpStripeGap = 32;  // uint32 words between counters
 constexpr int kMaxSeeds = 64;          // restart-set size limit per query
 constexpr int kSeedTable = kQ * kMaxSeeds;
+constexpr uint32_t kPpMid = 0x80000000u;
+constexpr uint32_t kPpNone = 0xffffffffu;
 
 GCHI_DEV float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 GCHI_DEV uint16_t f32_to_bf16(float f) {  // round to nearest even
@@ -103,25 +127,12 @@ struct Store<float> {
     static GCHI_DEV void st(float *p, float f) { *p = f; }
 };
 
-struct PpArgs {
-    PlanView pv;
-    const float *inv;
-    const uint32_t *seed_bits, *seed_v, *seed_q, *seed_n;
-    const float *tele;
-    float *hub_part;
-    double *res;
-    uint32_t *counter;
-    const uint32_t *active;  // query blocks still swept; active[nqb] = their count
-    size_t words;
-    uint32_t nqb;
-    float damping;
-    int residual;
-};
+// log2 of the values per row of query block qb; offset of its state
+GCHI_DEV int pp_lq(const PpArgs &a, uint32_t qb) { return qb + 1 == a.nqb ? a.lq : 6; }
+GCHI_DEV size_t pp_base(const PpArgs &a, uint32_t qb) { return (size_t)qb * a.N * kQ; }
 
-// restart mass of (v, lane) in query block qb
-GCHI_DEV float seed_mass(const PpArgs &a, uint32_t qb, uint32_t v, int lane) {
-    const uint32_t *bits = a.seed_bits + qb * a.words;
-    if (!((bits[v >> 5] >> (v & 31)) & 1u)) return 0.0f;
+// restart mass of (vertex v, query q of block qb), v known to be a seed of the block
+GCHI_DEV float seed_mass(const PpArgs &a, uint32_t qb, uint32_t v, uint32_t q) {
     const uint32_t *sv = a.seed_v + (size_t)qb * kSeedTable;
     const uint32_t *sq = a.seed_q + (size_t)qb * kSeedTable;
     uint32_t lo = 0, hi = a.seed_n[qb];
@@ -132,272 +143,331 @@ GCHI_DEV float seed_mass(const PpArgs &a, uint32_t qb, uint32_t v, int lane) {
     }
     float m = 0.0f;
     for (uint32_t k = lo; k < a.seed_n[qb] && sv[k] == v; k++)
-        if (sq[k] == (uint32_t)lane) m = a.tele[qb * kQ + lane];
+        if (sq[k] == q) m = a.tele[qb * kQ + q];
     return m;
 }
 
-// sum over in-edges [beg, end) of r_u * inv_u for this lane's query
-template <typename T>
-GCHI_DEV float gather_rows_1(const uint32_t *src_idx, uint32_t beg, uint32_t end, const float *inv, const T *R,
-                           int lane) {
+GCHI_DEV bool is_seed(const PpArgs &a, uint32_t qb, uint32_t k) {
+    return (a.seedk[(size_t)qb * a.kwords + (k >> 5)] >> (k & 31)) & 1u;
+}
+
+GCHI_DEV float lane_f(float v, uint32_t l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)l));
+}
+
+// What a wavefront knows of its item while it walks it (wavefront-uniform).
+struct PpWalk {
+    uint32_t k;       // row in progress
+    bool mid;         // it began before the item
+    uint32_t sw;      // seed bits of the rows 32 * (k / 32) ..
+};
+
+// The 64-edge groups of an item: source positions and weights of one group in
+// lanes, the next group's loads in flight behind it.
+struct PpGroup {
+    uint32_t my, ny;
+    float mw, nw;
+    uint64_t f, nf;   // row ends
+};
+
+GCHI_DEV void pp_groups_open(const PpArgs &a, uint64_t e0, PpGroup &g, int lane) {
+    g.my = __builtin_nontemporal_load(a.src + e0 + lane);
+    g.mw = __builtin_nontemporal_load(a.w + e0 + lane);
+    g.ny = __builtin_nontemporal_load(a.src + e0 + kWave + lane);  // padded past E
+    g.nw = __builtin_nontemporal_load(a.w + e0 + kWave + lane);
+    g.f = a.ends[e0 >> 6];
+    g.nf = a.ends[(e0 >> 6) + 1];
+}
+
+GCHI_DEV void pp_groups_next(const PpArgs &a, uint64_t e, PpGroup &g, int lane) {  // e: first edge of the new current group
+    g.my = g.ny;
+    g.mw = g.nw;
+    g.f = g.nf;
+    g.ny = __builtin_nontemporal_load(a.src + e + kWave + lane);
+    g.nw = __builtin_nontemporal_load(a.w + e + kWave + lane);
+    g.nf = a.ends[(e >> 6) + 1];
+}
+
+// One item of 64 queries: lane = query, one row per load, two sets of 16 in
+// flight.  (BF16 rows, two per load with half a wavefront each, took 174 us where
+// this form took 141 with the same launch: the selects and shuffles cost more
+// than the loads they save.  Sets of 4 / 8 / 16: 133 / 110 / 107 us in FP32.)
+template <typename T, bool RES>
+GCHI_DEV void pp_item(const PpArgs &a, uint32_t qb, uint32_t i, const T *__restrict__ Rin, T *__restrict__ Rout,
+                      int lane, double *res) {
+    constexpr uint32_t kSet = 16, kPerGroup = kWave / kSet;
+    struct Set {
+        float v[kSet], w[kSet];  // w is wavefront-uniform
+        uint32_t f;
+    };
+    const uint64_t e0 = (uint64_t)i * a.S;
+    const uint32_t n = (uint32_t)min<uint64_t>(a.S, a.E - e0), nb = (n + kSet - 1) / kSet;
+    const uint32_t *sk = a.seedk + (size_t)qb * a.kwords;
+    float *part = a.part + ((size_t)qb * a.nitems + i) * 2 * kQ + lane;
+    PpGroup g;
+    pp_groups_open(a, e0, g, lane);
+    PpWalk k{a.item[i] & ~kPpMid, (a.item[i] & kPpMid) != 0, 0u};
+    k.sw = sk[k.k >> 5];
+    auto load = [&](Set &s, uint32_t b) {
+        if (b >= nb) return;
+        if (b && b % kPerGroup == 0) pp_groups_next(a, e0 + (uint64_t)kSet * b, g, lane);
+        const uint32_t j = b % kPerGroup * kSet;
+        s.f = (uint32_t)(g.f >> j) & ((1u << kSet) - 1u);
+#pragma unroll
+        for (uint32_t q = 0; q < kSet; q++) {
+            const uint32_t id = (uint32_t)__builtin_amdgcn_readlane((int)g.my, (int)(j + q));
+            s.w[q] = lane_f(g.mw, j + q);
+            s.v[q] = Store<T>::ld(Rin + (size_t)id * kQ + lane);
+        }
+    };
+    float acc = 0.0f, rn = 0.0f, ro = 0.0f;  // rn, ro: the row before, its residual not yet added
+    auto end_row = [&]() {
+        if (k.mid) {
+            part[0] = acc;
+            k.mid = false;
+        } else {
+            float m = 0.0f;
+            if ((k.sw >> (k.k & 31)) & 1u) m = seed_mass(a, qb, a.vert[k.k], (uint32_t)lane);
+            if (RES) *res += fabs((double)rn - (double)ro);
+            rn = Store<T>::round(m + a.damping * acc);
+            if (RES) ro = Store<T>::ld(Rin + (size_t)k.k * kQ + lane);
+            Store<T>::st(Rout + (size_t)k.k * kQ + lane, rn);
+        }
+        acc = 0.0f;
+        k.k++;
+        if ((k.k & 31) == 0) k.sw = sk[k.k >> 5];
+    };
+    auto count = [&](const Set &s) {
+        if (s.f == 0) {
+#pragma unroll
+            for (uint32_t q = 0; q < kSet; q++) acc += s.v[q] * s.w[q];
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < kSet; q++) {
+                acc += s.v[q] * s.w[q];
+                if ((s.f >> q) & 1u) end_row();
+            }
+        }
+    };
+    Set sa, sb;
+    load(sa, 0);
+    for (uint32_t b = 0;; b += 2) {
+        load(sb, b + 1);
+        count(sa);
+        if (b + 1 >= nb) break;
+        load(sa, b + 2);
+        count(sb);
+        if (b + 2 >= nb) break;
+    }
+    if (RES) *res += fabs((double)rn - (double)ro);
+    // the row in progress: its first edge lies in this item (tail) or before (head)
+    const uint64_t last = e0 + n - 1;
+    if (!((a.ends[last >> 6] >> (last & 63)) & 1u)) part[k.mid ? 0 : kQ] = acc;
+}
+
+// 64 >> lq items, one per group of 2^lq lanes, for a last block of few queries.
+// Each group walks its own item, 8 edges at a time.
+template <typename T, bool RES>
+GCHI_DEV void pp_items_narrow(const PpArgs &a, uint32_t qb, uint32_t first, const T *__restrict__ Rin,
+                              T *__restrict__ Rout, int lane, double *res) {
+    const int lq = a.lq;
+    const uint32_t q = (uint32_t)lane & ((1u << lq) - 1u), i = first + ((uint32_t)lane >> lq);
+    const bool on = i < a.nitems;
+    const uint64_t e0 = on ? (uint64_t)i * a.S : 0ull;
+    const uint32_t n = on ? (uint32_t)min<uint64_t>(a.S, a.E - e0) : 0u;
+    float *part = a.part + ((size_t)qb * a.nitems + (on ? i : 0u)) * 2 * kQ + q;
+    const uint32_t meta = on ? a.item[i] : 0u;
+    uint32_t k = meta & ~kPpMid;
+    bool mid = (meta & kPpMid) != 0;
+    const uint8_t *ends = reinterpret_cast<const uint8_t *>(a.ends) + e0 / 8;
     float acc = 0.0f;
-    for (uint32_t e = beg; e < end; e += kWave) {
-        const uint32_t n = min((uint32_t)kWave, end - e);
-        const uint32_t my = lane < (int)n ? __builtin_nontemporal_load(&src_idx[e + lane]) : 0u;
-        const float myi = lane < (int)n ? inv[my] : 0.0f;
-        uint32_t j = 0;
-        // 8 row gathers in flight per wavefront; the additions stay in edge order
-        for (; j + 8 <= n; j += 8) {
-            float v[8], w[8];
+    for (uint32_t j = 0; j < n; j += 8) {
+        const uint4 i0 = *reinterpret_cast<const uint4 *>(a.src + e0 + j);
+        const uint4 i1 = *reinterpret_cast<const uint4 *>(a.src + e0 + j + 4);
+        const float4 w0 = *reinterpret_cast<const float4 *>(a.w + e0 + j);
+        const float4 w1 = *reinterpret_cast<const float4 *>(a.w + e0 + j + 4);
+        const uint32_t id[8] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w};
+        const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+        const uint32_t f = ends[j / 8];
+        float v[8];
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const uint32_t sq = __builtin_amdgcn_readlane(my, j + q);
-                w[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + q));
-                v[q] = Store<T>::ld(R + (size_t)sq * kQ + lane);
-            }
+        for (int u = 0; u < 8; u++) v[u] = Store<T>::ld(Rin + ((size_t)id[u] << lq) + q);
 #pragma unroll
-            for (int q = 0; q < 8; q++) acc += v[q] * w[q];
-        }
-        for (; j + 4 <= n; j += 4) {
-            uint32_t s0 = __builtin_amdgcn_readlane(my, j), s1 = __builtin_amdgcn_readlane(my, j + 1);
-            uint32_t s2 = __builtin_amdgcn_readlane(my, j + 2), s3 = __builtin_amdgcn_readlane(my, j + 3);
-            float i0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j));
-            float i1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 1));
-            float i2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 2));
-            float i3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 3));
-            float v0 = Store<T>::ld(R + (size_t)s0 * kQ + lane);
-            float v1 = Store<T>::ld(R + (size_t)s1 * kQ + lane);
-            float v2 = Store<T>::ld(R + (size_t)s2 * kQ + lane);
-            float v3 = Store<T>::ld(R + (size_t)s3 * kQ + lane);
-            acc += v0 * i0;
-            acc += v1 * i1;
-            acc += v2 * i2;
-            acc += v3 * i3;
-        }
-        for (; j < n; j++) {
-            uint32_t s0 = __builtin_amdgcn_readlane(my, j);
-            float i0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j));
-            acc += Store<T>::ld(R + (size_t)s0 * kQ + lane) * i0;
-        }
-    }
-    return acc;
-}
-
-// BF16 rows: a 64-query row is 128 bytes, so one load instruction can carry
-// two edges.  Lanes 0-31 take the even edges of the row (counted from beg),
-// lanes 32-63 the odd ones; lane 32h + p loads queries 2p and 2p+1 of its
-// edge's source row as one 32-bit word.  Each query's sum is its even-edge
-// sum plus its odd-edge sum (both in edge order), combined at the end and
-// moved to lane q for query q.
-GCHI_DEV float bf16_lo(uint32_t v) { return __uint_as_float(v << 16); }
-GCHI_DEV float bf16_hi(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
-
-GCHI_DEV float gather_rows_bf16x2(const uint32_t *src_idx, uint32_t beg, uint32_t end, const float *inv,
-                                  const uint16_t *R, int lane) {
-    const bool odd = lane >= 32;
-    const int p = lane & 31;
-    const uint32_t *R32 = reinterpret_cast<const uint32_t *>(R);  // row s: words s*32 .. s*32+31
-    float a0 = 0.0f, a1 = 0.0f;
-    for (uint32_t e = beg; e < end; e += kWave) {
-        const uint32_t n = min((uint32_t)kWave, end - e);
-        const uint32_t my = lane < (int)n ? __builtin_nontemporal_load(&src_idx[e + lane]) : 0u;
-        const float myi = lane < (int)n ? inv[my] : 0.0f;
-        uint32_t j = 0;
-        for (; j + 16 <= n; j += 16) {  // 8 edge pairs in flight
-            uint32_t v[8];
-            float w[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const uint32_t s0 = __builtin_amdgcn_readlane(my, j + 2 * q);
-                const uint32_t s1 = __builtin_amdgcn_readlane(my, j + 2 * q + 1);
-                const float w0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 2 * q));
-                const float w1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 2 * q + 1));
-                w[q] = odd ? w1 : w0;
-                v[q] = R32[(size_t)(odd ? s1 : s0) * (kQ / 2) + p];
-            }
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                a0 += bf16_lo(v[q]) * w[q];
-                a1 += bf16_hi(v[q]) * w[q];
-            }
-        }
-        for (; j + 2 <= n; j += 2) {
-            const uint32_t s0 = __builtin_amdgcn_readlane(my, j), s1 = __builtin_amdgcn_readlane(my, j + 1);
-            const float w0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j));
-            const float w1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j + 1));
-            const float w = odd ? w1 : w0;
-            const uint32_t v = R32[(size_t)(odd ? s1 : s0) * (kQ / 2) + p];
-            a0 += bf16_lo(v) * w;
-            a1 += bf16_hi(v) * w;
-        }
-        if (j < n) {  // the chunk's last edge is even: the odd half loads it and discards it
-            const uint32_t s0 = __builtin_amdgcn_readlane(my, j);
-            const float w0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myi), j));
-            const uint32_t v = R32[(size_t)s0 * (kQ / 2) + p];
-            if (!odd) {
-                a0 += bf16_lo(v) * w0;
-                a1 += bf16_hi(v) * w0;
+        for (int u = 0; u < 8; u++) {
+            acc += v[u] * w[u];
+            if ((f >> u) & 1u) {
+                if (mid) {
+                    part[0] = acc;
+                    mid = false;
+                } else {
+                    float m = 0.0f;
+                    if (is_seed(a, qb, k)) m = seed_mass(a, qb, a.vert[k], q);
+                    const float rn = Store<T>::round(m + a.damping * acc);
+                    const size_t at = ((size_t)k << lq) + q;
+                    if (RES) *res += fabs((double)rn - (double)Store<T>::ld(Rin + at));
+                    Store<T>::st(Rout + at, rn);
+                }
+                acc = 0.0f;
+                k++;
             }
         }
     }
-    // query 2p: even part (lane p) + odd part (lane 32 + p), in that order
-    const float o0 = __shfl_xor(a0, 32, kWave), o1 = __shfl_xor(a1, 32, kWave);
-    const float t0 = odd ? o0 + a0 : a0 + o0;
-    const float t1 = odd ? o1 + a1 : a1 + o1;
-    const float u0 = __shfl(t0, lane >> 1, kWave), u1 = __shfl(t1, lane >> 1, kWave);
-    return (lane & 1) ? u1 : u0;
+    if (on) {
+        const uint64_t last = e0 + n - 1;
+        if (!((a.ends[last >> 6] >> (last & 63)) & 1u)) part[mid ? 0 : kQ] = acc;
+    }
 }
 
-template <typename T>
-GCHI_DEV float gather_rows(const uint32_t *src_idx, uint32_t beg, uint32_t end, const float *inv, const T *R,
-                           int lane) {
-    if constexpr (std::is_same<T, uint16_t>::value)
-        return gather_rows_bf16x2(src_idx, beg, end, inv, R, lane);
-    else
-        return gather_rows_1<T>(src_idx, beg, end, inv, R, lane);
+// The units of a sweep: the narrow block's first (its chains are the longest),
+// then kPpWaves items of one query block each, block by block.
+struct PpUnits {
+    uint32_t narrow, wide, total;  // units of the narrow block; of every wide one; of all
+};
+
+GCHI_DEV PpUnits pp_units(const PpArgs &a, uint32_t per_wave_wide, uint32_t items) {
+    const uint32_t nact = a.active[a.nqb];
+    const bool nar = a.lq < 6 && nact && a.active[nact - 1] == a.nqb - 1;
+    PpUnits u;
+    const uint32_t group = per_wave_wide * kPpWaves;
+    u.wide = (items + group - 1) / group;
+    u.narrow = nar ? (items + (group << (6 - a.lq)) - 1) / (group << (6 - a.lq)) : 0u;
+    u.total = u.narrow + (nact - (nar ? 1u : 0u)) * u.wide;
+    return u;
 }
 
-template <typename T>
+// Adds the workgroup's residuals of block qb to the global ones.
+GCHI_DEV void pp_flush_res(const PpArgs &a, uint32_t qb, double *s_res) {
+    __syncthreads();
+    if (threadIdx.x < kQ) {
+        const double v = s_res[threadIdx.x];
+        if (v != 0.0) atomicAdd(&a.res[qb * kQ + threadIdx.x], v);
+        s_res[threadIdx.x] = 0.0;
+    }
+    __syncthreads();
+}
+
+template <typename T, bool RES>
 __global__ __launch_bounds__(kPpThreads) void ppr_sweep_kernel(PpArgs a, const T *__restrict__ Rin_all,
                                                               T *__restrict__ Rout_all) {
-    __shared__ float s_part[kPpWaves][kQ];
     __shared__ double s_res[kQ];
-    __shared__ uint32_t s_tile;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const uint32_t T_per_qb = a.pv.nchunk + a.pv.nblk;
-    const uint32_t nact = a.active[a.nqb];
-    const uint32_t ntiles = T_per_qb * nact;
-    const size_t stride_q = (size_t)a.pv.N * kQ;
-    uint32_t cur_qb = 0xffffffffu;
-    double res = 0.0;  // this lane's query, accumulated by this wave for cur_qb
-    if (threadIdx.x < kQ) s_res[threadIdx.x] = 0.0;
-    uint32_t stripe = blockIdx.x % kPpStripes, spent = 0;
-    for (;;) {
-        uint32_t t = ntiles;  // the next tile from the stripes; ntiles once all are drained
-        while (spent < kPpStripes) {  // block-uniform
-            if (threadIdx.x == 0) s_tile = atomicAdd(&a.counter[stripe * kPpStripeGap], 1u);
-            __syncthreads();
-            const uint64_t t64 = stripe + (uint64_t)kPpStripes * s_tile;
-            __syncthreads();  // s_tile is rewritten by the next ticket
-            if (t64 < ntiles) {
-                t = (uint32_t)t64;
-                break;
-            }
-            spent++;
-            stripe = (stripe + 1) % kPpStripes;
-        }
-        const uint32_t qi = t < ntiles ? t / T_per_qb : 0xffffffffu;  // index into the active list
-        const uint32_t qb = t < ntiles ? a.active[qi] : 0xffffffffu;
-        if (qb != cur_qb) {  // block-uniform: every thread read the same tile
-            if (a.residual && cur_qb != 0xffffffffu) {
-                // add the waves' residuals in wave order, then one atomic per query
-                for (int w = 0; w < kPpWaves; w++) {
-                    if (wave == w) s_res[lane] += res;
-                    __syncthreads();
-                }
-                if (wave == 0) {
-                    const double v = s_res[lane];
-                    if (v != 0.0) atomicAdd(&a.res[cur_qb * kQ + lane], v);
-                    s_res[lane] = 0.0;
-                }
-                __syncthreads();
-            }
-            res = 0.0;
-            cur_qb = qb;
-        }
-        if (t >= ntiles) break;
-        const uint32_t lt = t - qi * T_per_qb;
-        const T *Rin = Rin_all + qb * stride_q;
-        T *Rout = Rout_all + qb * stride_q;
-        if (lt < a.pv.nchunk) {
-            // hub chunk: 4 waves split <= 512 edges, partials combined in wave order
-            const uint64_t cb = a.pv.chunk_beg[lt];
-            const uint32_t cl = a.pv.chunk_len[lt];
-            const uint32_t per = (cl + kPpWaves - 1) / kPpWaves;
-            const uint32_t b0 = min(cl, per * wave), b1 = min(cl, per * (wave + 1));
-            float acc = gather_rows<T>(a.pv.hub_src + cb, b0, b1, a.inv, Rin, lane);
-            s_part[wave][lane] = acc;
-            __syncthreads();
-            if (wave == 0) {
-                float t4 = 0.0f;
-                for (int w = 0; w < kPpWaves; w++) t4 += s_part[w][lane];
-                a.hub_part[((size_t)qb * a.pv.nchunk + lt) * kQ + lane] = t4;
-            }
-            __syncthreads();
-            continue;
-        }
-        const uint32_t b = lt - a.pv.nchunk;
-        const uint32_t rb = a.pv.blk_row[b], re = a.pv.blk_row[b + 1];
-        for (uint32_t v = rb + wave; v < re; v += kPpWaves) {
-            if ((a.pv.hub_bits[v >> 5] >> (v & 31)) & 1u) continue;
-            float acc = gather_rows<T>(a.pv.reg_src, a.pv.reg_off[v], a.pv.reg_off[v + 1], a.inv, Rin, lane);
-            float rn = Store<T>::round(seed_mass(a, qb, v, lane) + a.damping * acc);
-            if (a.residual) res += fabs((double)rn - (double)Store<T>::ld(Rin + (size_t)v * kQ + lane));
-            Store<T>::st(Rout + (size_t)v * kQ + lane, rn);
-        }
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const PpUnits un = pp_units(a, 1, a.nitems);
+    uint32_t cur = kPpNone;
+    if (RES) {
+        if (threadIdx.x < kQ) s_res[threadIdx.x] = 0.0;
         __syncthreads();
     }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kPpThreads) void ppr_hub_kernel(PpArgs a, const T *__restrict__ Rin_all,
-                                                            T *__restrict__ Rout_all) {
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const uint32_t nw = gridDim.x * kPpWaves;
-    const size_t stride_q = (size_t)a.pv.N * kQ;
-    const uint32_t items = a.pv.nhub * a.active[a.nqb];
-    // residuals summed per wavefront while its items stay in one query block,
-    // then one atomic per query (not one per hub row and query)
-    double racc = 0.0;
-    uint32_t rqb = 0xffffffffu;
-    for (uint32_t it = blockIdx.x * kPpWaves + wave; it < items; it += nw) {
-        const uint32_t qb = a.active[it / a.pv.nhub], h = it % a.pv.nhub;
-        if (a.residual && qb != rqb) {  // wavefront-uniform
-            if (rqb != 0xffffffffu && racc != 0.0) atomicAdd(&a.res[rqb * kQ + lane], racc);
-            racc = 0.0;
-            rqb = qb;
+    for (uint32_t u = blockIdx.x; u < un.total; u += gridDim.x) {
+        const bool nar = u < un.narrow;
+        const uint32_t t = u - un.narrow, qi = nar ? 0u : t / un.wide;
+        const uint32_t qb = nar ? a.nqb - 1 : a.active[qi];
+        if (RES && qb != cur && cur != kPpNone) pp_flush_res(a, cur, s_res);  // block-uniform
+        cur = qb;
+        const T *Rin = Rin_all + pp_base(a, qb);
+        T *Rout = Rout_all + pp_base(a, qb);
+        double res = 0.0;
+        if (nar) {
+            pp_items_narrow<T, RES>(a, qb, (u * kPpWaves + wave) << (6 - a.lq), Rin, Rout, lane, &res);
+            if (RES) atomicAdd(&s_res[lane & ((1 << a.lq) - 1)], res);
+        } else {
+            const uint32_t i = (t - qi * un.wide) * kPpWaves + wave;
+            if (i < a.nitems) pp_item<T, RES>(a, qb, i, Rin, Rout, lane, &res);
+            if (RES) atomicAdd(&s_res[lane], res);
         }
-        const uint32_t c0 = a.pv.hub_chunk_off[h], c1 = a.pv.hub_chunk_off[h + 1];
-        // the chunk partials added in chunk order, 16 loads in flight
-        const float *part = a.hub_part + (size_t)qb * a.pv.nchunk * kQ + lane;
-        float acc = 0.0f;
-        for (uint32_t c = c0; c < c1; c += 16) {
-            float pv[16];
-#pragma unroll
-            for (uint32_t q = 0; q < 16; q++) pv[q] = part[(size_t)min(c + q, c1 - 1) * kQ];
-#pragma unroll
-            for (uint32_t q = 0; q < 16; q++)
-                if (c + q < c1) acc += pv[q];
-        }
-        const uint32_t v = a.pv.hub_v[h];
-        const T *Rin = Rin_all + qb * stride_q;
-        T *Rout = Rout_all + qb * stride_q;
-        float rn = Store<T>::round(seed_mass(a, qb, v, lane) + a.damping * acc);
-        if (a.residual) racc += fabs((double)rn - (double)Store<T>::ld(Rin + (size_t)v * kQ + lane));
-        Store<T>::st(Rout + (size_t)v * kQ + lane, rn);
     }
-    if (a.residual && rqb != 0xffffffffu && racc != 0.0) atomicAdd(&a.res[rqb * kQ + lane], racc);
-    if (blockIdx.x == 0)  // work queue ready for the next sweep
-        for (uint32_t i = threadIdx.x; i < kPpStripes; i += blockDim.x) a.counter[i * kPpStripeGap] = 0u;
+    if (RES && cur != kPpNone) pp_flush_res(a, cur, s_res);
 }
 
-template <typename T>
-__global__ void ppr_init_kernel(PpArgs a, T *R) {
-    // r = teleport vector: zero everything, then the seeds
-    const size_t total = (size_t)a.nqb * a.pv.N * kQ;
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const size_t qb = i / ((size_t)a.pv.N * kQ);
-        const size_t rem = i - qb * ((size_t)a.pv.N * kQ);
-        const uint32_t v = (uint32_t)(rem / kQ), lane = (uint32_t)(rem % kQ);
-        float m = 0.0f;
-        const uint32_t *bits = a.seed_bits + qb * a.words;
-        if ((bits[v >> 5] >> (v & 31)) & 1u) {
-            const uint32_t *sv = a.seed_v + qb * kSeedTable, *sq = a.seed_q + qb * kSeedTable;
-            for (uint32_t k = 0; k < a.seed_n[qb]; k++)
-                if (sv[k] == v && sq[k] == lane) m = a.tele[qb * kQ + lane];
+// The rows that cross items: the first item's tail, then the heads of the items
+// after it up to the row's last, added in that order, 16 loads in flight.
+template <typename T, bool RES>
+__global__ __launch_bounds__(kPpThreads) void ppr_split_kernel(PpArgs a, const T *__restrict__ Rin_all,
+                                                              T *__restrict__ Rout_all) {
+    __shared__ double s_res[kQ];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    constexpr uint32_t kPer = 4;  // items per wavefront (or group) and unit: about half have such a row
+    const PpUnits un = pp_units(a, kPer, a.nitems);
+    uint32_t cur = kPpNone;
+    if (RES) {
+        if (threadIdx.x < kQ) s_res[threadIdx.x] = 0.0;
+        __syncthreads();
+    }
+    for (uint32_t u = blockIdx.x; u < un.total; u += gridDim.x) {
+        const bool nar = u < un.narrow;
+        const uint32_t t = u - un.narrow, qi = nar ? 0u : t / un.wide;
+        const uint32_t qb = nar ? a.nqb - 1 : a.active[qi];
+        if (RES && qb != cur && cur != kPpNone) pp_flush_res(a, cur, s_res);
+        cur = qb;
+        const int lq = nar ? a.lq : 6;
+        const uint32_t q = (uint32_t)lane & ((1u << lq) - 1u), groups = 64u >> lq;
+        const T *Rin = Rin_all + pp_base(a, qb);
+        T *Rout = Rout_all + pp_base(a, qb);
+        const float *part = a.part + (size_t)qb * a.nitems * 2 * kQ + q;
+        const uint32_t unit = nar ? u : t - qi * un.wide;
+        const uint32_t i0 = ((unit * kPpWaves + wave) * groups + ((uint32_t)lane >> lq)) * kPer;
+        double res = 0.0;
+        for (uint32_t i = i0; i < min(i0 + kPer, a.nitems); i++) {
+            const uint32_t k = a.split[i];
+            if (k == kPpNone) continue;
+            const uint32_t il = (a.rstart[k + 1] - 1) / a.S;
+            float acc = part[(size_t)i * 2 * kQ + kQ];
+            for (uint32_t c = i + 1; c <= il; c += 16) {
+                float pv[16];
+#pragma unroll
+                for (uint32_t x = 0; x < 16; x++) pv[x] = part[(size_t)min(c + x, il) * 2 * kQ];
+#pragma unroll
+                for (uint32_t x = 0; x < 16; x++)
+                    if (c + x <= il) acc += pv[x];
+            }
+            float m = 0.0f;
+            if (is_seed(a, qb, k)) m = seed_mass(a, qb, a.vert[k], q);
+            const float rn = Store<T>::round(m + a.damping * acc);
+            const size_t at = ((size_t)k << lq) + q;
+            if (RES) res += fabs((double)rn - (double)Store<T>::ld(Rin + at));
+            Store<T>::st(Rout + at, rn);
         }
-        Store<T>::st(R + i, m);
+        if (RES && res != 0.0) atomicAdd(&s_res[q], res);
+    }
+    if (RES && cur != kPpNone) pp_flush_res(a, cur, s_res);
+}
+
+// ---- start values ----
+// r = teleport vector: R0 cleared (all rows, or only those without in-edges),
+// R1's rows without in-edges cleared; ppr_seed_kernel then writes the seeds.
+template <typename T>
+__global__ void ppr_clear_kernel(PpArgs a, T *__restrict__ R0, T *__restrict__ R1, int whole) {
+    struct __align__(4 * sizeof(T)) Four {
+        T x[4];
+    };
+    const Four zero = {};
+    for (uint32_t qb = blockIdx.y; qb < a.nqb; qb += gridDim.y) {
+        const int lq = pp_lq(a, qb);
+        const size_t n4 = ((size_t)a.N << lq) / 4, k4 = ((size_t)a.K << lq) / 4;  // rows of at least 4 values
+        Four *r0 = reinterpret_cast<Four *>(R0 + pp_base(a, qb)), *r1 = reinterpret_cast<Four *>(R1 + pp_base(a, qb));
+        const size_t stride = (size_t)gridDim.x * blockDim.x;
+        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x + (whole ? 0 : k4); i < n4; i += stride) {
+            r0[i] = zero;
+            if (i >= k4) r1[i] = zero;
+        }
+    }
+}
+
+// The seeds' masses: rows without in-edges in both buffers, the others in R0
+// (whole) with their bit in seedk.
+template <typename T>
+__global__ void ppr_seed_kernel(PpArgs a, T *__restrict__ R0, T *__restrict__ R1, uint32_t *seedk, int whole) {
+    for (uint32_t qb = blockIdx.x; qb < a.nqb; qb += gridDim.x) {
+        const int lq = pp_lq(a, qb);
+        for (uint32_t e = threadIdx.x; e < a.seed_n[qb]; e += blockDim.x) {
+            const uint32_t p = a.pos[a.seed_v[(size_t)qb * kSeedTable + e]];
+            const uint32_t q = a.seed_q[(size_t)qb * kSeedTable + e];
+            const size_t at = pp_base(a, qb) + ((size_t)p << lq) + q;
+            const float m = a.tele[qb * kQ + q];
+            if (whole || p >= a.K) Store<T>::st(R0 + at, m);
+            if (p >= a.K) Store<T>::st(R1 + at, m);
+            else atomicOr(&seedk[(size_t)qb * a.kwords + (p >> 5)], 1u << (p & 31));
+        }
     }
 }
 
@@ -406,51 +476,133 @@ __global__ void ppr_widen_kernel(const uint16_t *a, float *b, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) b[i] = bf16_to_f32(a[i]);
 }
 
-__global__ void inv_outdeg_kernel(const uint32_t *outdeg, uint32_t n, float *inv) {
+__global__ void ppr_extract_kernel(PpArgs a, const void *R, int fp32, uint32_t query, float *out) {
     uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride)
-        inv[v] = outdeg[v] ? 1.0f / (float)outdeg[v] : 0.0f;
-}
-
-__global__ void ppr_extract_kernel(const void *R, int fp32, uint32_t n, uint32_t q, float *out) {
-    uint32_t stride = gridDim.x * blockDim.x;
-    const size_t base = (size_t)(q / kQ) * n * kQ;
-    const uint32_t lane = q % kQ;
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
-        size_t i = base + (size_t)v * kQ + lane;
+    const uint32_t qb = query / kQ, q = query % kQ;
+    const int lq = pp_lq(a, qb);
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < a.N; v += stride) {
+        const size_t i = pp_base(a, qb) + ((size_t)a.pos[v] << lq) + q;
         out[v] = fp32 ? ((const float *)R)[i] : bf16_to_f32(((const uint16_t *)R)[i]);
     }
 }
 
-static PpArgs make_args(gchi_ppr_batch *b, float damping, int residual) {
-    PpArgs a;
-    a.pv = b->pv;
-    a.inv = b->inv_outdeg;
-    a.seed_bits = b->seed_bits;
-    a.seed_v = b->seed_v;
-    a.seed_q = b->seed_q;
-    a.seed_n = b->seed_n;
-    a.tele = b->tele;
-    a.hub_part = b->hub_part;
-    a.res = b->res;
-    a.counter = b->counter;
-    a.active = b->active;
-    a.words = b->words;
-    a.nqb = b->nqb;
+// ---- stream build (once per batch) ----
+GCHI_DEV bool pb_is_hub(const PlanView &p, uint32_t v) { return (p.hub_bits[v >> 5] >> (v & 31)) & 1u; }
+
+__global__ void pb_lengths(PlanView p, uint32_t *len, uint32_t *some) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < p.N; v += stride) {
+        if (p.nhub && pb_is_hub(p, v)) continue;
+        const uint32_t l = p.reg_off[v + 1] - p.reg_off[v];
+        len[v] = l;
+        some[v] = l != 0;
+    }
+}
+
+__global__ void pb_hub_lengths(PlanView p, uint32_t *len, uint32_t *some) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t h = blockIdx.x * blockDim.x + threadIdx.x; h < p.nhub; h += stride) {
+        const uint32_t c0 = p.hub_chunk_off[h], c1 = p.hub_chunk_off[h + 1];
+        const uint32_t l = c1 > c0 ? (uint32_t)(p.chunk_beg[c1 - 1] + p.chunk_len[c1 - 1] - p.chunk_beg[c0]) : 0u;
+        len[p.hub_v[h]] = l;
+        some[p.hub_v[h]] = l != 0;
+    }
+}
+
+// positions and row starts, and the row-end bits (cleared before)
+__global__ void pb_rows(uint32_t n, const uint32_t *len, const uint32_t *ord, const uint32_t *start, uint32_t *pos,
+                        uint32_t *vert, uint32_t *rstart, uint32_t *ends) {
+    const uint32_t stride = gridDim.x * blockDim.x, K = ord[n];
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
+        const uint32_t l = len[v], p = l ? ord[v] : K + (v - ord[v]);
+        pos[v] = p;
+        vert[p] = v;
+        if (l) {
+            rstart[p] = start[v];
+            const uint32_t e = start[v] + l - 1;
+            atomicOr(&ends[e >> 5], 1u << (e & 31));
+        }
+        if (v == 0) rstart[K] = start[n];
+    }
+}
+
+GCHI_DEV void pb_edge(const PlanView &p, const uint32_t *pos, uint32_t u, uint32_t e, uint32_t *src, float *w) {
+    src[e] = pos[u];
+    w[e] = p.outdeg[u] ? 1.0f / (float)p.outdeg[u] : 0.0f;
+}
+
+// 16 lanes per regular row
+__global__ void pb_regular(PlanView p, const uint32_t *pos, const uint32_t *start, uint32_t *src, float *w) {
+    const uint32_t l16 = threadIdx.x & 15u, stride = gridDim.x * blockDim.x / 16;
+    for (uint32_t v = (blockIdx.x * blockDim.x + threadIdx.x) / 16; v < p.N; v += stride) {
+        if (p.nhub && pb_is_hub(p, v)) continue;
+        const uint32_t b = p.reg_off[v], l = p.reg_off[v + 1] - b, s = start[v];
+        for (uint32_t k = l16; k < l; k += 16) pb_edge(p, pos, p.reg_src[b + k], s + k, src, w);
+    }
+}
+
+// one wavefront per hub chunk
+__global__ void pb_hubs(PlanView p, const uint32_t *pos, const uint32_t *start, uint32_t *src, float *w) {
+    const uint32_t lane = threadIdx.x & (kWave - 1), stride = gridDim.x * blockDim.x / kWave;
+    for (uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; c < p.nchunk; c += stride) {
+        uint32_t lo = 0, hi = p.nhub - 1;  // the chunk's hub: the last with hub_chunk_off[h] <= c
+        while (lo < hi) {
+            const uint32_t m = (lo + hi + 1) / 2;
+            if (p.hub_chunk_off[m] <= c) lo = m;
+            else hi = m - 1;
+        }
+        const uint64_t b = p.chunk_beg[c];
+        const uint32_t s = start[p.hub_v[lo]] + (uint32_t)(b - p.chunk_beg[p.hub_chunk_off[lo]]);
+        for (uint32_t k = lane; k < p.chunk_len[c]; k += kWave) pb_edge(p, pos, p.hub_src[b + k], s + k, src, w);
+    }
+}
+
+__global__ void pb_items(const uint32_t *rstart, const uint32_t *K_, uint32_t S, uint32_t nitems, uint32_t *item,
+                         uint32_t *split) {
+    const uint32_t stride = gridDim.x * blockDim.x, K = *K_;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nitems; i += stride) {
+        uint32_t at[2];
+        for (int s = 0; s < 2; s++) {  // the last row that begins at or before the item's first / last edge
+            const uint64_t e = s ? min<uint64_t>((uint64_t)(i + 1) * S, rstart[K]) - 1 : (uint64_t)i * S;
+            uint32_t lo = 0, hi = K - 1;
+            while (lo < hi) {
+                const uint32_t m = lo + (hi - lo + 1) / 2;
+                if (rstart[m] <= e) lo = m;
+                else hi = m - 1;
+            }
+            at[s] = lo;
+        }
+        item[i] = at[0] | ((uint64_t)rstart[at[0]] < (uint64_t)i * S ? kPpMid : 0u);
+        const bool begins = (uint64_t)rstart[at[1]] >= (uint64_t)i * S;
+        const bool goes_on = (uint64_t)rstart[at[1] + 1] > (uint64_t)(i + 1) * S;
+        split[i] = begins && goes_on ? at[1] : kPpNone;
+    }
+}
+
+static PpArgs make_args(const gchi_ppr_batch *b, float damping) {
+    PpArgs a = b->a;
     a.damping = damping;
-    a.residual = residual;
     return a;
+}
+
+template <typename T, bool RES>
+static void ppr_launch(gchi_ppr_batch *b, const PpArgs &a, const T *rin, T *rout, hipStream_t s) {
+    // more workgroups than fit at once: the hardware hands the later ones out as
+    // the first end (8 per CU, each looping over its units, took 153 us in FP32, 16
+    // 135, 32 110, one per unit 113)
+    const uint64_t units = (uint64_t)b->nqb * div_up(a.nitems, kPpWaves);
+    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(units, (uint64_t)b->ncu * 32));
+    const unsigned sgrid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(div_up(units, 4), (uint64_t)b->ncu * 32));
+    hipLaunchKernelGGL((ppr_sweep_kernel<T, RES>), dim3(grid), dim3(kPpThreads), 0, s, a, rin, rout);
+    hipLaunchKernelGGL((ppr_split_kernel<T, RES>), dim3(sgrid), dim3(kPpThreads), 0, s, a, rin, rout);
 }
 
 template <typename T>
 static int ppr_sweep(gchi_ppr_batch *b, const T *rin, T *rout, float damping, int residual, hipStream_t s) {
-    PpArgs a = make_args(b, damping, residual);
+    const PpArgs a = make_args(b, damping);
     if (residual) launch_fill_u64(reinterpret_cast<uint64_t *>(b->res), 0ull, (size_t)b->nqb * kQ, s);
-    const uint64_t tiles = (uint64_t)b->nqb * (b->pv.nblk + b->pv.nchunk);
-    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(tiles, (uint64_t)b->ncu * 8));
-    hipLaunchKernelGGL(ppr_sweep_kernel<T>, dim3(grid), dim3(kPpThreads), 0, s, a, rin, rout);
-    hipLaunchKernelGGL(ppr_hub_kernel<T>, dim3(grid_for((uint64_t)b->pv.nhub * b->nqb * kWave, kPpThreads, 2048) + 0),
-                       dim3(kPpThreads), 0, s, a, rin, rout);
+    if (residual) ppr_launch<T, true>(b, a, rin, rout, s);
+    else ppr_launch<T, false>(b, a, rin, rout, s);
     GCHI_LAUNCH_CHECK();
     return GCHI_OK;
 }
@@ -508,8 +660,8 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
     GCHI_CHECK(plan && out && nqueries > 0, GCHI_ERR_INVALID, "ppr_batch_create: bad argument");
     PlanView pv;
     GCHI_TRY(pr_plan_view(plan, &pv));  // before the batch exists: a refused plan leaks nothing
+    GCHI_CHECK(pv.N < kPpMid, GCHI_ERR_UNSUPPORTED, "ppr_batch_create: N must be < 2^31");
     gchi_ppr_batch *b = new gchi_ppr_batch();
-    b->pv = pv;
     b->nq = nqueries;
     {
         int dev = 0;
@@ -517,48 +669,117 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
             b->ncu = prop.multiProcessorCount;
     }
-    b->nqb = (nqueries + kQ - 1) / kQ;
-    b->words = (b->pv.N + 31) / 32;
-    const size_t state = (size_t)b->nqb * b->pv.N * kQ;
-    Sizer z;
-    z.take<float>(b->pv.N);
-    z.take<uint16_t>(state);
-    z.take<uint16_t>(state);
-    z.take<float>(state);
-    z.take<float>(state);
-    z.take<float>((size_t)b->nqb * std::max<uint32_t>(b->pv.nchunk, 1) * kQ);
-    z.take<double>((size_t)b->nqb * kQ);
-    z.take<uint32_t>((size_t)b->nqb * b->words);
-    z.take<uint32_t>((size_t)b->nqb * kSeedTable);
-    z.take<uint32_t>((size_t)b->nqb * kSeedTable);
-    z.take<uint32_t>(b->nqb);
-    z.take<float>((size_t)b->nqb * kQ);
-    z.take<uint32_t>(kPpStripes * kPpStripeGap);
-    z.take<uint32_t>((size_t)b->nqb + 1);
-    if (hipMalloc(&b->mem, z.off) != hipSuccess) {
+    const uint32_t N = pv.N, nqb = (nqueries + kQ - 1) / kQ;
+    const uint64_t E = pv.nedges;
+    b->nqb = nqb;
+    b->N = N;
+    PpArgs &a = b->a;
+    a.N = N;
+    a.nqb = nqb;
+    a.E = E;
+    // the last block's row: the power of two that holds its queries, at least 4 (8-byte rows in BF16)
+    const uint32_t rest = nqueries - (nqb - 1) * kQ;
+    a.lq = 2;
+    while ((1u << a.lq) < rest) a.lq++;
+    // edges per item: about four items per resident wavefront, so that the last
+    // round of items is short, within [64, 512] (longer items have fewer rows
+    // that cross them and amortise their first loads)
+    const uint64_t slots = (uint64_t)b->ncu * 8 * kPpWaves * 4;
+    const uint64_t lanes = E * ((uint64_t)(nqb - 1) * kQ + (1u << a.lq)) / kQ;
+    a.S = (uint32_t)std::min<uint64_t>(512, std::max<uint64_t>(1, lanes / slots / 64) * 64);
+    a.nitems = (uint32_t)div_up(E, a.S);
+    a.kwords = N / 32 + 1;
+    const size_t state = (size_t)nqb * N * kQ, epad = (size_t)E + 2 * a.S + 2 * kWave;
+    auto lay = [&](auto &c, auto get) {
+        get(0, c.template take<uint32_t>(epad));              // src
+        get(1, c.template take<float>(epad));                 // w
+        get(2, c.template take<uint64_t>(epad / 64 + 2));     // ends
+        get(3, c.template take<uint32_t>(a.nitems + 1));      // item
+        get(4, c.template take<uint32_t>(a.nitems + 1));      // split
+        get(5, c.template take<uint32_t>((size_t)N + 1));     // rstart
+        get(6, c.template take<uint32_t>(N));                 // pos
+        get(7, c.template take<uint32_t>(N));                 // vert
+        get(8, c.template take<uint32_t>((size_t)nqb * a.kwords));  // seedk
+        get(9, c.template take<uint32_t>((size_t)nqb * kSeedTable));
+        get(10, c.template take<uint32_t>((size_t)nqb * kSeedTable));
+        get(11, c.template take<uint32_t>(nqb));
+        get(12, c.template take<float>((size_t)nqb * kQ));    // tele
+        get(13, c.template take<float>((size_t)nqb * a.nitems * 2 * kQ + 1));  // part
+        get(14, c.template take<double>((size_t)nqb * kQ));   // res
+        get(15, c.template take<uint32_t>((size_t)nqb + 1));  // active
+        get(16, c.template take<uint16_t>(state));
+        get(17, c.template take<uint16_t>(state));
+        get(18, c.template take<float>(state));
+        get(19, c.template take<float>(state));
+        // build scratch
+        get(20, c.template take<uint32_t>((size_t)N + 1));    // len
+        get(21, c.template take<uint32_t>((size_t)N + 1));    // some
+        get(22, c.template take<uint32_t>((size_t)N + 1));    // ord
+        get(23, c.template take<uint32_t>((size_t)N + 1));    // start
+        get(24, c.template take<char>(scan_workspace((size_t)N + 1)));
+    };
+    SizerAdapter za;
+    lay(za, [](int, void *) {});
+    if (hipMalloc(&b->mem, za.z.off) != hipSuccess) {
         delete b;
-        return fail(GCHI_ERR_HIP, "ppr_batch_create: hipMalloc failed (state " + std::to_string(z.off) + " bytes)");
+        return fail(GCHI_ERR_HIP, "ppr_batch_create: hipMalloc failed (state " + std::to_string(za.z.off) + " bytes)");
     }
-    Carver c(b->mem, z.off);
-    b->inv_outdeg = c.take<float>(b->pv.N);
-    b->r16[0] = c.take<uint16_t>(state);
-    b->r16[1] = c.take<uint16_t>(state);
-    b->r32[0] = c.take<float>(state);
-    b->r32[1] = c.take<float>(state);
-    b->hub_part = c.take<float>((size_t)b->nqb * std::max<uint32_t>(b->pv.nchunk, 1) * kQ);
-    b->res = c.take<double>((size_t)b->nqb * kQ);
-    b->seed_bits = c.take<uint32_t>((size_t)b->nqb * b->words);
-    b->seed_v = c.take<uint32_t>((size_t)b->nqb * kSeedTable);
-    b->seed_q = c.take<uint32_t>((size_t)b->nqb * kSeedTable);
-    b->seed_n = c.take<uint32_t>(b->nqb);
-    b->tele = c.take<float>((size_t)b->nqb * kQ);
-    b->counter = c.take<uint32_t>(kPpStripes * kPpStripeGap);
-    b->active = c.take<uint32_t>((size_t)b->nqb + 1);
-    hipLaunchKernelGGL(inv_outdeg_kernel, dim3(grid_for(b->pv.N, 256, 65536)), dim3(256), 0, 0, b->pv.outdeg, b->pv.N,
-                       b->inv_outdeg);
-    launch_fill_u32(b->counter, 0u, kPpStripes * kPpStripeGap, 0);
-    GCHI_LAUNCH_CHECK();
-    GCHI_HIP(hipDeviceSynchronize());
+    void *m[25];
+    Carver c(b->mem, za.z.off);
+    lay(c, [&](int k, void *q) { m[k] = q; });
+    auto u32 = [&](int k) { return static_cast<uint32_t *>(m[k]); };
+    float *w = static_cast<float *>(m[1]);
+    a.src = u32(0);
+    a.w = w;
+    a.ends = static_cast<uint64_t *>(m[2]);
+    a.item = u32(3);
+    a.split = u32(4);
+    a.rstart = u32(5);
+    a.pos = u32(6);
+    a.vert = u32(7);
+    a.seedk = b->seedk = u32(8);
+    a.seed_v = b->seed_v = u32(9);
+    a.seed_q = b->seed_q = u32(10);
+    a.seed_n = b->seed_n = u32(11);
+    a.tele = b->tele = static_cast<float *>(m[12]);
+    a.part = static_cast<float *>(m[13]);
+    a.res = b->res = static_cast<double *>(m[14]);
+    a.active = b->active = u32(15);
+    b->r16[0] = m[16];
+    b->r16[1] = m[17];
+    b->r32[0] = static_cast<float *>(m[18]);
+    b->r32[1] = static_cast<float *>(m[19]);
+    uint32_t *len = u32(20), *some = u32(21), *ord = u32(22), *start = u32(23);
+    const size_t swb = scan_workspace((size_t)N + 1);
+    auto build = [&]() -> int {
+        const dim3 gv(grid_for(N, 256, 65536)), blk(256);
+        launch_fill_u32(u32(2), 0u, 2 * (epad / 64 + 2), 0);
+        launch_fill_u32(u32(0) + E, 0u, epad - E, 0);
+        launch_fill_u32(reinterpret_cast<uint32_t *>(w) + E, 0u, epad - E, 0);
+        hipLaunchKernelGGL(pb_lengths, gv, blk, 0, 0, pv, len, some);
+        if (pv.nhub) hipLaunchKernelGGL(pb_hub_lengths, dim3(grid_for(pv.nhub, 256, 65536)), blk, 0, 0, pv, len, some);
+        GCHI_TRY(exclusive_scan_u32(some, ord, N, m[24], swb, 0));
+        GCHI_TRY(exclusive_scan_u32(len, start, N, m[24], swb, 0));
+        hipLaunchKernelGGL(pb_rows, gv, blk, 0, 0, N, len, ord, start, u32(6), u32(7), u32(5), u32(2));
+        hipLaunchKernelGGL(pb_regular, dim3(grid_for((uint64_t)N * 16, 256, 65536)), blk, 0, 0, pv, u32(6), start,
+                           u32(0), w);
+        if (pv.nchunk)
+            hipLaunchKernelGGL(pb_hubs, dim3(grid_for((uint64_t)pv.nchunk * kWave, 256, 65536)), blk, 0, 0, pv, u32(6),
+                               start, u32(0), w);
+        if (a.nitems)
+            hipLaunchKernelGGL(pb_items, dim3(grid_for(a.nitems, 256, 65536)), blk, 0, 0, u32(5), ord + N, a.S,
+                               a.nitems, u32(3), u32(4));
+        GCHI_LAUNCH_CHECK();
+        GCHI_HIP(hipMemcpyAsync(&a.K, ord + N, 4, hipMemcpyDeviceToHost, 0));
+        GCHI_HIP(hipDeviceSynchronize());
+        return GCHI_OK;
+    };
+    const int st = build();
+    if (st != GCHI_OK) {
+        (void)hipFree(b->mem);
+        delete b;
+        return st;
+    }
     *out = b;
     return GCHI_OK;
 }
@@ -581,10 +802,9 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
     GCHI_CHECK(b && h_seed_off && h_seeds && cfg && result, GCHI_ERR_INVALID, "ppr_batch_run: null argument");
     GCHI_CHECK(cfg->damping > 0 && cfg->damping < 1 && cfg->tol > 0, GCHI_ERR_INVALID, "ppr_batch_run: bad config");
     hipStream_t s = as_stream(stream);
-    const uint32_t nqb = b->nqb, N = b->pv.N;
+    const uint32_t nqb = b->nqb, N = b->N;
     // seed tables (host-built, uploaded once per run)
-    std::vector<uint32_t> bits((size_t)nqb * b->words, 0), sv((size_t)nqb * kSeedTable, 0),
-        sq((size_t)nqb * kSeedTable, 0), sn(nqb, 0);
+    std::vector<uint32_t> sv((size_t)nqb * kSeedTable, 0), sq((size_t)nqb * kSeedTable, 0), sn(nqb, 0);
     std::vector<float> tele((size_t)nqb * kQ, 0.0f);
     for (uint32_t q = 0; q < b->nq; q++) {
         uint32_t k0 = h_seed_off[q], k1 = h_seed_off[q + 1];
@@ -598,7 +818,6 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
         tele[q] = (float)((1.0 - cfg->damping) / (double)seeds.size());
         for (uint32_t v : seeds) {
             GCHI_CHECK(v < N, GCHI_ERR_INVALID, "ppr_batch_run: seed out of range");
-            bits[(size_t)qb * b->words + (v >> 5)] |= 1u << (v & 31);
             size_t slot = (size_t)qb * kSeedTable + sn[qb]++;
             sv[slot] = v;
             sq[slot] = lane;
@@ -613,7 +832,6 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
             sq[(size_t)qb * kSeedTable + k] = t[k].second;
         }
     }
-    GCHI_HIP(hipMemcpyAsync(b->seed_bits, bits.data(), bits.size() * 4, hipMemcpyHostToDevice, s));
     GCHI_HIP(hipMemcpyAsync(b->seed_v, sv.data(), sv.size() * 4, hipMemcpyHostToDevice, s));
     GCHI_HIP(hipMemcpyAsync(b->seed_q, sq.data(), sq.size() * 4, hipMemcpyHostToDevice, s));
     GCHI_HIP(hipMemcpyAsync(b->seed_n, sn.data(), sn.size() * 4, hipMemcpyHostToDevice, s));
@@ -645,12 +863,16 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
         return m;
     };
     result->sweeps_bf16 = result->sweeps_fp32 = result->block_sweeps_fp32 = 0;
-    PpArgs a0 = make_args(b, d, 0);
+    const PpArgs a0 = make_args(b, d);
+    const dim3 cgrid(std::max(1u, 4096 / std::min(nqb, 64u)), std::min(nqb, 64u)), sgrid(std::min(nqb, 1024u));
+    launch_fill_u32(b->seedk, 0u, (size_t)nqb * a0.kwords, s);
     int sweeps = 0;
     b->cur = 0;
     b->fp32 = cfg->bf16_sweeps <= 0;
     if (!b->fp32) {
-        hipLaunchKernelGGL(ppr_init_kernel<uint16_t>, dim3(65536), dim3(256), 0, s, a0, (uint16_t *)b->r16[0]);
+        uint16_t *r0 = (uint16_t *)b->r16[0], *r1 = (uint16_t *)b->r16[1];
+        hipLaunchKernelGGL(ppr_clear_kernel<uint16_t>, cgrid, dim3(256), 0, s, a0, r0, r1, 1);
+        hipLaunchKernelGGL(ppr_seed_kernel<uint16_t>, sgrid, dim3(256), 0, s, a0, r0, r1, b->seedk, 1);
         GCHI_LAUNCH_CHECK();
         GCHI_TRY(ppr_capture_chunk(b, 0, check, d));
         double prev = 1e300;
@@ -667,12 +889,14 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
         const size_t state = (size_t)nqb * N * kQ;
         hipLaunchKernelGGL(ppr_widen_kernel, dim3(65536), dim3(256), 0, s, (const uint16_t *)b->r16[0], b->r32[0],
                            state);
-        GCHI_LAUNCH_CHECK();
         b->fp32 = true;
-    } else {
-        hipLaunchKernelGGL(ppr_init_kernel<float>, dim3(65536), dim3(256), 0, s, a0, b->r32[0]);
-        GCHI_LAUNCH_CHECK();
     }
+    // FP32 teleport values of the rows without in-edges in both buffers; of all
+    // rows when there was no BF16 phase
+    const int whole = cfg->bf16_sweeps <= 0;
+    hipLaunchKernelGGL(ppr_clear_kernel<float>, cgrid, dim3(256), 0, s, a0, b->r32[0], b->r32[1], whole);
+    hipLaunchKernelGGL(ppr_seed_kernel<float>, sgrid, dim3(256), 0, s, a0, b->r32[0], b->r32[1], b->seedk, whole);
+    GCHI_LAUNCH_CHECK();
     GCHI_TRY(ppr_capture_chunk(b, 1, check, d));
     bool converged = false;
     while (sweeps + check <= max_sweeps) {
@@ -711,8 +935,8 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
 extern "C" int gchi_ppr_batch_extract(const gchi_ppr_batch *b, uint32_t query, float *d_out, void *stream) {
     GCHI_CHECK(b && d_out && query < b->nq, GCHI_ERR_INVALID, "ppr_batch_extract: bad argument");
     const void *R = b->fp32 ? (const void *)b->r32[b->cur] : b->r16[b->cur];
-    hipLaunchKernelGGL(ppr_extract_kernel, dim3(grid_for(b->pv.N, 256, 65536)), dim3(256), 0, as_stream(stream), R,
-                       b->fp32 ? 1 : 0, b->pv.N, query, d_out);
+    hipLaunchKernelGGL(ppr_extract_kernel, dim3(grid_for(b->N, 256, 65536)), dim3(256), 0, as_stream(stream), b->a, R,
+                       b->fp32 ? 1 : 0, query, d_out);
     GCHI_LAUNCH_CHECK();
     return GCHI_OK;
 }

@@ -108,3 +108,44 @@ def test_batched_ppr_retires_converged_blocks(dev):
         r64, _ = oracle.ppr_f64(n, in_off, in_src, outdeg, queries[q], D)
         assert np.abs(r - r64).sum() <= TOL, q
     assert (resid * D / (1 - D) <= TOL).all()
+
+
+@pytest.mark.parametrize("nq", [1, 4, 5, 16, 17, 33, 64, 66, 100, 129])
+def test_batched_ppr_block_widths(dev, nq):
+    """Every width of the last query block (4, 8, 16, 32 and 64 values per row),
+    alone and behind full blocks, on a graph with hub rows, rows that cross
+    items, rows without in-edges (seeds among them) and a ragged edge count;
+    FP32 alone and behind BF16, against the plain FP32 form at the same
+    tolerance (both stop at a residual bound of TOL, so 2 TOL apart at most)."""
+    rng = np.random.default_rng(nq)
+    n = 3001
+    src = np.concatenate([rng.integers(0, n, 9001), rng.integers(0, n, 5000), np.arange(700)]).astype(np.uint32)
+    dst = np.concatenate([rng.integers(0, n // 2, 9001), np.full(5000, 17), np.full(700, 1400)]).astype(np.uint32)
+    src, dst = graphs.preprocess(src, dst)
+    g = dev.DeviceGraph(dev.to_dev_u32(src), dev.to_dev_u32(dst), n)
+    plan = dev.PageRankPlan(g, edges_per_block=2048, persistent=1)
+    queries = random_queries(n, nq, nq + 1)
+    queries[0] = np.array([n - 1, n - 2, 17], np.uint32)  # two seeds without in-edges, one a hub
+    plain = dev.PlainPpr(plan, D)
+    b = dev.PprBatch(plan, nq)
+    for bf16 in (60, 0):
+        info, resid = b.run(queries, D, TOL, bf16_sweeps=bf16)
+        assert info["converged"] == 1 and (resid * D / (1 - D) <= TOL).all()
+        for q in sorted({0, nq // 2, nq - 1}):
+            r = b.ranks(q).cpu().numpy().astype(np.float64)
+            rp, _ = plain.run(queries[q], TOL)
+            assert np.abs(r - rp.cpu().numpy()).sum() <= 2 * TOL, (q, bf16)
+
+
+def test_batched_ppr_graph_without_edges(dev):
+    """No in-edges at all: every rank is its teleport value."""
+    e = dev.to_dev_u32(np.zeros(0, np.uint32))
+    g = dev.DeviceGraph(e, e, 40)
+    plan = dev.PageRankPlan(g, edges_per_block=2048, persistent=1)
+    b = dev.PprBatch(plan, 3)
+    info, _ = b.run([np.array([q, q + 5], np.uint32) for q in range(3)], D, TOL)
+    assert info["converged"] == 1
+    for q in range(3):
+        want = np.zeros(40, np.float32)
+        want[[q, q + 5]] = np.float32((1 - D) / 2)
+        np.testing.assert_array_equal(b.ranks(q).cpu().numpy(), want)
