@@ -142,7 +142,7 @@ def sweep_kernels(info):
     """Kernel names of one sweep of the plan (what rocprofv3 lists)."""
     if info["persistent"] == 4:  # rank space: no per-sweep layout refresh
         return "pr_seg_sweep_kernel + pr_seg_finalize_kernel"
-    main = {0: "pr_sweep_kernel", 1: "pr_sweep_persistent_kernel", 2: "pr_sweep_wave_kernel",
+    main = {0: "pr_sweep_kernel", 1: "pr_sweep_kernel", 2: "pr_sweep_wave_kernel",
             3: "pr_sweep_hotwg_kernel"}[info["persistent"]]
     ks = ([] if not info["gather_sources"] else ["pr_gather_layout_kernel"]) + [main]
     ks += ["pr_finalize_kernel"] if info["ngraphs"] == 1 else ["pr_hub_apply_kernel", "pr_graph_reduce_kernel"]
@@ -333,7 +333,7 @@ def bench_multigraph(gchi, torch, ngraphs, sweeps, seed=9):
     """Many graphs of uneven size in one plan: each graph's CSC is built on its
     own (local ids), the batch plan copies them side by side (64-bit offsets
     across graphs, so the total may exceed 2^32 edges), and every sweep of all
-    graphs is one launch of the persistent sweep kernel plus the finalize pair."""
+    graphs is one launch of the sweep kernel plus the finalize pair."""
     graphs, ns = [], []
     for scale, ne, gseed in gchi.multigraph_workload(ngraphs, seed):
         s, d, cnt, mx = gchi.rmat_device(scale, ne, gseed)

@@ -2,7 +2,7 @@
 //
 // Candidates: edges per regular block W (which also sets the hub threshold),
 // the one-lane-per-row threshold, the launch form (one workgroup per tile,
-// persistent workgroups, or persistent wavefronts), and (N < 2^30) the
+// or persistent wavefronts), and (N < 2^30) the
 // out-degree gather layout with and without an LDS cache of the most
 // referenced source values, and the rank-space tiled sweep (form 4).  Each
 // candidate gets its own plan on the caller's graph and is
@@ -50,11 +50,10 @@ extern "C" int gchi_autotune_pr(const gchi_dgraph *g, int sweeps_per_candidate, 
     const int reps = sweeps_per_candidate > 0 ? sweeps_per_candidate : 4;
     std::vector<gchi_pr_tune> cand;
     for (int W : {512, 1024, 2048, 4096})
-        for (int sm : {8, 16, 32, 64})
-            for (int pers : {0, 1}) {
-                if (2 * W / (sm + 1) > 512) continue;
-                cand.push_back(gchi_pr_tune{W, sm, pers, 0});
-            }
+        for (int sm : {8, 16, 32, 64}) {
+            if (2 * W / (sm + 1) > 512) continue;
+            cand.push_back(gchi_pr_tune{W, sm, 0, 0});
+        }
     const bool layout_ok = g->nvertices < (1u << 30) && g->nedges > 0;
     for (int sm : {8, 16, 32, 64})
         for (int hot : {0, -1, 16384, 1 << 20}) {

@@ -28,8 +28,7 @@
 // Many graphs (a disjoint union with vertex bases) share one plan: blocks are
 // aligned to graph boundaries, so every block and hub belongs to one graph,
 // the apply can use a per-graph constant and FP64 statistics are per graph.
-// Tiles (hub chunks first, then regular blocks) are either one workgroup each
-// or pulled by persistent workgroups from a device work counter.
+// Tiles (hub chunks first, then regular blocks) are one workgroup each.
 // Gather layout (optional): sources are ranked by out-degree, descending, and
 // the plan's edges store that rank; each sweep first copies x into rank order
 // (xg), so the most referenced values share cache lines, and persistent
@@ -54,7 +53,7 @@ struct gchi_pr_plan {
     uint32_t nhub = 0;     // hub rows
     uint32_t nchunk = 0;   // hub chunks
     uint32_t nfin = 0;     // finalize workgroups (single-graph plans)
-    uint32_t npersist = 0; // workgroups of the persistent sweep
+    uint32_t npersist = 0; // workgroups of form 1 resident at once
     uint64_t e_reg = 0, e_hub = 0;
     const uint32_t *outdeg = nullptr;
     uint32_t *reg_off = nullptr;
@@ -79,7 +78,7 @@ struct gchi_pr_plan {
     double *blk_stat = nullptr;
     double *hub_stat = nullptr;
     double *fin_stat = nullptr;
-    uint32_t *counters = nullptr;  // [0] finalize ticket, [kPrStripeGap...] tile counter stripes
+    uint32_t *counters = nullptr;  // finalize ticket
     int hot = 0;           // tune value (0: vertex ids, -1: gather layout, > 0: layout + LDS cache)
     uint32_t A = 0;        // sources in the gather layout (out-degree > 0)
     uint32_t H = 0;        // layout values cached in LDS by the wavefront-tiled kernel
@@ -113,14 +112,6 @@ struct PrConsts {
     double seed_tele;
 };
 
-constexpr uint32_t kPrStripes = 16;    // tile counters of the persistent sweep
-constexpr uint32_t kPrStripeGap = 32;  // uint32 words between counters (128 bytes)
-constexpr uint32_t kPrCounterWords = kPrStripeGap * (kPrStripes + 1);
-
-GCHI_DEV void pr_reset_stripes(uint32_t *counters) {
-    for (uint32_t i = threadIdx.x; i < kPrStripes; i += blockDim.x) counters[kPrStripeGap * (i + 1)] = 0u;
-}
-
 struct PrArgs {
     const uint32_t *reg_off, *reg_src, *blk_row, *blk_graph, *tile_e0, *tile_e1, *hub_bits;
     const uint64_t *ebase, *chunk_beg;
@@ -129,7 +120,6 @@ struct PrArgs {
     const float *r_in;
     float *x_out, *r_out, *chunk_part;
     double *blk_stat;
-    uint32_t *tile_counter;
     uint32_t nchunk, nhubt, nblk, ntiles;  // hub chunks, hub tiles (NW chunks each), regular blocks, all tiles
     int short_max;
 };
@@ -223,20 +213,36 @@ GCHI_DEV void pr_tile(const PrArgs &a, const PrConsts &c, uint32_t tile, float *
     }
 
     // ---- regular block ----
+    // A tile is a chain of dependent loads (descriptor, edge ids, gathers, rows),
+    // so everything that can be is loaded together: the thread's first row beside
+    // the edge ids, and the rows that a wavefront sums are finished by the threads
+    // that found them, side by side (one lane after another, each waiting for its
+    // row's r and out-degree, they were most of a tile's time).
     const uint32_t b = tile - a.nhubt;
     const uint32_t rb = a.blk_row[b], re = a.blk_row[b + 1];
     const uint32_t g = a.blk_graph[b];
-    const uint32_t *ro = a.reg_off + g;  // the graph's offset slots: row v at ro[v]
     const uint32_t e0 = a.tile_e0[b], e1 = a.tile_e1[b];
+    const uint32_t *ro = a.reg_off + g;  // the graph's offset slots: row v at ro[v]
     const uint32_t span = e1 - e0;
     const uint32_t *rs = a.reg_src + a.ebase[g] + e0;
+    const double tele = c.g_tele ? c.g_tele[g] : c.teleport;
     if (tid == 0) *s_nlong = 0;
-    for (uint32_t base = 0; base < span; base += 8 * T) {
+    const uint32_t v0 = rb + tid, v0c = re > rb ? min(v0, re - 1) : 0u;
+    uint32_t beg = 0, end = 0, hubw = 0, od = 0;
+    float rold = 0.0f;
+    for (uint32_t base = 0; base < span || base == 0; base += 8 * T) {
         uint32_t idx[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             uint32_t k = base + (uint32_t)j * T + tid;
             idx[j] = k < span ? __builtin_nontemporal_load(&rs[k]) : 0u;
+        }
+        if (base == 0) {
+            beg = ro[v0c];
+            end = ro[v0c + 1];
+            hubw = a.hub_bits[v0c >> 5];
+            rold = a.r_in[v0c];
+            od = a.outdeg[v0c];
         }
         float val[8];
 #pragma unroll
@@ -254,27 +260,53 @@ GCHI_DEV void pr_tile(const PrArgs &a, const PrConsts &c, uint32_t tile, float *
     __syncthreads();
 
     double res = 0.0, sum = 0.0;
-    for (uint32_t v = rb + tid; v < re; v += T) {
-        if ((a.hub_bits[v >> 5] >> (v & 31)) & 1u) continue;
-        uint32_t beg = ro[v] - e0, end = ro[v + 1] - e0;
-        if ((int)(end - beg) <= a.short_max) {
+    auto finish = [&](uint32_t v, float s, float r0, uint32_t deg) {
+        double t = tele;
+        if (c.seed_bits && ((c.seed_bits[v >> 5] >> (v & 31)) & 1u)) t += c.seed_tele;
+        const float r = pr_apply(t, c.damping, s);
+        a.r_out[v] = r;
+        a.x_out[v] = pr_scatter(r, deg);
+        res += fabs((double)r - (double)r0);
+        sum += (double)r;
+    };
+    // short rows: one lane, in src order; long rows go to the list (begin and
+    // end in the staged values, both below 2^16)
+    auto first_pass = [&](uint32_t v, uint32_t vb, uint32_t ve, float r0, uint32_t deg) {
+        if ((int)(ve - vb) <= a.short_max) {
             float s = 0.0f;
-            for (uint32_t k = beg; k < end; k++) s += s_val[k];
-            pr_finish_row(v, g, s, c, a.r_in, a.outdeg, a.r_out, a.x_out, res, sum);
-        } else {
-            uint32_t slot = atomicAdd(s_nlong, 1u);
-            s_long[slot] = v;
+            for (uint32_t k = vb; k < ve; k++) s += s_val[k];
+            finish(v, s, r0, deg);
+            return false;
         }
+        s_long[atomicAdd(s_nlong, 1u)] = vb | (ve << 16);
+        return true;
+    };
+    bool long0 = false;
+    uint32_t more = 0;  // long rows among the thread's later ones
+    if (v0 < re && !((hubw >> (v0 & 31)) & 1u)) long0 = first_pass(v0, beg - e0, end - e0, rold, od);
+    for (uint32_t v = v0 + T; v < re; v += T) {
+        if ((a.hub_bits[v >> 5] >> (v & 31)) & 1u) continue;
+        more += first_pass(v, ro[v] - e0, ro[v + 1] - e0, a.r_in[v], a.outdeg[v]);
     }
     __syncthreads();
     const uint32_t nlong = *s_nlong;
-    for (uint32_t li = wave; li < nlong; li += NW) {
-        uint32_t v = s_long[li];
-        uint32_t beg = ro[v] - e0, end = ro[v + 1] - e0;
-        float s = 0.0f;
-        for (uint32_t k = beg + lane; k < end; k += kWave) s += s_val[k];
-        s = wave_sum(s);
-        if (lane == 0) pr_finish_row(v, g, s, c, a.r_in, a.outdeg, a.r_out, a.x_out, res, sum);
+    if (nlong) {  // workgroup-uniform
+        for (uint32_t li = wave; li < nlong; li += NW) {
+            const uint32_t vb = s_long[li] & 0xffffu, ve = s_long[li] >> 16;
+            float s = 0.0f;
+            for (uint32_t k = vb + lane; k < ve; k += kWave) s += s_val[k];
+            s = wave_sum(s);
+            if (lane == 0) s_val[vb] = s;  // the row's first value is its sum now
+        }
+        __syncthreads();
+        if (long0) finish(v0, s_val[beg - e0], rold, od);
+        for (uint32_t v = v0 + T; more; v += T) {
+            if ((a.hub_bits[v >> 5] >> (v & 31)) & 1u) continue;
+            const uint32_t vb = ro[v] - e0;
+            if ((int)(ro[v + 1] - e0 - vb) <= a.short_max) continue;
+            finish(v, s_val[vb], a.r_in[v], a.outdeg[v]);
+            more--;
+        }
     }
     res = wave_sum(res);
     sum = wave_sum(sum);
@@ -294,43 +326,20 @@ GCHI_DEV void pr_tile(const PrArgs &a, const PrConsts &c, uint32_t tile, float *
     }
 }
 
-__global__ __launch_bounds__(kPrThreads) void pr_sweep_kernel(PrArgs a, PrConsts c) {
+// One workgroup per tile (hub chunks first, then regular blocks); the hardware
+// hands them out as earlier ones end.  Resident workgroups that pulled tiles from device counters instead took 668 us a sweep
+// where this launch takes 535 (300 R-MAT graphs of scales 10-17, 153M edges; 699
+// with a static tile list): the ticket and its two barriers stand in front of
+// every tile's chain of loads.
+// (The same kernel with a loop over tiles: 660 us.)
+constexpr uint32_t kPrMaxGrid = 1u << 23;  // grid x threads stays below 2^32: more tiles take several launches
+
+__global__ __launch_bounds__(kPrThreads) void pr_sweep_kernel(PrArgs a, PrConsts c, uint32_t first) {
     extern __shared__ float s_val[];  // 2W floats
     __shared__ uint32_t s_long[kMaxLong];
     __shared__ uint32_t s_nlong;
     __shared__ double s_red[2 * kPrWaves];
-    pr_tile<kPrThreads>(a, c, blockIdx.x, s_val, s_long, &s_nlong, s_red);
-}
-
-// Persistent form: workgroups pull tiles from the work counters until the queue
-// is drained (hub chunks first, then regular blocks).  Atomics on one address
-// complete one after another (about 10 ns each here), so one counter would cap
-// a sweep at ~10^8 tiles per second; kPrStripes counters, each in its own
-// 128-byte line, hand out the tiles s, s + kPrStripes, ... of stripe s.  A
-// workgroup starts on stripe blockIdx % kPrStripes and moves to the next one
-// when it is drained, so the tiles in flight stay a narrow window of the tile
-// order (the sources the gathers touch stay in cache).  Every workgroup exits
-// once all stripes are drained; the finalize kernels reset the counters.
-__global__ __launch_bounds__(kPrThreads) void pr_sweep_persistent_kernel(PrArgs a, PrConsts c) {
-    extern __shared__ float s_val[];
-    __shared__ uint32_t s_long[kMaxLong];
-    __shared__ uint32_t s_nlong;
-    __shared__ double s_red[2 * kPrWaves];
-    __shared__ uint32_t s_tile;
-    uint32_t stripe = blockIdx.x % kPrStripes, spent = 0;
-    for (;;) {
-        if (threadIdx.x == 0) s_tile = atomicAdd(&a.tile_counter[stripe * kPrStripeGap], 1u);
-        __syncthreads();
-        const uint64_t tile = stripe + (uint64_t)kPrStripes * s_tile;
-        __syncthreads();  // s_tile is rewritten by the next ticket
-        if (tile >= a.ntiles) {  // block-uniform
-            if (++spent == kPrStripes) break;
-            stripe = (stripe + 1) % kPrStripes;
-            continue;
-        }
-        pr_tile<kPrThreads>(a, c, (uint32_t)tile, s_val, s_long, &s_nlong, s_red);
-        __syncthreads();
-    }
+    pr_tile<kPrThreads>(a, c, first + blockIdx.x, s_val, s_long, &s_nlong, s_red);
 }
 
 // Copies layout positions [0, H) of xg into the LDS cache, kFillAhead loads per
@@ -915,7 +924,6 @@ __global__ __launch_bounds__(kFinThreads) void pr_finalize_kernel(
             d_stats[1] = ts;
             counters[0] = 0u;
         }
-        pr_reset_stripes(counters);
     }
 }
 
@@ -949,8 +957,7 @@ __global__ __launch_bounds__(kFinThreads) void pr_graph_reduce_kernel(const uint
                                                                       const uint32_t *__restrict__ ghub,
                                                                       const double *__restrict__ blk_stat,
                                                                       const double *__restrict__ hub_stat,
-                                                                      uint32_t G, uint32_t *counters,
-                                                                      double *d_stats) {
+                                                                      uint32_t G, double *d_stats) {
     __shared__ double s_red[2 * (kFinThreads / kWave)];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     for (uint32_t g = blockIdx.x; g < G; g += gridDim.x) {
@@ -981,7 +988,6 @@ __global__ __launch_bounds__(kFinThreads) void pr_graph_reduce_kernel(const uint
         }
         __syncthreads();
     }
-    if (blockIdx.x == 0) pr_reset_stripes(counters);
 }
 
 __global__ void pr_init_kernel(const uint32_t *outdeg, uint32_t n, float init, const uint32_t *seed_bits,
@@ -1422,7 +1428,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     zz.take<double>(2 * (size_t)p->nblk);
     zz.take<double>(2 * (size_t)nhub + 2);
     zz.take<double>(2 * (size_t)p->nfin);
-    zz.take<uint32_t>(kPrCounterWords);
+    zz.take<uint32_t>(1);
     zz.take<uint32_t>(std::max<uint32_t>(A, 1));
     zz.take<float>(std::max<uint32_t>(A, 1));
     zz.take<uint32_t>(p->nblk + 1);
@@ -1448,7 +1454,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     p->blk_stat = c.take<double>(2 * (size_t)p->nblk);
     p->hub_stat = c.take<double>(2 * (size_t)nhub + 2);
     p->fin_stat = c.take<double>(2 * (size_t)p->nfin);
-    p->counters = c.take<uint32_t>(kPrCounterWords);
+    p->counters = c.take<uint32_t>(1);
     p->gorder = c.take<uint32_t>(std::max<uint32_t>(A, 1));
     p->xg = c.take<float>(std::max<uint32_t>(A, 1));
     p->tile_e0 = c.take<uint32_t>(p->nblk + 1);
@@ -1462,7 +1468,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     GCHI_HIP(hipMemcpyAsync(p->hub_chunk_off, hub_choff, (size_t)(nhub + 1) * 4, hipMemcpyDeviceToDevice, s));
     GCHI_HIP(hipMemcpyAsync(p->gblk, gblk, (size_t)(G + 1) * 4, hipMemcpyDeviceToDevice, s));
     GCHI_HIP(hipMemcpyAsync(p->vbase, vbase, (size_t)(G + 1) * 4, hipMemcpyDeviceToDevice, s));
-    launch_fill_u32(p->counters, 0u, kPrCounterWords, s);
+    launch_fill_u32(p->counters, 0u, 1, s);
     if (E)
         hipLaunchKernelGGL(plan_copy, dim3(grid_for((uint64_t)N * kWave, 256, 1u << 16)), dim3(256), 0, s, cv,
                            hub_flag, p->reg_off, p->ebase, grank, p->reg_src, bad);
@@ -1627,7 +1633,7 @@ int pr_sweep(const gchi_pr_plan *p, const gchi_pr_op *op, const float *x_in, con
     const uint32_t nhubt = (p->nchunk + kPrWaves - 1) / kPrWaves;
     PrArgs a{p->reg_off, p->reg_src, p->blk_row, p->blk_graph, p->tile_e0, p->tile_e1, p->hub_bits, p->ebase,
              p->chunk_beg, p->chunk_len, p->hub_src,
-             p->outdeg, xg, r_in, x_out, r_out, p->chunk_part, p->blk_stat, p->counters + kPrStripeGap,
+             p->outdeg, xg, r_in, x_out, r_out, p->chunk_part, p->blk_stat,
              p->nchunk, nhubt, p->nblk, nhubt + p->nblk, p->short_max};
     const size_t shmem = (size_t)2 * p->W * sizeof(float);
     if (p->persistent == 3) {
@@ -1638,10 +1644,10 @@ int pr_sweep(const gchi_pr_plan *p, const gchi_pr_op *op, const float *x_in, con
             hipLaunchKernelGGL((pr_sweep_wave_kernel<kWaveThreads, 8, true>), grid, blk, p->wave_lds, s, a, c, p->H);
         else
             hipLaunchKernelGGL((pr_sweep_wave_kernel<kWaveThreads, 8, false>), grid, blk, p->wave_lds, s, a, c, 0u);
-    } else if (p->persistent == 1) {
-        hipLaunchKernelGGL(pr_sweep_persistent_kernel, dim3(p->npersist), dim3(kPrThreads), shmem, s, a, c);
     } else {
-        hipLaunchKernelGGL(pr_sweep_kernel, dim3(nhubt + p->nblk), dim3(kPrThreads), shmem, s, a, c);
+        for (uint32_t t = 0; t < a.ntiles; t += std::min(kPrMaxGrid, a.ntiles - t))
+            hipLaunchKernelGGL(pr_sweep_kernel, dim3(std::min(kPrMaxGrid, a.ntiles - t)), dim3(kPrThreads), shmem, s, a,
+                               c, t);
     }
     if (p->G == 1) {
         hipLaunchKernelGGL(pr_finalize_kernel, dim3(p->nfin), dim3(kFinThreads), 0, s, p->hub_v, p->hub_chunk_off,
@@ -1653,7 +1659,7 @@ int pr_sweep(const gchi_pr_plan *p, const gchi_pr_op *op, const float *x_in, con
                                dim3(kFinThreads), 0, s, p->hub_v, p->hub_graph, p->hub_chunk_off, p->chunk_part,
                                p->outdeg, r_in, r_out, x_out, p->nhub, p->hub_stat, c);
         hipLaunchKernelGGL(pr_graph_reduce_kernel, dim3(std::min<uint32_t>(p->G, 4096)), dim3(kFinThreads), 0, s,
-                           p->gblk, p->ghub, p->blk_stat, p->hub_stat, p->G, p->counters, d_stats);
+                           p->gblk, p->ghub, p->blk_stat, p->hub_stat, p->G, d_stats);
     }
     GCHI_LAUNCH_CHECK();
     return GCHI_OK;

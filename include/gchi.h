@@ -201,8 +201,7 @@ typedef struct gchi_pr_tune {
     int edges_per_block;   /* W: multiple of 256 in [256,4096]; 0 = 2048.  Rows with
                               in-degree >= W are hub rows, cut into 512-edge chunks */
     int short_row_max;     /* rows up to this length use one lane per row; 0 = 32 */
-    int persistent;        /* 0: one workgroup per tile; 1: persistent workgroups pull
-                              tiles from a device work counter; 2: one 1024-thread
+    int persistent;        /* 0 or 1: one workgroup per tile; 2: one 1024-thread
                               workgroup per CU whose wavefronts each work through a
                               fixed list of tiles, software-pipelined (W = 256),
                               optionally with the LDS cache of hot_vertices; 3: four
@@ -332,7 +331,7 @@ int gchi_pr_blocked_sweep(const gchi_pr_blocked *b, const gchi_pr_op *op, float 
                           float *d_r_out, double *d_stats, void *stream);
 
 /* Autotuner: times every candidate launch shape (edges_per_block in
- * {512..4096}, short_row_max in {8..64}, persistent 0/1, the
+ * {512..4096}, short_row_max in {8..64}, the
  * wavefront-tiled sweep, W = 256, with hot_vertices in {0, -1, 16384, max},
  * and the cached persistent workgroups, W in {1024, 2048}) on the caller's
  * graph with HIP events (sweeps_per_candidate sweeps after a warm-up) and
@@ -344,10 +343,9 @@ int gchi_autotune_pr(const gchi_dgraph *g, int sweeps_per_candidate, gchi_pr_tun
 /* ------------------------------------------------- batched personalized PageRank */
 /* Many personalized-PageRank queries (restart sets of 1..64 seeds; kernel
  * r_v = (v in S ? (1-d)/|S| : 0) + d * sum r_u/outdeg_u, from r = restart vector)
- * swept together: 64 queries per block, ranks stored vertex-major (64 per
- * vertex), one wavefront per destination row with one lane per query, tiles
- * (query block, row block / hub chunk) pulled from a device work queue by a
- * persistent kernel.  Phase 1 stores ranks in BF16 (FP32 accumulation) for up to
+ * swept together: 64 queries per block (a last block of at most 32 has rows of
+ * 4, 8, 16 or 32), ranks stored row-major (64 per vertex), one lane per query;
+ * the in-edges are one stream cut into equal items, one wavefront each.  Phase 1 stores ranks in BF16 (FP32 accumulation) for up to
  * bf16_sweeps sweeps or until every query's L1 residual <= bf16_switch_residual
  * or stops falling; phase 2 refines in FP32 until every query satisfies
  * residual * d/(1-d) <= tol (a bound on the L1 distance to the fixed point,
