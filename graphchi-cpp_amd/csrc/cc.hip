@@ -344,58 +344,104 @@ __global__ void cc_iota(uint32_t *l, uint32_t n) {
 }
 
 // ---- selective scheduling ----
-constexpr uint32_t kCcsShort = 64;    // rows up to this length: one lane each
+// A round evaluates its long rows first: they hold the hubs, whose labels drop
+// the furthest, and the short rows then see those labels in the same round
+// (R-MAT scale 22, 67M entries: 6 rounds -> 5).  A row whose label is 0, or that
+// meets a 0, needs no further look at its neighbours: nothing is lower (vertex
+// 0's component; rows of others are read whole).  Round 0 still checks every
+// neighbour id.  Together with kCcsLanes lanes per short row, 16 flags per thread
+// in the compaction and the lists' own flags (no clearing passes) and two rounds per readback: 3317 -> 1421 us.
+constexpr uint32_t kCcsShort = 64;    // rows up to this length: kCcsLanes lanes each
 constexpr uint32_t kCcsChunk = 4096;  // longer rows: one wavefront per chunk
+constexpr int kCcsLanes = 4;  // 4 / 8 / 16: 445 / 488 / 579 us of short rows per call
+constexpr int kCcsThreads = 1024;     // compaction workgroup
+constexpr uint32_t kCcsPer = 16;      // vertices per thread of it
 
-// ctr: [0] short rows, [1] long-row chunks.  stat: [0] labels dropped,
-// [1] rows evaluated, [2] neighbour ids >= n seen.  Each wavefront compacts a
-// contiguous vertex range in two passes (count, reserve once, write), so the
-// shared counters see one atomic per wavefront and round, not one per 64
-// vertices: atomics on one address complete one after another.
-__global__ void ccs_compact(const uint32_t *off, uint32_t n, const uint8_t *cur, uint32_t *short_list,
-                            uint64_t *items, uint32_t *ctr, unsigned long long *stat) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint64_t wid = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / kWave;
-    const uint64_t per = ((n + nw - 1) / nw + kWave - 1) / kWave * kWave;
-    const uint64_t lo = wid * per, hi = lo + per < n ? lo + per : n;
+// The round's scheduled vertices (flags cur, cleared here: the array takes the
+// marks of the round after next) as lists: short rows, and the chunks of long
+// rows with their "label dropped" words cleared.  ctr: [0] short rows, [1]
+// long-row chunks.  stat: [0] labels dropped, [1] rows evaluated, [2] neighbour
+// ids >= n seen.  One atomic per counter and workgroup of 16384 vertices: atomics
+// on one address complete one after another.
+__global__ __launch_bounds__(kCcsThreads) void ccs_compact(const uint32_t *__restrict__ off, uint32_t n, uint8_t *cur,
+                                                           uint32_t *short_list, uint64_t *items, uint32_t *dropped,
+                                                           uint32_t *ctr, unsigned long long *stat) {
+    __shared__ uint32_t s_ns[kCcsThreads / kWave], s_ni[kCcsThreads / kWave], s_na[kCcsThreads / kWave];
+    __shared__ uint32_t s_base[2];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const uint64_t v0 = ((uint64_t)blockIdx.x * kCcsThreads + threadIdx.x) * kCcsPer;
+    uint32_t f[4] = {0, 0, 0, 0};  // cur is padded to whole groups of kCcsPer
+    if (v0 < n) {
+        uint4 *p = reinterpret_cast<uint4 *>(cur + v0);
+        const uint4 w = *p;
+        f[0] = w.x;
+        f[1] = w.y;
+        f[2] = w.z;
+        f[3] = w.w;
+        if (f[0] | f[1] | f[2] | f[3]) *p = make_uint4(0, 0, 0, 0);
+    }
+    uint32_t deg[kCcsPer];
     uint32_t ns = 0, ni = 0, na = 0;
-    for (uint64_t v = lo + lane; v < hi; v += kWave) {
-        if (!cur[v]) continue;
-        const uint32_t deg = off[v + 1] - off[v];
-        na++;
-        if (deg <= kCcsShort) ns++;
-        else ni += (deg + kCcsChunk - 1) / kCcsChunk;
-    }
-    ns = wave_sum(ns);
-    ni = wave_sum(ni);
-    na = wave_sum(na);
-    uint32_t sbase = 0, ibase = 0;
-    if (lane == 0) {
-        if (ns) sbase = atomicAdd(&ctr[0], ns);
-        if (ni) ibase = atomicAdd(&ctr[1], ni);
-        if (na) atomicAdd(&stat[1], (unsigned long long)na);
-    }
-    sbase = __shfl(sbase, 0, kWave);
-    ibase = __shfl(ibase, 0, kWave);
-    if (ns == 0 && ni == 0) return;
-    for (uint64_t base = lo; base < hi; base += kWave) {  // whole wavefronts: ballots and shuffles
-        const uint64_t v = base + lane;
-        const bool act = v < hi && cur[v];
-        const uint32_t deg = act ? off[v + 1] - off[v] : 0u;
-        const bool sh = act && deg <= kCcsShort;
-        const uint32_t nit = (act && deg > kCcsShort) ? (deg + kCcsChunk - 1) / kCcsChunk : 0u;
-        const uint64_t bs = __ballot(sh);
-        if (sh) short_list[sbase + __popcll(bs & lanemask_lt())] = (uint32_t)v;
-        sbase += (uint32_t)__popcll(bs);
-        uint32_t incl = nit;
+    if (f[0] | f[1] | f[2] | f[3]) {
+        uint32_t o[kCcsPer + 1];
 #pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const uint32_t t = __shfl_up(incl, o, kWave);
-            if (lane >= o) incl += t;
+        for (uint32_t k = 0; k <= kCcsPer; k++) o[k] = off[v0 + k <= n ? v0 + k : n];
+#pragma unroll
+        for (uint32_t k = 0; k < kCcsPer; k++) {
+            const bool on = ((f[k / 4] >> (8 * (k % 4))) & 0xffu) && v0 + k < n;
+            deg[k] = on ? o[k + 1] - o[k] : 0xffffffffu;
+            if (!on) continue;
+            na++;
+            if (deg[k] <= kCcsShort) ns++;
+            else ni += (deg[k] + kCcsChunk - 1) / kCcsChunk;
         }
-        for (uint32_t c = 0; c < nit; c++) items[ibase + incl - nit + c] = (v << 32) | c;
-        ibase += __shfl(incl, kWave - 1, kWave);
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < kCcsPer; k++) deg[k] = 0xffffffffu;
+    }
+    uint32_t ps = ns, pi = ni;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t a = __shfl_up(ps, o, kWave), b = __shfl_up(pi, o, kWave);
+        if (lane >= o) {
+            ps += a;
+            pi += b;
+        }
+    }
+    const uint32_t wa = wave_sum(na);
+    if (lane == kWave - 1) {
+        s_ns[wave] = ps;
+        s_ni[wave] = pi;
+        s_na[wave] = wa;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t ts = 0, ti = 0, ta = 0;
+        for (int w = 0; w < kCcsThreads / kWave; w++) {
+            const uint32_t x = s_ns[w], y = s_ni[w];
+            s_ns[w] = ts;
+            s_ni[w] = ti;
+            ts += x;
+            ti += y;
+            ta += s_na[w];
+        }
+        s_base[0] = ts ? atomicAdd(&ctr[0], ts) : 0u;
+        s_base[1] = ti ? atomicAdd(&ctr[1], ti) : 0u;
+        if (ta) atomicAdd(&stat[1], (unsigned long long)ta);
+    }
+    __syncthreads();
+    uint32_t as = s_base[0] + s_ns[wave] + ps - ns, ai = s_base[1] + s_ni[wave] + pi - ni;
+#pragma unroll
+    for (uint32_t k = 0; k < kCcsPer; k++) {
+        if (deg[k] == 0xffffffffu) continue;
+        if (deg[k] <= kCcsShort) {
+            short_list[as++] = (uint32_t)(v0 + k);
+        } else {
+            for (uint32_t c = 0; c * kCcsChunk < deg[k]; c++) {
+                items[ai] = ((v0 + k) << 32) | c;
+                dropped[ai++] = 0u;
+            }
+        }
     }
 }
 
@@ -410,26 +456,35 @@ __global__ void ccs_check_off(const uint32_t *off, uint32_t n, unsigned long lon
     if ((threadIdx.x & (kWave - 1)) == 0 && bad) atomicAdd(&stat[2], (unsigned long long)bad);
 }
 
-// One lane per short row: label = min over the row, neighbours scheduled if it dropped.
-__global__ void ccs_short(const uint32_t *off, const uint32_t *adj, uint32_t n, uint32_t *label,
-                          const uint32_t *short_list, const uint32_t *ctr, uint8_t *next, unsigned long long *stat) {
-    const uint32_t cnt = ctr[0];
+// kCcsLanes lanes per short row: label = min over the row, neighbours scheduled
+// if it dropped.  (One lane per row kept 64 rows of 1 to 64 entries in step, each
+// at its own cache lines.)
+__global__ void ccs_short(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, uint32_t n,
+                          uint32_t *label, const uint32_t *__restrict__ short_list, const uint32_t *__restrict__ ctr,
+                          uint8_t *next, int first, unsigned long long *stat) {
+    const uint32_t cnt = ctr[0], sub = threadIdx.x % kCcsLanes;
     uint32_t dropped = 0, bad = 0;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += stride) {
+    const uint32_t stride = gridDim.x * blockDim.x / kCcsLanes;
+    for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / kCcsLanes; i < cnt; i += stride) {
         const uint32_t v = short_list[i], b = off[v], e = off[v + 1];
         const uint32_t lv = label[v];
         uint32_t m = lv;
-#pragma unroll 4
-        for (uint32_t k = b; k < e; k++) {
-            const uint32_t u = adj[k];
-            if (u < n) m = min(m, label[u]);
-            else bad = 1;
+        for (uint32_t k = b + sub; k < e && (first || m != 0); k += 2 * kCcsLanes) {
+            const bool two = k + kCcsLanes < e;
+            const uint32_t u0 = adj[k], u1 = two ? adj[k + kCcsLanes] : u0;
+            bad |= u0 >= n || u1 >= n;
+            if (m == 0) continue;
+            const uint32_t l0 = label[u0 < n ? u0 : v], l1 = label[u1 < n ? u1 : v];
+            m = min(m, min(l0, l1));
         }
+#pragma unroll
+        for (int o = kCcsLanes / 2; o > 0; o >>= 1) m = min(m, (uint32_t)__shfl_xor((int)m, o, kWave));
         if (m < lv) {
-            label[v] = m;  // the only writer of a short row's label
-            dropped++;
-            for (uint32_t k = b; k < e; k++) {
+            if (sub == 0) {
+                label[v] = m;  // the only writer of a short row's label
+                dropped++;
+            }
+            for (uint32_t k = b + sub; k < e; k += kCcsLanes) {
                 const uint32_t u = adj[k];
                 if (u < n) next[u] = 1;
             }
@@ -443,10 +498,11 @@ __global__ void ccs_short(const uint32_t *off, const uint32_t *adj, uint32_t n, 
     }
 }
 
-// One wavefront per chunk of a long row: min over the chunk, atomicMin into the row.
-__global__ void ccs_long_min(const uint32_t *off, const uint32_t *adj, uint32_t n, uint32_t *label,
-                             const uint64_t *items, const uint32_t *ctr, uint8_t *dropped_flag,
-                             unsigned long long *stat) {
+// One wavefront per chunk of a long row: min over the chunk, atomicMin into the
+// row; dropped[first chunk of the row] = 1 when the label fell.
+__global__ void ccs_long_min(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, uint32_t n,
+                             uint32_t *label, const uint64_t *__restrict__ items, const uint32_t *__restrict__ ctr,
+                             uint32_t *dropped, int first, unsigned long long *stat) {
     const int lane = threadIdx.x & (kWave - 1);
     const uint32_t cnt = ctr[1];
     const uint32_t wid = (blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (gridDim.x * blockDim.x) / kWave;
@@ -457,21 +513,24 @@ __global__ void ccs_long_min(const uint32_t *off, const uint32_t *adj, uint32_t 
         const uint32_t b = off[v] + c * kCcsChunk, e = min(off[v + 1], b + kCcsChunk);
         const uint32_t lv = label[v];
         uint32_t m = 0xffffffffu;
-        for (uint32_t k0 = b + lane; k0 < e; k0 += 4 * kWave) {  // four gathers in flight per lane
-            uint32_t u[4];
+        bool low = lv == 0;  // wavefront-uniform: the label is or becomes 0, the lowest there is
+        for (uint32_t k0 = b + lane; k0 - lane < e && (first || !low); k0 += 4 * kWave) {  // four gathers in flight per lane
+            uint32_t u[4], l[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) u[q] = k0 + q * kWave < e ? adj[k0 + q * kWave] : 0xffffffffu;
+            for (int q = 0; q < 4; q++) u[q] = adj[min(k0 + q * kWave, e - 1)];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                if (u[q] < n) m = min(m, label[u[q]]);
-                else if (k0 + q * kWave < e) bad = 1;
-            }
+            for (int q = 0; q < 4; q++) bad |= u[q] >= n;
+            if (low) continue;  // round 0 looks at every id
+#pragma unroll
+            for (int q = 0; q < 4; q++) l[q] = label[u[q] < n ? u[q] : v];
+            m = min(min(m, min(l[0], l[1])), min(l[2], l[3]));
+            low = __ballot(m == 0) != 0;
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) m = min(m, (uint32_t)__shfl_xor(m, o, kWave));
         if (lane == 0 && m < lv) {
             const uint32_t old = atomicMin(&label[v], m);
-            if (m < old) dropped_flag[v] = 1;
+            if (m < old) dropped[j - c] = 1u;  // a row's chunks are consecutive items
         }
     }
     bad = wave_sum(bad);
@@ -479,9 +538,9 @@ __global__ void ccs_long_min(const uint32_t *off, const uint32_t *adj, uint32_t 
 }
 
 // Schedules the neighbours of every long row whose label dropped (per chunk).
-__global__ void ccs_long_mark(const uint32_t *off, const uint32_t *adj, uint32_t n, const uint64_t *items,
-                              const uint32_t *ctr, const uint8_t *dropped_flag, uint8_t *next,
-                              unsigned long long *stat) {
+__global__ void ccs_long_mark(const uint32_t *__restrict__ off, const uint32_t *__restrict__ adj, uint32_t n,
+                              const uint64_t *__restrict__ items, const uint32_t *__restrict__ ctr,
+                              const uint32_t *__restrict__ dropped_at, uint8_t *next, unsigned long long *stat) {
     const int lane = threadIdx.x & (kWave - 1);
     const uint32_t cnt = ctr[1];
     const uint32_t wid = (blockIdx.x * blockDim.x + threadIdx.x) / kWave, nw = (gridDim.x * blockDim.x) / kWave;
@@ -489,7 +548,7 @@ __global__ void ccs_long_mark(const uint32_t *off, const uint32_t *adj, uint32_t
     for (uint32_t j = wid; j < cnt; j += nw) {
         const uint64_t it = items[j];
         const uint32_t v = (uint32_t)(it >> 32), c = (uint32_t)it;
-        if (!dropped_flag[v]) continue;
+        if (!dropped_at[j - c]) continue;
         if (c == 0) dropped++;
         const uint32_t b = off[v] + c * kCcsChunk, e = min(off[v + 1], b + kCcsChunk);
         for (uint32_t k0 = b + lane; k0 < e; k0 += 4 * kWave) {
@@ -506,24 +565,22 @@ __global__ void ccs_long_mark(const uint32_t *off, const uint32_t *adj, uint32_t
 
 struct CcsWork {
     uint8_t *flags[2];
-    uint8_t *dropped;
     uint32_t *short_list;
     uint64_t *items;
-    uint32_t *ctr;
-    unsigned long long *stat;
+    uint32_t *dropped;  // per item
+    unsigned long long *stat;  // two rounds of [3] and the two list counters
 };
 
 template <typename C>
 static void ccs_layout(C &c, uint32_t n, uint64_t e, CcsWork *w) {
-    const size_t nb = align_up((size_t)n + 1, 4);
+    const size_t nb = align_up((size_t)n + 1, kCcsPer), ni = (size_t)n + e / kCcsChunk + 1;
     auto *f0 = c.template take<uint8_t>(nb);
     auto *f1 = c.template take<uint8_t>(nb);
-    auto *dr = c.template take<uint8_t>(nb);
     auto *sl = c.template take<uint32_t>((size_t)n + 1);
-    auto *it = c.template take<uint64_t>((size_t)n + e / kCcsChunk + 1);
-    auto *ct = c.template take<uint32_t>(2);
-    auto *st = c.template take<unsigned long long>(3);
-    if (w) *w = CcsWork{{f0, f1}, dr, sl, it, ct, st};
+    auto *it = c.template take<uint64_t>(ni);
+    auto *dr = c.template take<uint32_t>(ni);
+    auto *st = c.template take<unsigned long long>(8);
+    if (w) *w = CcsWork{{f0, f1}, sl, it, dr, st};
 }
 
 }  // namespace gchi
@@ -687,7 +744,7 @@ extern "C" int gchi_cc_scheduled_ex(const uint32_t *d_off, const uint32_t *d_adj
     CcsWork w;
     ccs_layout(c, nvertices, E, &w);
     const uint32_t n = nvertices;
-    const size_t nwords = align_up((size_t)n + 1, 4) / 4;
+    const size_t nwords = align_up((size_t)n + 1, kCcsPer) / 4;
     const unsigned gv = grid_for(n, 256, 65536);
     const unsigned gl = grid_for(n, 256, 2048);  // list kernels loop over their lists
     const unsigned gw = 4096;  // wavefronts loop over the chunk list
@@ -699,40 +756,44 @@ extern "C" int gchi_cc_scheduled_ex(const uint32_t *d_off, const uint32_t *d_adj
     GCHI_CHECK(h_bad == 0, GCHI_ERR_INVALID, "cc_scheduled: offsets are not a CSR");
     hipLaunchKernelGGL(cc_iota, dim3(gv), dim3(256), 0, s, d_labels, n);
     launch_fill_u32(reinterpret_cast<uint32_t *>(w.flags[0]), 0x01010101u, nwords, s);  // round 0: every vertex
+    launch_fill_u32(reinterpret_cast<uint32_t *>(w.flags[1]), 0u, nwords, s);
     // labels only drop and stay ids of the component: at most n rounds
     const uint64_t limit = max_rounds ? max_rounds : (uint64_t)n + 1;
     uint32_t rounds = 0;
     uint64_t evaluated = 0;
     bool fixed = false, stopped = false;
     int cur = 0;
-    while (rounds < limit) {
-        uint8_t *fc = w.flags[cur], *fn = w.flags[cur ^ 1];
-        launch_fill_u32(reinterpret_cast<uint32_t *>(fn), 0u, nwords, s);
-        launch_fill_u32(reinterpret_cast<uint32_t *>(w.dropped), 0u, nwords, s);
-        launch_fill_u32(w.ctr, 0u, 2, s);
-        launch_fill_u64(reinterpret_cast<uint64_t *>(w.stat), 0ull, 3, s);
-        hipLaunchKernelGGL(ccs_compact, dim3(grid_for(n, 256 * 16, 1024)), dim3(256), 0, s, d_off, n, fc,
-                           w.short_list, w.items, w.ctr, w.stat);
-        hipLaunchKernelGGL(ccs_short, dim3(gl), dim3(256), 0, s, d_off, d_adj, n, d_labels, w.short_list, w.ctr, fn,
-                           w.stat);
-        hipLaunchKernelGGL(ccs_long_min, dim3(gw), dim3(256), 0, s, d_off, d_adj, n, d_labels, w.items, w.ctr,
-                           w.dropped, w.stat);
-        hipLaunchKernelGGL(ccs_long_mark, dim3(gw), dim3(256), 0, s, d_off, d_adj, n, w.items, w.ctr, w.dropped, fn,
-                           w.stat);
+    // Without a hook two rounds go out per readback: a round behind the fixed
+    // point has nothing scheduled.
+    while (rounds < limit && !fixed && !stopped) {
+        const uint32_t batch = !on_round && limit - rounds > 1 ? 2 : 1;
+        launch_fill_u64(reinterpret_cast<uint64_t *>(w.stat), 0ull, 8, s);  // and the list counters
+        for (uint32_t k = 0; k < batch; k++, cur ^= 1) {
+            uint8_t *fc = w.flags[cur], *fn = w.flags[cur ^ 1];
+            unsigned long long *stat = w.stat + 4 * k;
+            uint32_t *ctr = reinterpret_cast<uint32_t *>(stat + 3);
+            const int first = rounds + k == 0;
+            hipLaunchKernelGGL(ccs_compact, dim3((unsigned)div_up(n, (uint64_t)kCcsThreads * kCcsPer)),
+                               dim3(kCcsThreads), 0, s, d_off, n, fc, w.short_list, w.items, w.dropped, ctr, stat);
+            hipLaunchKernelGGL(ccs_long_min, dim3(gw), dim3(256), 0, s, d_off, d_adj, n, d_labels, w.items, ctr,
+                               w.dropped, first, stat);
+            hipLaunchKernelGGL(ccs_long_mark, dim3(gw), dim3(256), 0, s, d_off, d_adj, n, w.items, ctr, w.dropped, fn,
+                               stat);
+            hipLaunchKernelGGL(ccs_short, dim3(gl), dim3(256), 0, s, d_off, d_adj, n, d_labels, w.short_list, ctr, fn,
+                               first, stat);
+        }
         GCHI_LAUNCH_CHECK();
-        unsigned long long st[3] = {0, 0, 0};
+        unsigned long long st[8] = {};
         GCHI_HIP(hipMemcpyAsync(st, w.stat, sizeof(st), hipMemcpyDeviceToHost, s));
         GCHI_HIP(hipStreamSynchronize(s));
-        GCHI_CHECK(st[2] == 0, GCHI_ERR_INVALID, "cc_scheduled: neighbour id >= nvertices");
-        rounds++;
-        evaluated += st[1];
-        if (st[0] == 0) fixed = true;
-        if (on_round && on_round(user, rounds - 1, st[0], st[1]) != 0) {
-            stopped = true;
-            break;
+        for (uint32_t k = 0; k < batch && !fixed && !stopped; k++) {
+            const unsigned long long *r = st + 4 * k;
+            GCHI_CHECK(r[2] == 0, GCHI_ERR_INVALID, "cc_scheduled: neighbour id >= nvertices");
+            rounds++;
+            evaluated += r[1];
+            if (r[0] == 0) fixed = true;
+            if (on_round && on_round(user, rounds - 1, r[0], r[1]) != 0) stopped = true;
         }
-        if (fixed) break;
-        cur ^= 1;
     }
     *h_rounds = rounds;
     if (h_evaluated) *h_evaluated = evaluated;

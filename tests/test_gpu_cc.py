@@ -209,3 +209,27 @@ def test_cc_pull_scale24_equals_unionfind(dev):
     lab, sweeps = dev.cc_pull(g.in_off, g.in_src, n)
     np.testing.assert_array_equal(dev.to_host_u32(lab, n), want)
     print(f"\npull sweeps at scale 24: {sweeps}")
+
+
+@pytest.mark.parametrize("n,edges,extra", [(17, 40, 0), (16385, 60000, 0), (33000, 200000, 9000)])
+def test_cc_scheduled_zero_component_and_padding(dev, n, edges, extra):
+    """Vertex counts around the compaction's groups of 16 and workgroups of
+    16384 vertices; components with and without vertex 0 (rows of the first stop
+    at a 0, the others are read whole), rows around 64 entries and one of `extra`
+    entries; a bad neighbour id behind an early 0 is still refused."""
+    rng = np.random.default_rng(n)
+    half = n // 2
+    a, b = rng.integers(0, half, edges), rng.integers(0, half, edges)
+    c, d = rng.integers(half, n, edges // 3), rng.integers(half, n, edges // 3)
+    src = np.concatenate([a, c, np.zeros(64, np.int64), np.full(extra, half - 1)]).astype(np.uint32)
+    dst = np.concatenate([b, d, np.arange(64) % max(half, 1), rng.integers(0, half, extra)]).astype(np.uint32)
+    g = _sym_csr(dev, src, dst, n)
+    lab, rounds, evals = dev.cc_scheduled(g.in_off, g.in_src, n)
+    np.testing.assert_array_equal(dev.to_host_u32(lab, n), oracle.cc_unionfind(n, src, dst))
+    assert rounds >= 1 and evals >= n
+    adj = dev.to_host_u32(g.in_src, g.E).copy()
+    off = dev.to_host_u32(g.in_off, n + 1)
+    v = int(np.argmax(np.diff(off.astype(np.int64))))
+    adj[off[v + 1] - 1] = n
+    with pytest.raises(dev.GchiError):
+        dev.cc_scheduled(g.in_off, dev.to_dev_u32(adj), n)
