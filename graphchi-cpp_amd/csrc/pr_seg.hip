@@ -574,47 +574,19 @@ __global__ void seg_order_keys(const uint32_t *outdeg, uint32_t n, uint64_t *key
         keys[v] = ((uint64_t)(0xffffffffu - outdeg[v]) << 32) | v;
 }
 
+constexpr uint32_t kNoEdges = 0xffffffffu;  // row_beg of a row without in-edges
 __global__ void seg_ranks(const uint64_t *keys, const uint32_t *in_off, const uint32_t *outdeg, uint32_t n,
-                          uint32_t *perm, uint32_t *rank, uint32_t *outdeg_r, uint32_t *nslot) {
+                          uint32_t *perm, uint32_t *rank, uint32_t *outdeg_r, uint32_t *nslot, uint32_t *row_beg) {
     uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const uint32_t v = (uint32_t)keys[i];
         perm[i] = v;
         rank[v] = i;
         outdeg_r[i] = outdeg[v];
-        const uint32_t d = in_off[v + 1] - in_off[v];
+        const uint32_t b = in_off[v], d = in_off[v + 1] - b;
         nslot[i] = d ? d : 1u;
+        row_beg[i] = d ? b : kNoEdges;
     }
-}
-
-// One wavefront per row: its sources' ranks into its slots (N for a row with
-// none); row-start flag bits.  A source id >= n sets *bad and is stored as N.
-__global__ void seg_fill(const uint32_t *in_off, const uint32_t *in_src, const uint32_t *perm, const uint32_t *rank,
-                         const uint64_t *soff, uint32_t n, uint32_t *slots, uint32_t *flag_words, uint32_t *bad) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint64_t wid = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / kWave;
-    for (uint64_t i = wid; i < n; i += nw) {
-        const uint32_t v = perm[i];
-        const uint32_t b = in_off[v], e = in_off[v + 1];
-        const uint64_t s0 = soff[i];
-        if (lane == 0) {
-            atomicOr(&flag_words[s0 >> 5], 1u << (s0 & 31));
-            if (e == b) slots[s0] = n;
-        }
-        for (uint32_t k = b + lane; k < e; k += kWave) {
-            const uint32_t u = in_src[k];
-            uint32_t ru = n;
-            if (u < n) ru = rank[u];
-            else atomicOr(bad, 1u);
-            slots[s0 + (k - b)] = ru;
-        }
-    }
-}
-
-__global__ void seg_fill_value(uint32_t *p, uint64_t n, uint32_t v) {
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
 // last row whose first slot is <= s (soff strictly increasing, soff[0] = 0)
@@ -639,6 +611,75 @@ __global__ void seg_tiles(const uint64_t *soff, uint32_t n, uint64_t S, uint32_t
         }
         tile_row0[t] = meta;
     }
+}
+
+// One wavefront per tile, all 512 slots in flight at once: the tile's rows set a
+// bit at their first slot, so a slot's row is the count of bits up to it and
+// its in-edge is that row's first one plus a distance; the rank gathers (8 per
+// lane, independent) are what is left to wait for.  The flag bits are those
+// same words, stored whole.  Slots from S on hold N and no flag.  A source id
+// >= n sets *bad and is stored as N.  One wavefront per row instead, whatever
+// its length, took 1,213 us on 33.6M edges of an R-MAT graph of 2^21 vertices,
+// where most rows have a few edges; 221 us.
+constexpr int kFillThreads = 256;
+constexpr int kFillWaves = kFillThreads / kWave;
+constexpr int kFillWords = kSegTile / 64;
+__global__ __launch_bounds__(kFillThreads) void seg_fill(const uint32_t *__restrict__ in_src,
+                                                         const uint32_t *__restrict__ row_beg,
+                                                         const uint32_t *__restrict__ rank,
+                                                         const uint64_t *__restrict__ soff,
+                                                         const uint32_t *__restrict__ tile_row0, uint32_t n, uint64_t S,
+                                                         uint32_t T, uint32_t *__restrict__ slots,
+                                                         uint64_t *__restrict__ flag_words, uint32_t *bad) {
+    __shared__ uint32_t s_base[kFillWaves][kSegTile + 1];  // first in-edge of a row, less its first slot
+    __shared__ uint64_t s_mark[kFillWaves][kFillWords], s_none[kFillWaves][kFillWords];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    const uint32_t t = blockIdx.x * kFillWaves + wave;
+    if (t >= T) return;  // no barrier below: a wavefront works alone
+    uint32_t *base = s_base[wave];
+    uint64_t *mark = s_mark[wave], *none = s_none[wave];
+    if (lane < kFillWords) mark[lane] = none[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t q0 = (uint64_t)t * kSegTile;
+    const uint32_t row0 = tile_row0[t] & ~kSegCont;
+    const uint32_t rows = (t + 1 < T ? tile_row0[t + 1] & ~kSegCont : n - 1) - row0 + 1;  // <= kSegTile + 1
+    for (uint32_t i = lane; i < rows; i += kWave) {
+        const uint64_t q = soff[row0 + i];
+        if (q >= q0 + kSegTile) continue;  // the next tile's first row
+        const uint32_t b = row_beg[row0 + i];
+        base[i] = b - (uint32_t)(q - q0);  // modulo 2^32; a row begun before the tile adds the distance
+        if (q >= q0) {
+            const uint32_t at = (uint32_t)(q - q0);
+            atomicOr(reinterpret_cast<unsigned long long *>(&mark[at / 64]), 1ull << (at % 64));
+            if (b == kNoEdges) atomicOr(reinterpret_cast<unsigned long long *>(&none[at / 64]), 1ull << (at % 64));
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t before = (mark[0] & 1ull) ? 0u : 1u;  // a row begun before the tile is row 0 of it
+    uint32_t src[kFillWords];
+    bool ok[kFillWords];
+#pragma unroll
+    for (int j = 0; j < kFillWords; j++) {
+        const uint64_t m = mark[j];
+        const uint32_t at = (uint32_t)j * 64 + lane;
+        const uint32_t r = before + (uint32_t)__popcll(m & (lanemask_lt() | (1ull << lane))) - 1;
+        before += (uint32_t)__popcll(m);
+        ok[j] = q0 + at < S && !((none[j] >> lane) & 1ull);
+        src[j] = ok[j] ? in_src[base[r] + at] : n;
+        if (lane == 0) flag_words[(uint64_t)t * kFillWords + j] = m;
+    }
+    bool out = false;
+#pragma unroll
+    for (int j = 0; j < kFillWords; j++) {
+        out |= ok[j] && src[j] >= n;
+        ok[j] = ok[j] && src[j] < n;
+        src[j] = ok[j] ? rank[src[j]] : n;
+    }
+#pragma unroll
+    for (int j = 0; j < kFillWords; j++) slots[q0 + (uint32_t)j * 64 + lane] = src[j];
+    if (out) atomicOr(bad, 1u);
 }
 
 // split[i] = 1 when row i's first and last slot lie in tiles of different
@@ -716,6 +757,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     uint32_t *rank = tp.alloc<uint32_t>(N);
     uint32_t *nslot = tp.alloc<uint32_t>(N + 1);
     uint64_t *soff = tp.alloc<uint64_t>((size_t)N + 1);
+    uint32_t *row_beg = tp.alloc<uint32_t>(N);
     uint32_t *split = tp.alloc<uint32_t>(N + 1);
     uint32_t *spos = tp.alloc<uint32_t>(N + 1);
     uint32_t *bad = tp.alloc<uint32_t>(1);
@@ -723,7 +765,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     GCHI_TRY(gchi_sort_workspace(N, 64, 0, &sb));
     const size_t swb = std::max(sb, scan_workspace((size_t)N + 1));
     void *sw = tp.alloc<char>(swb);
-    GCHI_CHECK(keys && rank && nslot && soff && split && spos && bad && sw, GCHI_ERR_HIP,
+    GCHI_CHECK(keys && rank && nslot && soff && row_beg && split && spos && bad && sw, GCHI_ERR_HIP,
                "pr_plan (form 4): hipMalloc failed");
     gchi_seg_plan *p = new gchi_seg_plan();
     p->N = N;
@@ -742,7 +784,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     uint32_t *perm_t = tp.alloc<uint32_t>(N), *od_t = tp.alloc<uint32_t>(N);
     if (!perm_t || !od_t) return fail_free(fail(GCHI_ERR_HIP, "pr_plan (form 4): hipMalloc failed"));
     hipLaunchKernelGGL(seg_ranks, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, keys, g->in_off, g->outdeg, N,
-                       perm_t, rank, od_t, nslot);
+                       perm_t, rank, od_t, nslot, row_beg);
     if ((st = exclusive_scan_u32_to_u64(nslot, soff, N, sw, swb, s)) != GCHI_OK) return fail_free(st);
     uint64_t S = 0;
     if ((st = seg_read(&S, soff + N, 8, s)) != GCHI_OK) return fail_free(st);
@@ -817,19 +859,15 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     p->rs[1] = c.take<float>(N);
     GCHI_HIP(hipMemcpyAsync(p->perm, perm_t, (size_t)N * 4, hipMemcpyDeviceToDevice, s));
     GCHI_HIP(hipMemcpyAsync(p->outdeg_r, od_t, (size_t)N * 4, hipMemcpyDeviceToDevice, s));
-    launch_fill_u32(flag_words, 0u, nslots / 32, s);
     launch_fill_u32(bad, 0u, 1, s);
     launch_fill_u32(p->counter, 0u, 64, s);
     // x of the no-source id N stays 0 in both state buffers: sweeps never
     // write it, and rows without in-edges gather it
     launch_fill_u32(reinterpret_cast<uint32_t *>(p->xs[0]) + N, 0u, 1, s);
     launch_fill_u32(reinterpret_cast<uint32_t *>(p->xs[1]) + N, 0u, 1, s);
-    if (nslots > S)
-        hipLaunchKernelGGL(seg_fill_value, dim3(grid_for(nslots - S, 256, 4096)), dim3(256), 0, s, p->slots + S,
-                           nslots - S, N);
-    hipLaunchKernelGGL(seg_fill, dim3(grid_for((uint64_t)N * kWave, 256, 1u << 16)), dim3(256), 0, s, g->in_off,
-                       g->in_src, p->perm, rank, soff, N, p->slots, flag_words, bad);
     hipLaunchKernelGGL(seg_tiles, dim3(grid_for(T, 256, 65536)), dim3(256), 0, s, soff, N, S, T, p->tile_row0);
+    hipLaunchKernelGGL(seg_fill, dim3((T + kFillWaves - 1) / kFillWaves), dim3(kFillThreads), 0, s, g->in_src, row_beg,
+                       rank, soff, p->tile_row0, N, S, T, p->slots, reinterpret_cast<uint64_t *>(flag_words), bad);
     if (nsplit)
         hipLaunchKernelGGL(seg_split_list, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, soff, split, spos, N,
                            p->split_v, p->split_beg, p->split_end);

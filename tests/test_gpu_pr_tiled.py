@@ -175,3 +175,30 @@ def test_tiled_personalized_matches_vertex_layout(dev):
         ex.launch()
         outs.append(ex.ranks().cpu().numpy().copy())
     assert_close(outs[1], outs[0])
+
+
+@pytest.mark.parametrize("n", [511, 512, 513, 1024, 1537])
+@pytest.mark.parametrize("shape", ["one", "one_row", "gaps"])
+def test_tiled_plan_rows_at_tile_edges(dev, n, shape):
+    """Tiles full of one-slot rows, one row over whole tiles and empty rows on
+    either side of a tile's edge: row sums of at most two terms equal the FP32
+    oracle's bit for bit, the long row's the FP64 oracle's to the module's
+    tolerance (511 equal terms added one by one in FP32 are themselves further
+    off than that)."""
+    v = np.arange(n, dtype=np.uint32)
+    if shape == "one":  # a ring: every row has one in-edge, 512 rows to a tile
+        src, dst = v, np.roll(v, 1)
+    elif shape == "one_row":  # vertex 0 takes n - 1 in-edges, the others none
+        src, dst = v[1:], np.zeros(n - 1, np.uint32)
+    else:  # every third row empty, every third with two in-edges
+        dst = np.concatenate([v[v % 3 == 1], v[v % 3 == 2], v[v % 3 == 2]])
+        src = ((dst.astype(np.uint64) * 7 + 1 + np.arange(len(dst)) % 5) % n).astype(np.uint32)
+    g = dev.DeviceGraph(dev.to_dev_u32(src), dev.to_dev_u32(dst), n)
+    in_off, in_src, outdeg, _ = oracle.csc(n, src, dst)
+    want, _ = oracle.pagerank_f32(n, in_off, in_src, outdeg, 0.15, DAMPING, 1.0, 3)
+    for tune in FORMS[:2]:
+        r, _, _, _ = run(dev, g, tune, 0.15, 3)
+        if shape == "one_row":
+            assert_close(r, oracle.pagerank_f64(n, in_off, in_src, outdeg, 0.15, DAMPING, 1.0, 3))
+        else:
+            np.testing.assert_array_equal(r, want)
