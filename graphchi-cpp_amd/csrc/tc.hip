@@ -728,7 +728,7 @@ static void tc_prep_layout(C &c, uint64_t E, uint32_t N, uint32_t **deg, uint64_
 
 // deg[v] += in + out degree of v without self-loops (deg zeroed by the caller),
 // from runs of equal ids: the src passes order the keys by src, the dst passes
-// by dst.  vkeys (N+1 entries) serves as run-start scratch, ekeys and sw as the
+// by dst.  vkeys (N+1 entries) serves as scratch of the runs' ends, ekeys and sw as the
 // sort buffers.
 static int tc_degree_counts(const uint32_t *src, const uint32_t *dst, uint64_t E, uint32_t N, uint32_t *deg,
                             uint32_t *err, uint64_t *vkeys, uint64_t *ekeys, void *sw, size_t swb, hipStream_t s) {
@@ -736,15 +736,15 @@ static int tc_degree_counts(const uint32_t *src, const uint32_t *dst, uint64_t E
     const int fb = bits_for(N);  // wide enough for n, the skip mark
     const int sb = (fb + 7) / 8 * 8;
     const uint32_t fmask = fb >= 32 ? 0xffffffffu : ((1u << fb) - 1u);
-    uint32_t *run_start = reinterpret_cast<uint32_t *>(vkeys);
+    uint32_t *run_start = reinterpret_cast<uint32_t *>(vkeys), *run_end = run_start + N;
     hipLaunchKernelGGL(tc_degree_pack, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, src, dst, E, N, sb, ekeys, err);
     GCHI_LAUNCH_CHECK();
     uint64_t *by_src = nullptr, *by_dst = nullptr;
     GCHI_TRY(radix_sort_u64_bits(ekeys, nullptr, nullptr, E, 0, sb, sw, swb, s, &by_src, err));
-    GCHI_TRY(count_field_runs(by_src, E, 0, fmask, N, run_start, deg, nullptr, 0u, s, true));
+    GCHI_TRY(count_field_runs(by_src, E, 0, fmask, N, run_start, deg, nullptr, 0u, s, run_end));
     GCHI_TRY(radix_sort_u64_bits(by_src, by_src == ekeys ? nullptr : ekeys, nullptr, E, sb, sb + fb, sw, swb, s,
                                  &by_dst, err));
-    return count_field_runs(by_dst, E, sb, fmask, N, run_start, deg, nullptr, 0u, s, true);
+    return count_field_runs(by_dst, E, sb, fmask, N, run_start, deg, nullptr, 0u, s, run_end);
 }
 
 }  // namespace gchi
