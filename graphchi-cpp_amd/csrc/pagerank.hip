@@ -1251,14 +1251,17 @@ __global__ void plan_graph_hubs(const uint32_t *hub_v, uint32_t nhub, const uint
 
 // Temporary device allocations of the plan build, freed on every exit path.
 struct TmpPool {
+    hipStream_t s;
     std::vector<void *> ptrs;
+    explicit TmpPool(hipStream_t stream) : s(stream) {}
     ~TmpPool() {
-        for (void *q : ptrs) (void)hipFree(q);
+        const hipError_t waited = hipStreamSynchronize(s);
+        for (void *q : ptrs) pool_free(q, waited);
     }
     template <typename T>
     T *alloc(size_t count) {
         void *q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return nullptr;
+        if (pool_alloc(&q, std::max<size_t>(count, 1) * sizeof(T), s) != hipSuccess) return nullptr;
         ptrs.push_back(q);
         return static_cast<T *>(q);
     }
@@ -1291,7 +1294,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     const uint32_t N = in.N;
     const uint64_t E = in.E;
     const uint32_t G = in.G;
-    TmpPool tp;
+    TmpPool tp(s);
     const size_t nwords = (N + 31) / 32;
     uint32_t *off_ext = tp.alloc<uint32_t>((size_t)N + G);
     uint64_t *g_src = tp.alloc<uint64_t>(G);
@@ -1319,7 +1322,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
         GCHI_LAUNCH_CHECK();
     } else {
         // per-graph CSCs: offsets and out-degrees copied side by side, ids offset by vbase
-        GCHI_HIP(hipMalloc(&p->own_outdeg, (size_t)std::max<uint32_t>(N, 1) * 4));
+        GCHI_HIP(pool_alloc(reinterpret_cast<void **>(&p->own_outdeg), (size_t)std::max<uint32_t>(N, 1) * 4, s));
         p->outdeg = p->own_outdeg;
         std::vector<uint64_t> h_src(G);
         for (uint32_t k = 0; k < G; k++) {
@@ -1434,7 +1437,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint64_t>(G);
-    GCHI_HIP(hipMalloc(&p->mem, zz.off));
+    GCHI_HIP(pool_alloc(&p->mem, zz.off, s));
     Carver c(p->mem, zz.off);
     p->reg_off = c.take<uint32_t>((size_t)N + G);
     p->reg_src = c.take<uint32_t>(std::max<uint64_t>(p->e_reg, 1));
@@ -1602,8 +1605,8 @@ static int plan_create(const PlanInput &in, const gchi_pr_tune *tune, gchi_pr_pl
         }
     }
     if (st != GCHI_OK) {
-        if (p->mem) (void)hipFree(p->mem);
-        if (p->own_outdeg) (void)hipFree(p->own_outdeg);
+        pool_free_device(p->mem);
+        pool_free_device(p->own_outdeg);
         delete p;
         return st;
     }
@@ -1760,8 +1763,8 @@ extern "C" int gchi_pr_plan_create_batch(const gchi_dgraph *graphs, uint32_t ngr
 extern "C" int gchi_pr_plan_destroy(gchi_pr_plan *p) {
     if (!p) return GCHI_OK;
     seg_plan_destroy(p->seg);
-    if (p->mem) (void)hipFree(p->mem);
-    if (p->own_outdeg) (void)hipFree(p->own_outdeg);
+    pool_free_device(p->mem);
+    pool_free_device(p->own_outdeg);
     delete p;
     return GCHI_OK;
 }

@@ -728,14 +728,17 @@ struct gchi_seg_plan {
 namespace gchi {
 
 struct SegTmp {
+    hipStream_t s;
     std::vector<void *> ptrs;
+    explicit SegTmp(hipStream_t stream) : s(stream) {}
     ~SegTmp() {
-        for (void *q : ptrs) (void)hipFree(q);
+        const hipError_t waited = hipStreamSynchronize(s);
+        for (void *q : ptrs) pool_free(q, waited);
     }
     template <typename T>
     T *alloc(size_t count) {
         void *q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return nullptr;
+        if (pool_alloc(&q, std::max<size_t>(count, 1) * sizeof(T), s) != hipSuccess) return nullptr;
         ptrs.push_back(q);
         return static_cast<T *>(q);
     }
@@ -752,7 +755,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     const uint64_t E = g->nedges;
     GCHI_CHECK(N > 0 && N < (1u << 31), GCHI_ERR_UNSUPPORTED, "pr_plan (form 4): needs 0 < N < 2^31");
     GCHI_CHECK(hot >= -1, GCHI_ERR_INVALID, "pr_plan (form 4): hot_vertices must be -1, 0 or positive");
-    SegTmp tp;
+    SegTmp tp(s);
     uint64_t *keys = tp.alloc<uint64_t>(N);
     uint32_t *rank = tp.alloc<uint32_t>(N);
     uint32_t *nslot = tp.alloc<uint32_t>(N + 1);
@@ -771,7 +774,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     p->N = N;
     p->E = E;
     auto fail_free = [&](int st) {
-        if (p->mem) (void)hipFree(p->mem);
+        pool_free(p->mem, hipStreamSynchronize(s));
         delete p;
         return st;
     };
@@ -834,7 +837,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     z.take<float>((size_t)N + 1);        // xs[1]
     z.take<float>(N);                    // rs[0]
     z.take<float>(N);                    // rs[1]
-    if (hipMalloc(&p->mem, z.off) != hipSuccess) {
+    if (pool_alloc(&p->mem, z.off, s) != hipSuccess) {
         p->mem = nullptr;
         return fail_free(fail(GCHI_ERR_HIP, "pr_plan (form 4): hipMalloc failed (" + std::to_string(z.off) +
                                                 " bytes)"));
@@ -897,7 +900,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
 
 void seg_plan_destroy(gchi_seg_plan *p) {
     if (!p) return;
-    if (p->mem) (void)hipFree(p->mem);
+    pool_free_device(p->mem);
     delete p;
 }
 

@@ -151,10 +151,13 @@ __global__ void sh_run_flags(const uint32_t *src, uint64_t e, uint32_t *flags) {
         flags[i] = (i == 0 || src[i] != src[i - 1]) ? 1u : 0u;
 }
 
+// first record of every run; run_start[runs] = e
 __global__ void sh_run_starts(const uint32_t *flags, const uint32_t *ridx, uint64_t e, uint32_t *run_start) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < e; i += stride)
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < e; i += stride) {
         if (flags[i]) run_start[ridx[i]] = (uint32_t)i;
+        if (i == 0) run_start[ridx[e]] = (uint32_t)e;
+    }
 }
 
 GCHI_HD uint64_t zero_bytes(uint32_t gap) { return gap ? 2ull * ((gap + 254u) / 255u) : 0ull; }
@@ -218,9 +221,10 @@ __global__ void sh_write_dsts(const uint32_t *src, const uint32_t *dst, const ui
     }
 }
 
-// .adjidx: greedy over run starts (first run start >= last + 1M), one thread
+// .adjidx: greedy over run starts (first run start >= last + 1M), one thread.
+// out[0] = the stream's bytes, out[1] = entries
 __global__ void sh_index(const uint32_t *src, const uint32_t *run_start, uint32_t nruns, const uint64_t *off,
-                         uint64_t *triples, uint32_t max_entries, uint32_t *count) {
+                         uint64_t *triples, uint32_t max_entries, uint64_t *out) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     uint64_t last = 0;
     uint32_t ni = 0;
@@ -243,7 +247,8 @@ __global__ void sh_index(const uint32_t *src, const uint32_t *run_start, uint32_
         last = b;
         lo_k = k + 1;
     }
-    *count = ni;
+    out[0] = off[nruns];
+    out[1] = ni;
 }
 
 static int sh_read(void *h, const void *d, size_t n, hipStream_t s) {
@@ -300,7 +305,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     zz.take<uint32_t>(E + 1);
     zz.take<uint32_t>(E + 1);
     zz.take<int32_t>(2 * (size_t)N);
-    if (hipMalloc(&sh->mem, zz.off) != hipSuccess) {
+    if (pool_alloc(&sh->mem, zz.off, s) != hipSuccess) {
         delete sh;
         return fail(GCHI_ERR_HIP, "shard_build: hipMalloc failed");
     }
@@ -324,8 +329,8 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     size_t swb = std::max(sort_workspace_bytes(E, std::max(db, pb), false), scan_workspace((size_t)N + 1));
     z.take<char>(swb);
     void *scratch = nullptr;
-    if (hipMalloc(&scratch, z.off) != hipSuccess) {
-        (void)hipFree(sh->mem);
+    if (pool_alloc(&scratch, z.off, s) != hipSuccess) {
+        pool_free(sh->mem, hipSuccess);
         delete sh;
         return fail(GCHI_ERR_HIP, "shard_build: hipMalloc failed");
     }
@@ -341,9 +346,10 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     uint64_t *keys = sc.take<uint64_t>(E + 1);
     void *sw = sc.take<char>(swb);
     auto done = [&](int st) {
-        (void)hipFree(scratch);
+        const hipError_t waited = hipStreamSynchronize(s);
+        pool_free(scratch, waited);
         if (st != GCHI_OK) {
-            (void)hipFree(sh->mem);
+            pool_free(sh->mem, waited);
             delete sh;
         } else {
             *out = sh;
@@ -377,10 +383,15 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     if (st == GCHI_OK) {
         hipLaunchKernelGGL(sh_interval_cut, dim3(1), dim3(64), 0, s, P, N, max_id, nshards, d_ends, d_counts, d_ns,
                            d_ns + 1);
+        // ends, counts, created / status and the error word in one copy
+        const char *m0 = reinterpret_cast<const char *>(d_ends), *m1 = reinterpret_cast<const char *>(err + 1);
+        std::vector<char> meta(m1 - m0);
+        st = sh_read(meta.data(), m0, meta.size(), s);
+        auto at = [&](const void *d) { return meta.data() + (static_cast<const char *>(d) - m0); };
         int h_ns[2] = {0, 0};
         uint32_t h_err = 0;
-        st = sh_read(h_ns, d_ns, sizeof(h_ns), s);
-        if (st == GCHI_OK) st = sh_read(&h_err, err, 4, s);
+        memcpy(h_ns, at(d_ns), sizeof(h_ns));
+        memcpy(&h_err, at(err), 4);
         if (st == GCHI_OK && (h_err & GCHI_WORK_TIMEOUT))
             st = fail(GCHI_ERR_TIMEOUT, "shard_build: a sort look-back wait gave up");
         if (st == GCHI_OK && h_err) st = fail(GCHI_ERR_INVALID, "shard_build: vertex id > max_id");
@@ -390,8 +401,8 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
             sh->nshards = h_ns[0];
             sh->ends.resize(sh->nshards);
             sh->counts.resize(sh->nshards);
-            st = sh_read(sh->ends.data(), d_ends, 4 * sh->nshards, s);
-            if (st == GCHI_OK) st = sh_read(sh->counts.data(), d_counts, 8 * sh->nshards, s);
+            memcpy(sh->ends.data(), at(d_ends), 4 * (size_t)sh->nshards);
+            memcpy(sh->counts.data(), at(d_counts), 8 * (size_t)sh->nshards);
         }
     }
     if (st == GCHI_OK && E) {
@@ -416,7 +427,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
 
 extern "C" int gchi_shard_destroy(gchi_shards *sh) {
     if (!sh) return GCHI_OK;
-    if (sh->mem) (void)hipFree(sh->mem);
+    pool_free_device(sh->mem);
     delete sh;
     return GCHI_OK;
 }
@@ -466,12 +477,12 @@ extern "C" int gchi_shard_encode(const gchi_shards *sh, int shard, uint8_t *h_ad
     z.take<uint32_t>(e + 1);  // sizes
     z.take<uint64_t>(e + 2);  // offsets
     z.take<uint64_t>(3 * (size_t)(max_index + 1));
-    z.take<uint32_t>(1);
+    z.take<uint64_t>(2);
     size_t swb = scan_workspace(e + 1);
     z.take<char>(swb);
     z.take<uint8_t>(1);
     void *scratch = nullptr;
-    GCHI_HIP(hipMalloc(&scratch, z.off));
+    GCHI_HIP(pool_alloc(&scratch, z.off, s));
     Carver c(scratch, z.off);
     uint32_t *flags = c.take<uint32_t>(e + 1);
     uint32_t *ridx = c.take<uint32_t>(e + 1);
@@ -479,7 +490,7 @@ extern "C" int gchi_shard_encode(const gchi_shards *sh, int shard, uint8_t *h_ad
     uint32_t *sizes = c.take<uint32_t>(e + 1);
     uint64_t *off = c.take<uint64_t>(e + 2);
     uint64_t *d_idx = c.take<uint64_t>(3 * (size_t)(max_index + 1));
-    uint32_t *d_nidx = c.take<uint32_t>(1);
+    uint64_t *d_out = c.take<uint64_t>(2);
     void *sw = c.take<char>(swb);
     uint8_t *adj = nullptr;
     int st = GCHI_OK;
@@ -490,38 +501,46 @@ extern "C" int gchi_shard_encode(const gchi_shards *sh, int shard, uint8_t *h_ad
     if (st == GCHI_OK) st = sh_read(&nruns, ridx + e, 4, s);
     if (st == GCHI_OK) {
         hipLaunchKernelGGL(sh_run_starts, dim3(grid_for(e, 256, 65536)), dim3(256), 0, s, flags, ridx, e, rstart);
-        uint32_t ee = (uint32_t)e;
-        if (hipMemcpyAsync(rstart + nruns, &ee, 4, hipMemcpyHostToDevice, s) != hipSuccess)
-            st = fail(GCHI_ERR_HIP, "shard_encode: copy failed");
     }
     if (st == GCHI_OK) {
         hipLaunchKernelGGL(sh_run_sizes, dim3(grid_for(nruns, 256, 65536)), dim3(256), 0, s, src, rstart, nruns,
                            sizes);
         st = exclusive_scan_u32_to_u64(sizes, off, nruns, sw, swb, s);
     }
-    if (st == GCHI_OK) st = sh_read(&total, off + nruns, 8, s);
-    *adj_bytes = total;
-    if (st == GCHI_OK && h_adj) {
-        if (hipMalloc(&adj, total) != hipSuccess) st = fail(GCHI_ERR_HIP, "shard_encode: hipMalloc failed");
+    if (st == GCHI_OK && !h_adj) {
+        st = sh_read(&total, off + nruns, 8, s);
+    } else if (st == GCHI_OK) {
+        // the stream's bytes are known only on the device: at most 4 per record, 5
+        // and one zero pair per run, and a pair per 255 vertices without records
+        const size_t most = 4 * (size_t)e + 7 * (size_t)nruns + 2 * ((size_t)sh->max_id / 255 + 1);
+        uint64_t out[2] = {0, 0};
+        const uint32_t want = h_index && nindex ? max_index : 0u;
+        if (pool_alloc(reinterpret_cast<void **>(&adj), most, s) != hipSuccess)
+            st = fail(GCHI_ERR_HIP, "shard_encode: hipMalloc failed");
         if (st == GCHI_OK) {
             hipLaunchKernelGGL(sh_write_heads, dim3(grid_for(nruns, 256, 65536)), dim3(256), 0, s, src, rstart, nruns,
                                off, adj);
             hipLaunchKernelGGL(sh_write_dsts, dim3(grid_for(e, 256, 65536)), dim3(256), 0, s, src, dst, flags, ridx,
                                rstart, e, off, adj);
-            if (h_index && nindex)
-                hipLaunchKernelGGL(sh_index, dim3(1), dim3(64), 0, s, src, rstart, nruns, off, d_idx, max_index,
-                                   d_nidx);
+            hipLaunchKernelGGL(sh_index, dim3(1), dim3(64), 0, s, src, rstart, nruns, off, d_idx, want, d_out);
             hipError_t le = hipGetLastError();
             if (le != hipSuccess) st = hip_fail(le, "shard_encode kernels", __FILE__, __LINE__);
         }
-        if (st == GCHI_OK) st = sh_read(h_adj, adj, total, s);
-        if (st == GCHI_OK && h_index && nindex) {
-            st = sh_read(nindex, d_nidx, 4, s);
-            if (st == GCHI_OK && *nindex) st = sh_read(h_index, d_idx, 24 * (size_t)*nindex, s);
+        if (st == GCHI_OK) st = sh_read(out, d_out, sizeof(out), s);
+        total = out[0];
+        hipError_t ce = hipSuccess;
+        if (st == GCHI_OK) ce = hipMemcpyAsync(h_adj, adj, total, hipMemcpyDeviceToHost, s);
+        if (st == GCHI_OK && ce == hipSuccess && want) {
+            *nindex = (uint32_t)out[1];
+            if (out[1]) ce = hipMemcpyAsync(h_index, d_idx, 24 * (size_t)out[1], hipMemcpyDeviceToHost, s);
         }
+        if (st == GCHI_OK && ce == hipSuccess) ce = hipStreamSynchronize(s);
+        if (st == GCHI_OK && ce != hipSuccess) st = hip_fail(ce, "shard_encode copies", __FILE__, __LINE__);
     }
-    if (adj) (void)hipFree(adj);
-    (void)hipFree(scratch);
+    *adj_bytes = total;
+    const hipError_t waited = hipStreamSynchronize(s);
+    pool_free(adj, waited);
+    pool_free(scratch, waited);
     return st;
 }
 

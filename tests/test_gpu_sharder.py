@@ -159,3 +159,49 @@ def test_reference_cc_consumes_device_shards_with_zlib_edata(dev, golden):
         np.testing.assert_array_equal(np.fromfile(base + ".4B.vout", dtype=np.uint32), golden["cc_rmat14_p3__labels"])
     finally:
         shutil.rmtree(tmp, ignore_errors=True)
+
+
+def test_builds_share_pooled_memory_over_threads_and_streams(dev):
+    """Plans and shards built, used and destroyed by four threads on streams of
+    their own, in sizes that reuse one another's freed memory, give what one
+    thread on one stream gives, bit for bit."""
+    import threading
+
+    import torch
+    jobs = []
+    for i, (scale, factor) in enumerate([(12, 16), (15, 13), (13, 2), (14, 15)]):
+        src, dst = graphs.rmat_pairs(scale, factor, 0x9001 + i)[:2]
+        jobs.append((dev.to_dev_u32(src), dev.to_dev_u32(dst), 1 << scale))
+
+    def work(job):
+        s, d, n = job
+        g = dev.DeviceGraph(s, d, n)
+        plan = dev.PageRankPlan(g, persistent=4)
+        ex = dev.PageRankExec(plan, dev.pr_op(0.15, 0.85), 1.0, 3)
+        ex.launch()
+        ranks = ex.ranks().cpu().numpy().tobytes()
+        sh = dev.Shards(s, d, n - 1, 3)
+        adj = [sh.encode(p)[0] for p in range(len(sh.ends))]
+        return [ranks] + [bytes(a) for a in adj]
+
+    want = [work(j) for j in jobs]
+    torch.cuda.synchronize()
+    got, errors = [[None] * 6 for _ in jobs], []
+
+    def run(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for i in range(6):
+                    got[k][i] = work(jobs[(k + i) % len(jobs)])
+        except Exception as exc:  # noqa: BLE001
+            errors.append(exc)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for k in range(len(jobs)):
+        for i in range(6):
+            assert got[k][i] == want[(k + i) % len(jobs)], (k, i)
