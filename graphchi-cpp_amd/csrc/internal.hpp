@@ -33,14 +33,11 @@ int tc_scratch_setup(int dev);
 // Waits for s, then maps a status word to GCHI_ERR_TIMEOUT / GCHI_ERR_INVALID.
 int read_work_status(const uint32_t *err, hipStream_t s);
 
-// Device memory from the library's pool (runtime.hip): scratch of one call, and
-// the memory of plans and shards.  s is the stream that will use it first (an
-// error while it captures).  pool_free takes the result of the wait for the one
-// stream that used the memory; pool_free_device, for a handle's memory, waits for
-// its device (a handle does not know which streams have used it).
+// Scratch of one call from the library's pool of device memory (runtime.hip).  s is
+// the one stream that uses it (an error while it captures); pool_free takes the
+// result of the wait for that stream.
 hipError_t pool_alloc(void **p, size_t bytes, hipStream_t s);
 void pool_free(void *p, hipError_t waited);
-void pool_free_device(void *p);
 
 unsigned grid_for(uint64_t n, unsigned threads, unsigned cap);
 // Over keys sorted on a field f = (key >> shift) & mask: cnt[f] = the number of

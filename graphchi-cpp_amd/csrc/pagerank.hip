@@ -1322,7 +1322,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
         GCHI_LAUNCH_CHECK();
     } else {
         // per-graph CSCs: offsets and out-degrees copied side by side, ids offset by vbase
-        GCHI_HIP(pool_alloc(reinterpret_cast<void **>(&p->own_outdeg), (size_t)std::max<uint32_t>(N, 1) * 4, s));
+        GCHI_HIP(hipMalloc(&p->own_outdeg, (size_t)std::max<uint32_t>(N, 1) * 4));
         p->outdeg = p->own_outdeg;
         std::vector<uint64_t> h_src(G);
         for (uint32_t k = 0; k < G; k++) {
@@ -1437,7 +1437,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint64_t>(G);
-    GCHI_HIP(pool_alloc(&p->mem, zz.off, s));
+    GCHI_HIP(hipMalloc(&p->mem, zz.off));
     Carver c(p->mem, zz.off);
     p->reg_off = c.take<uint32_t>((size_t)N + G);
     p->reg_src = c.take<uint32_t>(std::max<uint64_t>(p->e_reg, 1));
@@ -1605,8 +1605,8 @@ static int plan_create(const PlanInput &in, const gchi_pr_tune *tune, gchi_pr_pl
         }
     }
     if (st != GCHI_OK) {
-        pool_free_device(p->mem);
-        pool_free_device(p->own_outdeg);
+        if (p->mem) (void)hipFree(p->mem);
+        if (p->own_outdeg) (void)hipFree(p->own_outdeg);
         delete p;
         return st;
     }
@@ -1763,8 +1763,8 @@ extern "C" int gchi_pr_plan_create_batch(const gchi_dgraph *graphs, uint32_t ngr
 extern "C" int gchi_pr_plan_destroy(gchi_pr_plan *p) {
     if (!p) return GCHI_OK;
     seg_plan_destroy(p->seg);
-    pool_free_device(p->mem);
-    pool_free_device(p->own_outdeg);
+    if (p->mem) (void)hipFree(p->mem);
+    if (p->own_outdeg) (void)hipFree(p->own_outdeg);
     delete p;
     return GCHI_OK;
 }

@@ -774,7 +774,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     p->N = N;
     p->E = E;
     auto fail_free = [&](int st) {
-        pool_free(p->mem, hipStreamSynchronize(s));
+        if (p->mem) (void)hipFree(p->mem);
         delete p;
         return st;
     };
@@ -837,7 +837,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     z.take<float>((size_t)N + 1);        // xs[1]
     z.take<float>(N);                    // rs[0]
     z.take<float>(N);                    // rs[1]
-    if (pool_alloc(&p->mem, z.off, s) != hipSuccess) {
+    if (hipMalloc(&p->mem, z.off) != hipSuccess) {
         p->mem = nullptr;
         return fail_free(fail(GCHI_ERR_HIP, "pr_plan (form 4): hipMalloc failed (" + std::to_string(z.off) +
                                                 " bytes)"));
@@ -900,7 +900,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
 
 void seg_plan_destroy(gchi_seg_plan *p) {
     if (!p) return;
-    pool_free_device(p->mem);
+    if (p->mem) (void)hipFree(p->mem);
     delete p;
 }
 

@@ -34,8 +34,10 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line) {
 // at R-MAT scale 21.  Freed blocks are kept for the next call, up to kPoolKeep
 // bytes over all devices (the longest kept go back first) and until an allocation
 // fails (then all go back).  A block enters the pool only once no stream uses it,
-// so it can be handed to any thread and stream.  (The runtime's own stream-ordered
-// pool took 25 us per allocation, 40 per free and 450 per hipFree of its memory.)
+// so it can be handed to any thread and stream; the memory of a handle, which does
+// not know the streams that use it, is hipMalloc'ed and hipFree'd (a wait for the
+// whole device would end the captures of other threads).  The runtime's own
+// stream-ordered pool took 25 us per allocation and 40 per free.
 constexpr size_t kPoolKeep = (size_t)1 << 30;
 namespace {
 struct PoolBlock {
@@ -49,7 +51,7 @@ struct Pool {
     std::unordered_map<void *, PoolBlock> out;     // handed out
     size_t bytes = 0;                              // of the kept blocks
 };
-// never destroyed: handles may outlive the library's static objects
+// never destroyed: a call may come after the library's static objects are gone
 Pool &pool() {
     static Pool *p = new Pool();
     return *p;
@@ -126,23 +128,6 @@ void pool_free(void *p, hipError_t waited) {
         }
     }
     for (const PoolBlock &b : back) (void)hipFree(b.p);
-}
-
-void pool_free_device(void *p) {
-    if (!p) return;
-    int cur = 0, dev = 0;
-    {
-        Pool &g = pool();
-        std::lock_guard<std::mutex> lock(g.mu);
-        auto it = g.out.find(p);
-        if (it == g.out.end()) return;
-        dev = it->second.dev;
-    }
-    hipError_t e = hipGetDevice(&cur);
-    if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (cur != dev) (void)hipSetDevice(cur);
-    pool_free(p, e);
 }
 
 // ------------------------------------------------------------------ fills

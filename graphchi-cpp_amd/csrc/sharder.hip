@@ -305,7 +305,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     zz.take<uint32_t>(E + 1);
     zz.take<uint32_t>(E + 1);
     zz.take<int32_t>(2 * (size_t)N);
-    if (pool_alloc(&sh->mem, zz.off, s) != hipSuccess) {
+    if (hipMalloc(&sh->mem, zz.off) != hipSuccess) {
         delete sh;
         return fail(GCHI_ERR_HIP, "shard_build: hipMalloc failed");
     }
@@ -330,7 +330,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     z.take<char>(swb);
     void *scratch = nullptr;
     if (pool_alloc(&scratch, z.off, s) != hipSuccess) {
-        pool_free(sh->mem, hipSuccess);
+        (void)hipFree(sh->mem);
         delete sh;
         return fail(GCHI_ERR_HIP, "shard_build: hipMalloc failed");
     }
@@ -349,7 +349,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
         const hipError_t waited = hipStreamSynchronize(s);
         pool_free(scratch, waited);
         if (st != GCHI_OK) {
-            pool_free(sh->mem, waited);
+            (void)hipFree(sh->mem);
             delete sh;
         } else {
             *out = sh;
@@ -427,7 +427,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
 
 extern "C" int gchi_shard_destroy(gchi_shards *sh) {
     if (!sh) return GCHI_OK;
-    pool_free_device(sh->mem);
+    if (sh->mem) (void)hipFree(sh->mem);
     delete sh;
     return GCHI_OK;
 }
