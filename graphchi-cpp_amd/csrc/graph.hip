@@ -27,18 +27,17 @@ unsigned grid_for(uint64_t n, unsigned threads, unsigned cap) {
 
 // One pass over the keys: run_start[f] = index of the first key of the run of
 // field f, run_end[f] = one past its last key, each by the one thread that sees
-// the field change; low_out, when given, receives key & low_mask.  It is bound
-// by the read of the keys, so a thread has kRunKeys of them in flight: a pass
-// for the starts and one for the lengths, a key at a time, took 190 us on 33.6M
-// keys; 69.
+// the field change.  It is bound by the read of the keys, so a thread has
+// kRunKeys of them in flight: a pass for the starts and one for the lengths, a
+// key at a time, took 190 us on 33.6M 64-bit keys; 69.
 constexpr int kRunKeys = 8;
-__global__ __launch_bounds__(256) void field_runs(const uint64_t *__restrict__ k, uint64_t n, int shift, uint32_t mask,
+template <typename K>
+__global__ __launch_bounds__(256) void field_runs(const K *__restrict__ k, uint64_t n, int shift, uint32_t mask,
                                                   uint32_t nv, uint32_t *__restrict__ run_start,
-                                                  uint32_t *__restrict__ run_end, uint32_t *__restrict__ low_out,
-                                                  uint32_t low_mask) {
+                                                  uint32_t *__restrict__ run_end) {
     constexpr uint64_t kSpan = 256 * kRunKeys;
     for (uint64_t base = (uint64_t)blockIdx.x * kSpan; base < n; base += (uint64_t)gridDim.x * kSpan) {
-        uint64_t key[kRunKeys], next[kRunKeys];
+        K key[kRunKeys], next[kRunKeys];
 #pragma unroll
         for (int u = 0; u < kRunKeys; u++) {
             const uint64_t i = base + (uint64_t)u * 256 + threadIdx.x;
@@ -50,7 +49,6 @@ __global__ __launch_bounds__(256) void field_runs(const uint64_t *__restrict__ k
             const uint64_t i = base + (uint64_t)u * 256 + threadIdx.x;
             if (i >= n) continue;
             const uint32_t f = (uint32_t)(key[u] >> shift) & mask, g = (uint32_t)(next[u] >> shift) & mask;
-            if (low_out) low_out[i] = (uint32_t)key[u] & low_mask;
             if (i == 0 && f < nv) run_start[f] = 0;
             if (i + 1 == n || f != g) {
                 if (f < nv) run_end[f] = (uint32_t)(i + 1);
@@ -73,28 +71,24 @@ __global__ void field_run_counts(const uint32_t *run_start, const uint32_t *run_
     }
 }
 
-int count_field_runs(const uint64_t *keys, uint64_t n, int shift, uint32_t mask, uint32_t nv, uint32_t *run_start,
-                     uint32_t *cnt, uint32_t *low_out, uint32_t low_mask, hipStream_t s, uint32_t *run_end) {
+template <typename K>
+int count_field_runs(const K *keys, uint64_t n, int shift, uint32_t mask, uint32_t nv, uint32_t *run_start,
+                     uint32_t *cnt, hipStream_t s, uint32_t *run_end) {
     if (n == 0) return GCHI_OK;
     if (run_end) launch_fill_u32(run_end, 0u, nv, s);
     uint32_t *end = run_end ? run_end : cnt;
-    hipLaunchKernelGGL(field_runs, dim3(grid_for(div_up(n, kRunKeys), 256, 65536)), dim3(256), 0, s, keys, n, shift,
-                       mask, nv, run_start, end, low_out, low_mask);
+    hipLaunchKernelGGL(field_runs<K>, dim3(grid_for(div_up(n, kRunKeys), 256, 65536)), dim3(256), 0, s, keys, n,
+                       shift, mask, nv, run_start, end);
     hipLaunchKernelGGL(field_run_counts, dim3(grid_for(nv, 256, 65536)), dim3(256), 0, s, run_start, end, nv, cnt,
                        run_end ? 1 : 0);
     GCHI_LAUNCH_CHECK();
     return GCHI_OK;
 }
 
-__global__ void pack_csc_keys(const uint32_t *src, const uint32_t *dst, uint64_t n, uint32_t nv, int sb,
-                              uint64_t *keys, uint32_t *err) {
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint32_t s = src[i], d = dst[i];
-        if (s >= nv || d >= nv) atomicOr(err, 1u);
-        keys[i] = ((uint64_t)d << sb) | (uint64_t)s;
-    }
-}
+template int count_field_runs<uint32_t>(const uint32_t *, uint64_t, int, uint32_t, uint32_t, uint32_t *, uint32_t *,
+                                        hipStream_t, uint32_t *);
+template int count_field_runs<uint64_t>(const uint64_t *, uint64_t, int, uint32_t, uint32_t, uint32_t *, uint32_t *,
+                                        hipStream_t, uint32_t *);
 
 struct CscBits {
     int vb;  // bits of a vertex id
@@ -114,7 +108,7 @@ static void csc_layout(C &c, uint64_t E, uint32_t N, uint64_t **keys, uint32_t *
     *keys = c.template take<uint64_t>(E ? E : 1);
     *indeg = c.template take<uint32_t>(N ? N : 1);
     *run_start = c.template take<uint32_t>(N ? N : 1);
-    size_t ss = std::max(sort_workspace_bytes(E, std::max(cb.sb, cb.vb), false), scan_workspace((size_t)N + 1));
+    size_t ss = std::max(sort_workspace_bytes(E, cb.sb + cb.vb, false), scan_workspace((size_t)N + 1));
     *sw = c.template take<char>(ss);
     *sw_bytes = ss;
 }
@@ -137,18 +131,22 @@ int csc_build(const uint32_t *src, const uint32_t *dst, uint64_t E, uint32_t N, 
     if (outdeg) launch_fill_u32(outdeg, 0u, N, s);
     launch_fill_u32(ind, 0u, N, s);
     if (E) {
-        const unsigned g = grid_for(E, 256, 65536);
-        hipLaunchKernelGGL(pack_csc_keys, dim3(g), dim3(256), 0, s, src, dst, E, N, cb.sb, keys, err);
-        GCHI_LAUNCH_CHECK();
+        PairIO io;
+        io.lo_in = src;
+        io.hi_in = dst;
+        io.lo_out = in_src;
+        io.id_bits = cb.sb;
+        io.limit = N;
+        io.lo_mask = vmask;
         // src passes: keys ordered by src; out-degrees from its runs
-        uint64_t *by_src = nullptr, *by_dst = nullptr;
-        GCHI_TRY(radix_sort_u64_bits(keys, nullptr, nullptr, E, 0, cb.sb, sw, swb, s, &by_src, err));
-        if (outdeg) GCHI_TRY(count_field_runs(by_src, E, 0, vmask, N, run_start, outdeg, nullptr, 0u, s));
-        // dst passes (stable, so src order within a dst run is kept); the
-        // buffer not holding by_src takes the other half of the ping-pong
-        uint64_t *other = by_src == keys ? nullptr : keys;
-        GCHI_TRY(radix_sort_u64_bits(by_src, other, nullptr, E, cb.sb, cb.sb + cb.vb, sw, swb, s, &by_dst, err));
-        GCHI_TRY(count_field_runs(by_dst, E, cb.sb, vmask, N, run_start, ind, in_src, vmask, s));
+        auto by_src = [&](uint64_t *k) {
+            return outdeg ? count_field_runs(k, E, 0, vmask, N, run_start, outdeg, s) : GCHI_OK;
+        };
+        // dst passes (stable, so src order within a dst run is kept): the last
+        // one stores src to in_src and dst beside it
+        uint64_t *by_dst = nullptr;
+        GCHI_TRY(radix_sort_pairs(io, keys, nullptr, E, 0, cb.sb, cb.sb + cb.vb, sw, swb, s, &by_dst, err, by_src));
+        GCHI_TRY(count_field_runs(reinterpret_cast<const uint32_t *>(by_dst), E, 0, vmask, N, run_start, ind, s));
     }
     GCHI_TRY(exclusive_scan_u32(ind, in_off, N, sw, swb, s));
     return GCHI_OK;

@@ -780,7 +780,8 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     };
     // rank order and the slot counts of the rows
     hipLaunchKernelGGL(seg_order_keys, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, g->outdeg, N, keys);
-    int st = radix_sort_u64(keys, nullptr, N, 64, sw, sb, s, nullptr);
+    // (stable, and the ids ascend: only the degree half needs sorting)
+    int st = radix_sort_u64_bits(keys, nullptr, nullptr, N, 32, 64, sw, sb, s, nullptr, nullptr);
     if (st == GCHI_OK) st = read_work_status(static_cast<const uint32_t *>(sw), s);
     if (st != GCHI_OK) return fail_free(st);
     // perm, outdeg_r live in the plan; rank is temporary

@@ -22,7 +22,6 @@
 namespace gchi {
 
 constexpr int kRsThreads = 256;
-constexpr int kRsWaves = kRsThreads / kWave;
 constexpr int kRsItems = 16;
 constexpr int kRsTile = kRsThreads * kRsItems;  // 4096 keys
 // Key-only passes use 512-thread workgroups (8192-key tiles): half as many
@@ -44,37 +43,34 @@ struct StatusBits {
     static constexpr SW kVal = ((SW)1 << kShift) - 1;
 };
 constexpr uint32_t kSpinLimit = 1u << 26;  // default bound of one look-back wait
-constexpr int kRsLookback = 4;
-constexpr int kRsHistKeys = 8;  // keys per thread in flight in the histogram pass  // predecessor tiles read per look-back round trip
+constexpr int kRsLookback = 4;  // predecessor tiles read per look-back round trip
+constexpr int kRsHistKeys = 8;  // keys per thread in flight in the histogram pass
+// Six digits of 33.6M pairs: a key's digits one by one took 150 us, a digit of the
+// eight keys at a time 114, 512-thread workgroups 110 (1,024 threads: 105, but a
+// skewed digit's atomics then meet more: 180 against 175 us in triangle counting).
+constexpr int kRsHistThreads = 512, kRsHistCopies = 4, kRsHistBlocks = 512;
 
 struct PassDesc {
     int shift[kRsMaxPasses];
     int bits[kRsMaxPasses];
 };
 
-// (src, dst) pairs read as the key (dst << id_bits) | src by a first pass, and
-// written back as pairs by a last pass, so the pair sort needs no separate pack
-// and unpack over HBM.  IO bit 1: the pass (or histogram) reads pairs; bit 2:
-// the pass writes pairs.
-struct PairIO {
-    const uint32_t *src_in, *dst_in;
-    uint32_t *src_out, *dst_out;
-    int id_bits;
-};
+// IO bit 1: the pass (or histogram) reads pairs; bit 2: the pass writes pairs
+// (PairIO, internal.hpp).
 constexpr int kIoPackIn = 1, kIoUnpackOut = 2;
 
 template <int IO>
 GCHI_DEV uint64_t load_key(const uint64_t *kin, const PairIO &io, uint64_t i) {
-    if (IO & kIoPackIn) return ((uint64_t)io.dst_in[i] << io.id_bits) | (uint64_t)io.src_in[i];
+    if (IO & kIoPackIn) return ((uint64_t)io.hi_in[i] << io.id_bits) | (uint64_t)io.lo_in[i];
     return kin[i];
 }
 
 template <int IO>
-__global__ __launch_bounds__(kRsThreads) void rs_histogram(const uint64_t *keys, uint64_t n, int npasses,
-                                                           PassDesc pd, uint32_t *ghist, PairIO io) {
-    __shared__ uint32_t s_h[kRsWaves][kRsMaxPasses][kRsRadix];  // 32 KB
-    const int wave = threadIdx.x / kWave;
-    for (int i = threadIdx.x; i < kRsWaves * kRsMaxPasses * kRsRadix; i += kRsThreads)
+__global__ __launch_bounds__(kRsHistThreads) void rs_histogram(const uint64_t *keys, uint64_t n, int npasses,
+                                                           PassDesc pd, uint32_t *ghist, PairIO io, uint32_t *err) {
+    __shared__ uint32_t s_h[kRsHistCopies][kRsMaxPasses][kRsRadix];  // 32 KB
+    const int wave = threadIdx.x / kWave % kRsHistCopies;
+    for (int i = threadIdx.x; i < kRsHistCopies * kRsMaxPasses * kRsRadix; i += kRsHistThreads)
         (&s_h[0][0][0])[i] = 0;
     __syncthreads();
     // kRsHistKeys keys per thread are loaded before any is counted (one load in
@@ -82,30 +78,41 @@ __global__ __launch_bounds__(kRsThreads) void rs_histogram(const uint64_t *keys,
     // the common digit of the high passes for graph ids, is counted by one
     // ballot per wavefront instead of up to 64 LDS atomics on one word.
     const int lane = threadIdx.x & (kWave - 1);
-    constexpr uint64_t kSpan = (uint64_t)kRsThreads * kRsHistKeys;
+    constexpr uint64_t kSpan = (uint64_t)kRsHistThreads * kRsHistKeys;
+    bool bad = false;
     for (uint64_t base = (uint64_t)blockIdx.x * kSpan; base < n; base += (uint64_t)gridDim.x * kSpan) {
         uint64_t kk[kRsHistKeys];
 #pragma unroll
         for (int u = 0; u < kRsHistKeys; u++) {
-            const uint64_t i = base + (uint64_t)u * kRsThreads + threadIdx.x;
-            kk[u] = i < n ? load_key<IO>(keys, io, i) : 0ull;
-        }
-#pragma unroll
-        for (int u = 0; u < kRsHistKeys; u++) {
-            const bool valid = base + (uint64_t)u * kRsThreads + threadIdx.x < n;
-            for (int p = 0; p < npasses; p++) {
-                const uint32_t d = (uint32_t)(kk[u] >> pd.shift[p]) & ((1u << pd.bits[p]) - 1u);
-                const uint64_t zero = __ballot(valid && d == 0u);
-                if (valid && d != 0u) atomicAdd(&s_h[wave][p][d], 1u);
-                if (lane == 0 && zero) atomicAdd(&s_h[wave][p][0], (uint32_t)__popcll(zero));
+            const uint64_t i = base + (uint64_t)u * kRsHistThreads + threadIdx.x;
+            if (IO & kIoPackIn) {
+                const uint32_t l = i < n ? io.lo_in[i] : 0u, h = i < n ? io.hi_in[i] : 0u;
+                bad |= i < n && max(l, h) >= io.limit;
+                kk[u] = ((uint64_t)h << io.id_bits) | l;
+            } else {
+                kk[u] = i < n ? keys[i] : 0ull;
             }
         }
+        for (int p = 0; p < npasses; p++) {
+            const int shift = pd.shift[p];
+            const uint32_t dmask = (1u << pd.bits[p]) - 1u;
+            uint32_t zeros = 0;
+#pragma unroll
+            for (int u = 0; u < kRsHistKeys; u++) {
+                const bool valid = base + (uint64_t)u * kRsHistThreads + threadIdx.x < n;
+                const uint32_t d = (uint32_t)(kk[u] >> shift) & dmask;
+                zeros += (uint32_t)__popcll(__ballot(valid && d == 0u));
+                if (valid && d != 0u) atomicAdd(&s_h[wave][p][d], 1u);
+            }
+            if (lane == 0 && zeros) atomicAdd(&s_h[wave][p][0], zeros);
+        }
     }
+    if (bad) atomicOr(err, GCHI_WORK_BAD_ID);
     __syncthreads();
-    for (int i = threadIdx.x; i < npasses * kRsRadix; i += kRsThreads) {
+    for (int i = threadIdx.x; i < npasses * kRsRadix; i += kRsHistThreads) {
         int p = i / kRsRadix, d = i % kRsRadix;
         uint32_t c = 0;
-        for (int w = 0; w < kRsWaves; w++) c += s_h[w][p][d];
+        for (int w = 0; w < kRsHistCopies; w++) c += s_h[w][p][d];
         if (c) atomicAdd(&ghist[i], c);
     }
 }
@@ -128,6 +135,49 @@ __global__ void rs_hist_scan(uint32_t *ghist) {
     h[threadIdx.x] = s[threadIdx.x];
 }
 
+// A wavefront's keys and their ranks among its equal digits (wh: its counts so
+// far per digit).  Every instruction here runs once per 64 keys and the loop was a
+// third of a pass: the eight ballots are unrolled whatever the digit's width (its
+// bits above are 0), a lane's bit is spread to a mask once for the ballot and for
+// the comparison with it, and a full tile checks no key's index.  33.6M keys:
+// 202 -> 168 us per pass.
+template <bool kVals, int IO, bool kFull>
+GCHI_DEV void rs_load_rank(const uint64_t *kin, const uint32_t *vin, const PairIO &io, uint64_t wbase, uint64_t n,
+                           int shift, uint32_t dmask, uint32_t *wh, uint64_t (&k)[kRsItems], uint32_t (&v)[kRsItems],
+                           uint32_t (&rank)[kRsItems]) {
+    const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+    for (int i = 0; i < kRsItems; i++) {
+        const uint64_t idx = wbase + (uint64_t)i * kWave + lane;
+        k[i] = kFull || idx < n ? load_key<IO>(kin, io, idx) : 0ull;
+        if (kVals) v[i] = kFull || idx < n ? vin[idx] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kRsItems; i++) {
+        const bool valid = kFull || wbase + (uint64_t)i * kWave + lane < n;
+        const uint32_t d = (uint32_t)(k[i] >> shift) & dmask;
+        uint32_t lo = 0, hi = 0;  // bit l set: lane l's digit differs
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const int32_t m = __builtin_amdgcn_sbfe((int32_t)d, b, 1);
+            const uint64_t bal = __ballot(m < 0);
+            lo |= (uint32_t)bal ^ (uint32_t)m;
+            hi |= (uint32_t)(bal >> 32) ^ (uint32_t)m;
+        }
+        uint64_t peers = ~(((uint64_t)hi << 32) | lo);
+        if (!kFull) peers &= __ballot(valid);
+        const uint32_t below =
+            __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
+        const uint32_t cnt = (uint32_t)__popcll(peers);
+        uint32_t b0 = 0;
+        if (valid) b0 = wh[d];
+        __builtin_amdgcn_wave_barrier();
+        if (valid && below == cnt - 1) wh[d] = b0 + cnt;
+        __builtin_amdgcn_wave_barrier();
+        rank[i] = b0 + below;
+    }
+}
+
 template <bool kVals, int T, int IO, typename SW>
 __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict__ kin,
                                                                const uint32_t *__restrict__ vin,
@@ -141,7 +191,6 @@ __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict
     constexpr int TILE = T * kRsItems;
     static_assert(T >= kRsRadix && T % kRsRadix == 0, "a thread per digit");
     __shared__ uint32_t s_wh[NW][kRsRadix];
-    __shared__ uint32_t s_toff[kRsRadix];
     __shared__ uint32_t s_gb[kRsRadix];
     __shared__ uint64_t s_keys[TILE];
     __shared__ uint32_t s_vals[kVals ? TILE : 1];
@@ -164,32 +213,10 @@ __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict
     uint32_t v[kRsItems];
     uint32_t rank[kRsItems];
     const uint64_t wbase = tbase + (uint64_t)wave * (kRsItems * kWave);
-#pragma unroll
-    for (int i = 0; i < kRsItems; i++) {
-        uint64_t idx = wbase + (uint64_t)i * kWave + lane;
-        k[i] = idx < n ? load_key<IO>(kin, io, idx) : 0ull;
-        if (kVals) v[i] = idx < n ? vin[idx] : 0u;
-    }
-    const uint64_t lt = lanemask_lt();
-#pragma unroll
-    for (int i = 0; i < kRsItems; i++) {
-        uint64_t idx = wbase + (uint64_t)i * kWave + lane;
-        bool valid = idx < n;
-        uint32_t d = (uint32_t)(k[i] >> shift) & dmask;
-        uint64_t peers = __ballot(valid);
-        for (int b = 0; b < nbits; b++) {
-            uint64_t bal = __ballot((d >> b) & 1u);
-            peers &= ((d >> b) & 1u) ? bal : ~bal;
-        }
-        uint32_t below = (uint32_t)__popcll(peers & lt);
-        uint32_t cnt = (uint32_t)__popcll(peers);
-        uint32_t b0 = 0;
-        if (valid) b0 = s_wh[wave][d];
-        __builtin_amdgcn_wave_barrier();
-        if (valid && below == cnt - 1) s_wh[wave][d] = b0 + cnt;
-        __builtin_amdgcn_wave_barrier();
-        rank[i] = b0 + below;
-    }
+    if (tile_n == TILE)
+        rs_load_rank<kVals, IO, true>(kin, vin, io, wbase, n, shift, dmask, s_wh[wave], k, v, rank);
+    else
+        rs_load_rank<kVals, IO, false>(kin, vin, io, wbase, n, shift, dmask, s_wh[wave], k, v, rank);
     __syncthreads();
 
     // per-digit: wave exclusive offsets and tile count (thread tid owns digit tid)
@@ -223,7 +250,8 @@ __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict
         uint32_t wb = 0;
         for (int w = 0; w < wave; w++) wb += s_scan[w];
         const uint32_t toff = wb + incl - tcount;
-        s_toff[tid] = toff;
+#pragma unroll
+        for (int w = 0; w < NW; w++) s_wh[w][tid] += toff;
 
         // decoupled look-back for digit tid, kRsLookback predecessors per round
         // trip: their status words are loaded together, then consumed in order
@@ -278,7 +306,7 @@ __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict
         uint64_t idx = wbase + (uint64_t)i * kWave + lane;
         if (idx < n) {
             uint32_t d = (uint32_t)(k[i] >> shift) & dmask;
-            uint32_t pos = s_toff[d] + s_wh[wave][d] + rank[i];
+            uint32_t pos = s_wh[wave][d] + rank[i];
             s_keys[pos] = k[i];
             if (kVals) s_vals[pos] = v[i];
         }
@@ -297,8 +325,8 @@ __global__ __launch_bounds__(T) void rs_onesweep_pass(const uint64_t *__restrict
             // counted, so their positions can run past n: those are dropped.
             if (g >= n) continue;
             if (IO & kIoUnpackOut) {
-                io.src_out[g] = (uint32_t)(key & ((1ull << io.id_bits) - 1ull));
-                io.dst_out[g] = (uint32_t)(key >> io.id_bits);
+                io.lo_out[g] = (uint32_t)key & io.lo_mask;
+                io.hi_out[g] = (uint32_t)(key >> io.id_bits) & io.hi_mask;
             } else {
                 kout[g] = key;
             }
@@ -386,14 +414,15 @@ static void launch_key_pass(int io_mode, const uint64_t *kin, uint64_t *kout, ui
     }
 }
 
-// The sort itself; with pio, the keys come from pio's (src, dst) input and the
-// result goes to its (src, dst) output (keys and alt are then the two
-// intermediate buffers, and nothing is copied back).  A look-back wait that
+// The sort itself; with pio, the keys come from pio's pairs when it has an input
+// and the result goes to its output when it has one (keys and alt are then the
+// two intermediate buffers, and nothing is copied back).  A look-back wait that
 // exceeds its bound sets GCHI_WORK_TIMEOUT in *err (the workspace's own status
 // word when err is null, cleared here); a caller that passes its own word
 // clears it and reads it back once the stream has run.
 static int sort_impl(uint64_t *keys, uint64_t *alt, uint32_t *vals, uint64_t n, int lo, int hi, void *work,
-                     size_t work_bytes, hipStream_t s, uint64_t **out, const PairIO *pio, uint32_t *err) {
+                     size_t work_bytes, hipStream_t s, uint64_t **out, const PairIO *pio, uint32_t *err,
+                     int mid = 0, const SortHook *at_mid = nullptr) {
     if (out) *out = keys;
     if ((n <= 1 || hi <= lo) && !work) return GCHI_OK;  // nothing to sort and no status word to clear
     GCHI_CHECK(lo >= 0 && hi <= 64, GCHI_ERR_INVALID, "sort: key bits outside [0, 64)");
@@ -411,7 +440,7 @@ static int sort_impl(uint64_t *keys, uint64_t *alt, uint32_t *vals, uint64_t n, 
         err = w.err;
         launch_fill_u32(err, 0u, 1, s);
     }
-    if (n <= 1 || hi <= lo) return GCHI_OK;
+    if (n <= (pio ? 0u : 1u) || hi <= lo) return GCHI_OK;
     const int np = npasses_for(bits);
     const uint64_t ntiles = div_up(n, hv ? kRsTile : kRsTileK);  // <= the laid-out div_up(n, kRsTile)
     PassDesc pd;
@@ -421,13 +450,14 @@ static int sort_impl(uint64_t *keys, uint64_t *alt, uint32_t *vals, uint64_t n, 
     }
     launch_fill_u32(w.ghist, 0u, (size_t)np * kRsRadix, s);
     launch_fill_u32(w.counters, 0u, np, s);
-    unsigned hblocks = (unsigned)std::min<uint64_t>(ntiles, 1024);
+    const unsigned hblocks = (unsigned)std::min<uint64_t>(div_up(n, kRsHistThreads * kRsHistKeys), kRsHistBlocks);
     const PairIO io = pio ? *pio : PairIO{};
-    if (pio)
-        hipLaunchKernelGGL(rs_histogram<kIoPackIn>, dim3(hblocks), dim3(kRsThreads), 0, s, keys, n, np, pd, w.ghist,
-                           io);
+    if (io.lo_in)
+        hipLaunchKernelGGL(rs_histogram<kIoPackIn>, dim3(hblocks), dim3(kRsHistThreads), 0, s, keys, n, np, pd,
+                           w.ghist, io, err);
     else
-        hipLaunchKernelGGL(rs_histogram<0>, dim3(hblocks), dim3(kRsThreads), 0, s, keys, n, np, pd, w.ghist, io);
+        hipLaunchKernelGGL(rs_histogram<0>, dim3(hblocks), dim3(kRsHistThreads), 0, s, keys, n, np, pd, w.ghist, io,
+                           err);
     hipLaunchKernelGGL(rs_hist_scan, dim3(np), dim3(kRsRadix), 0, s, w.ghist);
     GCHI_LAUNCH_CHECK();
     uint64_t *ka = keys, *kb = alt ? alt : w.ktmp;
@@ -439,7 +469,9 @@ static int sort_impl(uint64_t *keys, uint64_t *alt, uint32_t *vals, uint64_t n, 
         const size_t nwords = (size_t)ntiles * kRsRadix;  // this pass's look-back words
         if (narrow) launch_fill_u32(st32, 0u, nwords, s);
         else launch_fill_u64(st, 0ull, nwords, s);
-        const int iom = pio ? (p == 0 ? kIoPackIn : 0) | (p == np - 1 ? kIoUnpackOut : 0) : 0;
+        PairIO io_p = io;
+        if (io.lo_out && !io.hi_out) io_p.hi_out = reinterpret_cast<uint32_t *>(kb);
+        const int iom = (p == 0 && io.lo_in ? kIoPackIn : 0) | (p == np - 1 && io.lo_out ? kIoUnpackOut : 0);
         if (hv && narrow)
             hipLaunchKernelGGL((rs_onesweep_pass<true, kRsThreads, 0, uint32_t>), dim3((unsigned)ntiles),
                                dim3(kRsThreads), 0, s, ka, va, kb, vb, n, pd.shift[p], pd.bits[p],
@@ -452,17 +484,19 @@ static int sort_impl(uint64_t *keys, uint64_t *alt, uint32_t *vals, uint64_t n, 
                                g_force_stall);
         else if (narrow)
             launch_key_pass(iom, ka, kb, n, pd.shift[p], pd.bits[p], w.ghist + p * kRsRadix, st32, w.counters + p,
-                            err, io, ntiles, s);
+                            err, io_p, ntiles, s);
         else
             launch_key_pass(iom, ka, kb, n, pd.shift[p], pd.bits[p], w.ghist + p * kRsRadix, st, w.counters + p, err,
-                            io, ntiles, s);
+                            io_p, ntiles, s);
         GCHI_LAUNCH_CHECK();
         std::swap(ka, kb);
         std::swap(va, vb);
+        if (at_mid && lo + 8 * (p + 1) == mid) GCHI_TRY((*at_mid)(ka));
     }
-    if (pio) return GCHI_OK;
     if (out) {
         *out = ka;
+    } else if (io.lo_out) {
+        return GCHI_OK;
     } else if (ka != keys) {
         unsigned b = (unsigned)std::min<uint64_t>(div_up(n, 256), 65536);
         hipLaunchKernelGGL(copy_u64, dim3(b), dim3(256), 0, s, ka, keys, n);
@@ -482,6 +516,12 @@ int radix_sort_u64(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, voi
                    hipStream_t s, uint32_t *err) {
     GCHI_CHECK(key_bits >= 0 && key_bits <= 64, GCHI_ERR_INVALID, "sort: key_bits outside [0, 64]");
     return radix_sort_u64_bits(keys, nullptr, vals, n, 0, key_bits, work, work_bytes, s, nullptr, err);
+}
+
+int radix_sort_pairs(const PairIO &io, uint64_t *keys, uint64_t *alt, uint64_t n, int lo, int mid, int hi, void *work,
+                     size_t work_bytes, hipStream_t s, uint64_t **out, uint32_t *err, const SortHook &at_mid) {
+    return sort_impl(keys, alt, nullptr, n, lo, hi, work, work_bytes, s, out, &io, err, mid,
+                     at_mid ? &at_mid : nullptr);
 }
 
 int read_work_status(const uint32_t *err, hipStream_t s) {
@@ -539,7 +579,13 @@ extern "C" int gchi_sort_pairs_dst_src(const uint32_t *d_src, const uint32_t *d_
     uint64_t *keys = c.take<uint64_t>(n);
     if (n == 0) return radix_sort_u64(nullptr, nullptr, 0, 0, sw, sw_bytes, s, nullptr);  // clears the status
     GCHI_CHECK(d_src && d_dst && d_src_out && d_dst_out, GCHI_ERR_INVALID, "sort_pairs: null pointer");
-    const PairIO io{d_src, d_dst, d_src_out, d_dst_out, id_bits};
+    PairIO io;
+    io.lo_in = d_src;
+    io.hi_in = d_dst;
+    io.lo_out = d_src_out;
+    io.hi_out = d_dst_out;
+    io.id_bits = id_bits;
+    io.lo_mask = id_bits >= 32 ? 0xffffffffu : (1u << id_bits) - 1u;
     if (n == 1) {  // nothing to sort: the pair is copied
         GCHI_TRY(radix_sort_u64(nullptr, nullptr, 0, 0, sw, sw_bytes, s, nullptr));
         if (d_src_out != d_src) GCHI_HIP(hipMemcpyAsync(d_src_out, d_src, 4, hipMemcpyDeviceToDevice, s));

@@ -106,16 +106,6 @@ __global__ void sh_interval_cut(const uint64_t *P, uint32_t n, uint32_t max_id, 
 
 // (src << db) | dst, db = the id bits rounded up to a whole radix digit, so that
 // the first db/8 sort passes order the edges by dst alone.
-__global__ void sh_pack(const uint32_t *src, const uint32_t *dst, uint64_t e, uint32_t nv, int db, uint64_t *keys,
-                        uint32_t *err) {
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < e; i += stride) {
-        const uint32_t sv = src[i], dv = dst[i];
-        if (sv >= nv || dv >= nv) atomicOr(err, 1u);
-        keys[i] = ((uint64_t)sv << db) | dv;
-    }
-}
-
 // (src << db | dst) -> (shard << 2*idb | src << idb | dst), shard = the first
 // interval whose end is >= dst (the last one for larger ids).
 __global__ void sh_rekey(uint64_t *keys, uint64_t e, int db, int idb, const uint32_t *ends, int ns) {
@@ -134,13 +124,13 @@ __global__ void sh_rekey(uint64_t *keys, uint64_t e, int db, int idb, const uint
     }
 }
 
-__global__ void sh_unpack(const uint64_t *keys, uint64_t e, int idb, uint32_t *src, uint32_t *dst) {
+// (src << db | dst) -> one shard's records
+__global__ void sh_unpack(const uint64_t *keys, uint64_t e, int db, uint32_t idmask, uint32_t *src, uint32_t *dst) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t m = (1ull << idb) - 1ull;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < e; i += stride) {
-        uint64_t k = keys[i];
-        dst[i] = (uint32_t)(k & m);
-        src[i] = (uint32_t)((k >> idb) & m);
+        const uint64_t k = keys[i];
+        dst[i] = (uint32_t)k & idmask;
+        src[i] = (uint32_t)(k >> db) & idmask;
     }
 }
 
@@ -326,7 +316,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     z.take<uint32_t>(1);            // err
     z.take<uint64_t>(E + 1);        // keys
     const int db = (idb + 7) / 8 * 8;
-    size_t swb = std::max(sort_workspace_bytes(E, std::max(db, pb), false), scan_workspace((size_t)N + 1));
+    size_t swb = std::max(sort_workspace_bytes(E, std::max(db + idb, pb), false), scan_workspace((size_t)N + 1));
     z.take<char>(swb);
     void *scratch = nullptr;
     if (pool_alloc(&scratch, z.off, s) != hipSuccess) {
@@ -366,14 +356,14 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     uint64_t *by_src_dst = keys;
     int st = GCHI_OK;
     if (E) {
-        hipLaunchKernelGGL(sh_pack, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, d_src, d_dst, E, N, db, keys, err);
-        uint64_t *by_dst = nullptr;
-        st = radix_sort_u64_bits(keys, nullptr, nullptr, E, 0, db, sw, swb, s, &by_dst, err);
-        if (st == GCHI_OK) st = count_field_runs(by_dst, E, 0, idmask, N, run_start, indeg, nullptr, 0u, s);
-        if (st == GCHI_OK)
-            st = radix_sort_u64_bits(by_dst, by_dst == keys ? nullptr : keys, nullptr, E, db, db + idb, sw, swb, s,
-                                     &by_src_dst, err);
-        if (st == GCHI_OK) st = count_field_runs(by_src_dst, E, db, idmask, N, run_start, outdeg, nullptr, 0u, s);
+        PairIO io;
+        io.lo_in = d_dst;
+        io.hi_in = d_src;
+        io.id_bits = db;
+        io.limit = N;
+        auto by_dst = [&](uint64_t *k) { return count_field_runs(k, E, 0, idmask, N, run_start, indeg, s); };
+        st = radix_sort_pairs(io, keys, nullptr, E, 0, db, db + idb, sw, swb, s, &by_src_dst, err, by_dst);
+        if (st == GCHI_OK) st = count_field_runs(by_src_dst, E, db, idmask, N, run_start, outdeg, s);
     }
     if (st == GCHI_OK) {
         hipLaunchKernelGGL(sh_degrees_interleave, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, indeg, outdeg, N,
@@ -406,15 +396,21 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
         }
     }
     if (st == GCHI_OK && E) {
-        // stable pass on the shard id: (shard, src, dst) order
-        hipLaunchKernelGGL(sh_rekey, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, by_src_dst, E, db, idb, d_ends,
-                           sh->nshards);
-        uint64_t *sorted = nullptr;
-        st = radix_sort_u64_bits(by_src_dst, by_src_dst == keys ? nullptr : keys, nullptr, E, 2 * idb,
-                                 2 * idb + pb, sw, swb, s, &sorted, err);
-        if (st == GCHI_OK)
-            hipLaunchKernelGGL(sh_unpack, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, sorted, E, idb, sh->src,
-                               sh->dst);
+        if (pb == 0) {
+            hipLaunchKernelGGL(sh_unpack, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, by_src_dst, E, db, idmask,
+                               sh->src, sh->dst);
+        } else {
+            // stable pass on the shard id: (shard, src, dst) order
+            hipLaunchKernelGGL(sh_rekey, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, by_src_dst, E, db, idb,
+                               d_ends, sh->nshards);
+            PairIO io;
+            io.lo_out = sh->dst;
+            io.hi_out = sh->src;
+            io.id_bits = idb;
+            io.lo_mask = io.hi_mask = idmask;
+            st = radix_sort_pairs(io, by_src_dst, by_src_dst == keys ? nullptr : keys, E, 2 * idb, 0, 2 * idb + pb, sw,
+                                  swb, s, nullptr, err, {});
+        }
         if (st == GCHI_OK) st = read_work_status(err, s);  // waits for the stream
         hipError_t e = hipStreamSynchronize(s);
         if (st == GCHI_OK && e != hipSuccess) st = hip_fail(e, "shard_build", __FILE__, __LINE__);

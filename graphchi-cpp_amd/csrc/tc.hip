@@ -728,8 +728,8 @@ static void tc_prep_layout(C &c, uint64_t E, uint32_t N, uint32_t **deg, uint64_
 
 // deg[v] += in + out degree of v without self-loops (deg zeroed by the caller),
 // from runs of equal ids: the src passes order the keys by src, the dst passes
-// by dst.  vkeys (N+1 entries) serves as scratch of the runs' ends, ekeys and sw as the
-// sort buffers.
+// by dst.  vkeys (N+1 entries) serves as scratch of the runs' ends, ekeys and sw
+// as the sort buffers.
 static int tc_degree_counts(const uint32_t *src, const uint32_t *dst, uint64_t E, uint32_t N, uint32_t *deg,
                             uint32_t *err, uint64_t *vkeys, uint64_t *ekeys, void *sw, size_t swb, hipStream_t s) {
     if (!E) return GCHI_OK;
@@ -739,12 +739,10 @@ static int tc_degree_counts(const uint32_t *src, const uint32_t *dst, uint64_t E
     uint32_t *run_start = reinterpret_cast<uint32_t *>(vkeys), *run_end = run_start + N;
     hipLaunchKernelGGL(tc_degree_pack, dim3(grid_for(E, 256, 65536)), dim3(256), 0, s, src, dst, E, N, sb, ekeys, err);
     GCHI_LAUNCH_CHECK();
-    uint64_t *by_src = nullptr, *by_dst = nullptr;
-    GCHI_TRY(radix_sort_u64_bits(ekeys, nullptr, nullptr, E, 0, sb, sw, swb, s, &by_src, err));
-    GCHI_TRY(count_field_runs(by_src, E, 0, fmask, N, run_start, deg, nullptr, 0u, s, run_end));
-    GCHI_TRY(radix_sort_u64_bits(by_src, by_src == ekeys ? nullptr : ekeys, nullptr, E, sb, sb + fb, sw, swb, s,
-                                 &by_dst, err));
-    return count_field_runs(by_dst, E, sb, fmask, N, run_start, deg, nullptr, 0u, s, run_end);
+    uint64_t *by_dst = nullptr;
+    auto by_src = [&](uint64_t *k) { return count_field_runs(k, E, 0, fmask, N, run_start, deg, s, run_end); };
+    GCHI_TRY(radix_sort_pairs(PairIO{}, ekeys, nullptr, E, 0, sb, sb + fb, sw, swb, s, &by_dst, err, by_src));
+    return count_field_runs(by_dst, E, sb, fmask, N, run_start, deg, s, run_end);
 }
 
 }  // namespace gchi
@@ -789,7 +787,7 @@ extern "C" int gchi_tc_prepare(const uint32_t *d_src, const uint32_t *d_dst, uin
     GCHI_TRY(tc_degree_counts(d_src, d_dst, E, N, deg, err, vkeys, ekeys, sw, swb, s));
     hipLaunchKernelGGL(tc_degree_keys, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, deg, N, idb, vkeys);
     GCHI_LAUNCH_CHECK();
-    GCHI_TRY(radix_sort_u64(vkeys, nullptr, N, idb + degb, sw, swb, s, err));
+    GCHI_TRY(radix_sort_u64_bits(vkeys, nullptr, nullptr, N, idb, idb + degb, sw, swb, s, nullptr, err));
     hipLaunchKernelGGL(tc_vertexmap, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, vkeys, N, idb, d_vertexmap);
     const uint64_t sentinel = (2 * idb >= 64) ? ~0ull : ((1ull << (2 * idb)) - 1ull);
     uint32_t *lo_count = deg;  // reuse: degrees are no longer needed
@@ -1003,7 +1001,7 @@ extern "C" int gchi_degree_order(const uint32_t *d_src, const uint32_t *d_dst, u
     GCHI_TRY(tc_degree_counts(d_src, d_dst, nedges, N, deg, err, vkeys, ekeys, sw, swb, s));
     hipLaunchKernelGGL(tc_degree_keys, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, deg, N, idb, vkeys);
     GCHI_LAUNCH_CHECK();
-    GCHI_TRY(radix_sort_u64(vkeys, nullptr, N, idb + degb, sw, swb, s, err));
+    GCHI_TRY(radix_sort_u64_bits(vkeys, nullptr, nullptr, N, idb, idb + degb, sw, swb, s, nullptr, err));
     hipLaunchKernelGGL(tc_vertexmap, dim3(grid_for(N, 256, 65536)), dim3(256), 0, s, vkeys, N, idb, d_vertexmap);
     uint32_t h_err = 0;
     GCHI_HIP(hipMemcpyAsync(&h_err, err, 4, hipMemcpyDeviceToHost, s));

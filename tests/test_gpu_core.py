@@ -133,3 +133,31 @@ def test_sort_lookback_timeout_is_reported(dev):
     hs, hd = dev.to_host_u32(s, cnt), dev.to_host_u32(d, cnt)
     o = np.lexsort((hs, hd))
     np.testing.assert_array_equal(dev.to_host_u32(so, cnt), hs[o])
+
+
+@pytest.mark.parametrize("e", [1, 2, 8191, 8192, 8193, 40000])
+@pytest.mark.parametrize("n", [2, 256, 257, 70000])
+def test_csc_build_pairs_sorted_at_tile_and_digit_edges(dev, n, e):
+    """Edge counts around one sort tile, id widths around a digit: the packed
+    sort, the degrees counted half-way and the sources stored by its last pass
+    give the oracle's CSC exactly."""
+    rng = np.random.default_rng(1000 * n + e)
+    src = rng.integers(0, n, e).astype(np.uint32)
+    dst = rng.integers(0, n, e).astype(np.uint32)
+    src[-1] = dst[0] = n - 1
+    g = dev.DeviceGraph(dev.to_dev_u32(src), dev.to_dev_u32(dst), n)
+    in_off, in_src, outdeg, _ = oracle.csc(n, src, dst)
+    np.testing.assert_array_equal(g.in_off.cpu().numpy().view(np.uint32)[:n + 1], in_off)
+    np.testing.assert_array_equal(g.in_src.cpu().numpy().view(np.uint32)[:e], in_src)
+    np.testing.assert_array_equal(g.outdeg.cpu().numpy().view(np.uint32)[:n], outdeg)
+    for shards in (1, 2):  # one shard needs no pass on the shard id
+        sh = dev.Shards(dev.to_dev_u32(src), dev.to_dev_u32(dst), n - 1, shards)
+        lo = 0
+        for p in range(sh.nshards):
+            hi = int(sh.ends[p]) if p + 1 < sh.nshards else n - 1
+            keep = np.flatnonzero((dst >= lo) & (dst <= hi))
+            order = keep[np.lexsort((dst[keep], src[keep]))]
+            hs, hd = sh.edges_host(p)
+            np.testing.assert_array_equal(hs, src[order])
+            np.testing.assert_array_equal(hd, dst[order])
+            lo = hi + 1
