@@ -208,25 +208,42 @@ __global__ void scan_tile_bases(uint64_t *tile_sums, size_t ntiles) {
     if (threadIdx.x == 0) tile_sums[ntiles] = carry;
 }
 
+// A thread scans kScanItems consecutive elements, but memory is read and written
+// side by side, through LDS (a word of padding per thread keeps the lanes on
+// different banks).  Straight from memory, a lane 64 bytes from the next, took
+// 14.4 us for 1.4M elements; 6.3.
 template <typename OutT>
-__global__ void scan_tiles(const uint32_t *in, size_t n, const uint64_t *tile_bases, OutT *out) {
+__global__ __launch_bounds__(kScanThreads) void scan_tiles(const uint32_t *in, size_t n, const uint64_t *tile_bases,
+                                                           OutT *out) {
     __shared__ uint64_t s_tmp[kScanThreads / kWave];
-    size_t base = (size_t)blockIdx.x * kScanTile + (size_t)threadIdx.x * kScanItems;
+    __shared__ OutT s_v[kScanTile + kScanThreads];
+    const size_t base = (size_t)blockIdx.x * kScanTile;
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        const int at = i * kScanThreads + threadIdx.x;
+        s_v[at + at / kScanItems] = base + at < n ? in[base + at] : 0u;
+    }
+    __syncthreads();
     uint32_t v[kScanItems];
+    OutT *mine = s_v + threadIdx.x * (kScanItems + 1);
     uint64_t acc = 0;
 #pragma unroll
     for (int i = 0; i < kScanItems; i++) {
-        size_t idx = base + i;
-        v[i] = idx < n ? in[idx] : 0u;
+        v[i] = (uint32_t)mine[i];
         acc += v[i];
     }
     uint64_t tot;
     uint64_t run = tile_bases[blockIdx.x] + block_exclusive_scan<uint64_t>(acc, s_tmp, &tot);
 #pragma unroll
     for (int i = 0; i < kScanItems; i++) {
-        size_t idx = base + i;
-        if (idx < n) out[idx] = (OutT)run;
+        mine[i] = (OutT)run;
         run += v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        const int at = i * kScanThreads + threadIdx.x;
+        if (base + at < n) out[base + at] = s_v[at + at / kScanItems];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         size_t ntiles = gridDim.x;

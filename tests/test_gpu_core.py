@@ -136,7 +136,7 @@ def test_sort_lookback_timeout_is_reported(dev):
 
 
 @pytest.mark.parametrize("e", [1, 2, 8191, 8192, 8193, 40000])
-@pytest.mark.parametrize("n", [2, 256, 257, 70000])
+@pytest.mark.parametrize("n", [2, 256, 257, 4096, 4097, 70000])
 def test_csc_build_pairs_sorted_at_tile_and_digit_edges(dev, n, e):
     """Edge counts around one sort tile, id widths around a digit: the packed
     sort, the degrees counted half-way and the sources stored by its last pass
