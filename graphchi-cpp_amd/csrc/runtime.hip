@@ -114,11 +114,11 @@ void pool_free(void *p, hipError_t waited) {
         std::lock_guard<std::mutex> lock(g.mu);
         auto it = g.out.find(p);
         if (it == g.out.end()) return;
-        if (waited == hipSuccess) {
+        if (waited == hipSuccess && it->second.bytes <= kPoolKeep) {
             g.kept.push_back(it->second);
             g.bytes += it->second.bytes;
         } else {
-            back.push_back(it->second);  // may still be in use: hipFree waits, or refuses
+            back.push_back(it->second);  // too large to keep, or still in use: hipFree waits, or refuses
         }
         g.out.erase(it);
         while (g.bytes > kPoolKeep) {
