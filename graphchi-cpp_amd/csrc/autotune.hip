@@ -68,8 +68,8 @@ extern "C" int gchi_autotune_pr(const gchi_dgraph *g, int sweeps_per_candidate, 
     const size_t N = g->nvertices;
     float *buf = nullptr;
     double *st = nullptr;
-    GCHI_HIP(hipMalloc(&buf, 4 * N * sizeof(float)));
-    if (hipMalloc(&st, 2 * sizeof(double)) != hipSuccess) {
+    GCHI_HIP(device_alloc(&buf, 4 * N * sizeof(float)));
+    if (device_alloc(&st, 2 * sizeof(double)) != hipSuccess) {
         (void)hipFree(buf);
         return fail(GCHI_ERR_HIP, "autotune_pr: hipMalloc failed");
     }

@@ -60,6 +60,14 @@ int read_work_status(const uint32_t *err, hipStream_t s);
 // result of the wait for that stream.
 hipError_t pool_alloc(void **p, size_t bytes, hipStream_t s);
 void pool_free(void *p, hipError_t waited);
+// hipMalloc for everything that outlives a call: when it fails for lack of memory,
+// the pool's kept blocks go back first and it is tried again.
+hipError_t device_alloc(void **p, size_t bytes);
+template <typename T>
+hipError_t device_alloc(T **p, size_t bytes) {
+    return device_alloc(reinterpret_cast<void **>(p), bytes);
+}
+size_t pool_trim();  // gives all kept blocks back; their bytes
 
 unsigned grid_for(uint64_t n, unsigned threads, unsigned cap);
 // Over keys sorted on a field f = (key >> shift) & mask: cnt[f] = the number of

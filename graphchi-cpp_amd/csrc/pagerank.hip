@@ -1322,7 +1322,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
         GCHI_LAUNCH_CHECK();
     } else {
         // per-graph CSCs: offsets and out-degrees copied side by side, ids offset by vbase
-        GCHI_HIP(hipMalloc(&p->own_outdeg, (size_t)std::max<uint32_t>(N, 1) * 4));
+        GCHI_HIP(device_alloc(&p->own_outdeg, (size_t)std::max<uint32_t>(N, 1) * 4));
         p->outdeg = p->own_outdeg;
         std::vector<uint64_t> h_src(G);
         for (uint32_t k = 0; k < G; k++) {
@@ -1437,7 +1437,7 @@ static int plan_build(const PlanInput &in, int W, gchi_pr_plan *p, hipStream_t s
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint32_t>(p->nblk + 1);
     zz.take<uint64_t>(G);
-    GCHI_HIP(hipMalloc(&p->mem, zz.off));
+    GCHI_HIP(device_alloc(&p->mem, zz.off));
     Carver c(p->mem, zz.off);
     p->reg_off = c.take<uint32_t>((size_t)N + G);
     p->reg_src = c.take<uint32_t>(std::max<uint64_t>(p->e_reg, 1));
@@ -1929,7 +1929,7 @@ extern "C" int gchi_pr_blocked_create(const gchi_dgraph *g, const uint32_t *h_bs
         z.take<uint32_t>((size_t)(h_bstart[j + 1] - h_bstart[j]) + 1);
         z.take<uint32_t>((size_t)(h_bstart[j + 1] - h_bstart[j] + 31) / 32);
     }
-    if (hipMalloc(&b->mem, z.off) != hipSuccess) {
+    if (device_alloc(&b->mem, z.off) != hipSuccess) {
         b->mem = nullptr;
         blocked_free(b);
         return fail(GCHI_ERR_HIP, "pr_blocked_create: hipMalloc failed");

@@ -720,7 +720,7 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
     };
     SizerAdapter za;
     lay(za, [](int, void *) {});
-    if (hipMalloc(&b->mem, za.z.off) != hipSuccess) {
+    if (device_alloc(&b->mem, za.z.off) != hipSuccess) {
         delete b;
         return fail(GCHI_ERR_HIP, "ppr_batch_create: hipMalloc failed (state " + std::to_string(za.z.off) + " bytes)");
     }

@@ -838,7 +838,7 @@ int seg_plan_create(const gchi_dgraph *g, int hot, gchi_seg_plan **out, hipStrea
     z.take<float>((size_t)N + 1);        // xs[1]
     z.take<float>(N);                    // rs[0]
     z.take<float>(N);                    // rs[1]
-    if (hipMalloc(&p->mem, z.off) != hipSuccess) {
+    if (device_alloc(&p->mem, z.off) != hipSuccess) {
         p->mem = nullptr;
         return fail_free(fail(GCHI_ERR_HIP, "pr_plan (form 4): hipMalloc failed (" + std::to_string(z.off) +
                                                 " bytes)"));

@@ -4,11 +4,12 @@
 #include "common.hpp"
 #include "internal.hpp"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <list>
 #include <mutex>
-#include <unordered_map>
-#include <vector>
+#include <new>
 
 namespace gchi {
 
@@ -28,14 +29,16 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line) {
     return GCHI_ERR_HIP;
 }
 
-// ------------------------------------------------------------------ memory pool
+// ------------------------------------------------------------------ device memory
 // hipMalloc and hipFree cost about 50 and 110-190 us each here, and a plan or
 // shard build makes a dozen of both: 2.2 of 6.5 ms of an edge list's way to ranks
-// at R-MAT scale 21.  Freed blocks are kept for the next call, up to kPoolKeep
-// bytes over all devices (the longest kept go back first) and until an allocation
-// fails (then all go back).  A block enters the pool only once no stream uses it,
-// so it can be handed to any thread and stream; the memory of a handle, which does
-// not know the streams that use it, is hipMalloc'ed and hipFree'd (a wait for the
+// at R-MAT scale 21.  Freed scratch blocks are kept for the next call, up to
+// kPoolKeep bytes over all devices (the longest kept go back first), and all go
+// back when an allocation of the library fails (scratch, a handle's memory or
+// gchi_malloc, which then try again) and in gchi_pool_trim, for callers that
+// allocate elsewhere.  A block enters the pool only once no stream uses it, so it
+// can be handed to any thread and stream; the memory of a handle, which does not
+// know the streams that use it, is hipMalloc'ed and hipFree'd (a wait for the
 // whole device would end the captures of other threads).  The runtime's own
 // stream-ordered pool took 25 us per allocation and 40 per free.
 constexpr size_t kPoolKeep = (size_t)1 << 30;
@@ -45,18 +48,52 @@ struct PoolBlock {
     size_t bytes;
     int dev;
 };
+typedef std::list<PoolBlock> Blocks;  // spliced from one list to another: only a new block allocates a node
 struct Pool {
     std::mutex mu;
-    std::vector<PoolBlock> kept;                   // oldest first
-    std::unordered_map<void *, PoolBlock> out;     // handed out
-    size_t bytes = 0;                              // of the kept blocks
+    Blocks kept;       // oldest first
+    Blocks out;        // handed out
+    size_t bytes = 0;  // of the kept blocks
 };
 // never destroyed: a call may come after the library's static objects are gone
 Pool &pool() {
-    static Pool *p = new Pool();
+    alignas(Pool) static char mem[sizeof(Pool)];
+    static Pool *p = new (mem) Pool();
     return *p;
 }
+
+size_t give_back(const Blocks &blocks) {
+    size_t bytes = 0;
+    for (const PoolBlock &b : blocks)
+        if (hipFree(b.p) == hipSuccess) bytes += b.bytes;
+    return bytes;
+}
 }  // namespace
+
+size_t pool_trim() {
+    Pool &g = pool();
+    Blocks back;
+    {
+        std::lock_guard<std::mutex> lock(g.mu);
+        back.splice(back.end(), g.kept);
+        g.bytes = 0;
+    }
+    return give_back(back);
+}
+
+hipError_t device_alloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        (void)pool_trim();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here: the next launch check must not find it
+        *p = nullptr;
+    }
+    return e;
+}
 
 hipError_t pool_alloc(void **p, size_t bytes, hipStream_t s) {
     // a build inside a capture stays an error: its kernels would be replayed on
@@ -70,64 +107,51 @@ hipError_t pool_alloc(void **p, size_t bytes, hipStream_t s) {
     {
         // the smallest kept block that fits and is at most a quarter larger
         std::lock_guard<std::mutex> lock(g.mu);
-        size_t best = g.kept.size();
-        for (size_t i = 0; i < g.kept.size(); i++) {
-            const PoolBlock &b = g.kept[i];
-            if (b.dev == dev && b.bytes >= bytes && b.bytes <= bytes + bytes / 4 + 65536 &&
-                (best == g.kept.size() || b.bytes < g.kept[best].bytes))
-                best = i;
-        }
-        if (best < g.kept.size()) {
-            const PoolBlock b = g.kept[best];
-            g.out.emplace(b.p, b);
-            g.kept.erase(g.kept.begin() + best);
-            g.bytes -= b.bytes;
-            *p = b.p;
+        auto best = g.kept.end();
+        for (auto b = g.kept.begin(); b != g.kept.end(); ++b)
+            if (b->dev == dev && b->bytes >= bytes && b->bytes <= bytes + bytes / 4 + 65536 &&
+                (best == g.kept.end() || b->bytes < best->bytes))
+                best = b;
+        if (best != g.kept.end()) {
+            g.bytes -= best->bytes;
+            *p = best->p;
+            g.out.splice(g.out.end(), g.kept, best);
             return hipSuccess;
         }
     }
-    void *q = nullptr;
-    hipError_t e = hipMalloc(&q, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        std::vector<PoolBlock> back;
-        {
-            std::lock_guard<std::mutex> lock(g.mu);
-            back.swap(g.kept);
-            g.bytes = 0;
-        }
-        for (const PoolBlock &b : back) (void)hipFree(b.p);
-        e = hipMalloc(&q, bytes);
+    Blocks fresh;
+    try {
+        fresh.push_back(PoolBlock{nullptr, bytes, dev});
+    } catch (const std::bad_alloc &) {
+        return hipErrorOutOfMemory;
     }
-    if (e != hipSuccess) return e;
+    if (hipError_t e = device_alloc(&fresh.front().p, bytes)) return e;
+    *p = fresh.front().p;
     std::lock_guard<std::mutex> lock(g.mu);
-    g.out.emplace(q, PoolBlock{q, bytes, dev});
-    *p = q;
+    g.out.splice(g.out.end(), fresh);
     return hipSuccess;
 }
 
 void pool_free(void *p, hipError_t waited) {
     if (!p) return;
     Pool &g = pool();
-    std::vector<PoolBlock> back;
+    Blocks back;
     {
         std::lock_guard<std::mutex> lock(g.mu);
-        auto it = g.out.find(p);
+        auto it = std::find_if(g.out.begin(), g.out.end(), [&](const PoolBlock &b) { return b.p == p; });
         if (it == g.out.end()) return;
-        if (waited == hipSuccess && it->second.bytes <= kPoolKeep) {
-            g.kept.push_back(it->second);
-            g.bytes += it->second.bytes;
+        if (waited == hipSuccess && it->bytes <= kPoolKeep) {
+            g.bytes += it->bytes;
+            g.kept.splice(g.kept.end(), g.out, it);
         } else {
-            back.push_back(it->second);  // too large to keep, or still in use: hipFree waits, or refuses
+            back.splice(back.end(), g.out, it);  // too large to keep, or still in use: hipFree waits, or refuses
         }
-        g.out.erase(it);
         while (g.bytes > kPoolKeep) {
-            back.push_back(g.kept.front());
             g.bytes -= g.kept.front().bytes;
-            g.kept.erase(g.kept.begin());
+            back.splice(back.end(), g.kept, g.kept.begin());
         }
     }
-    for (const PoolBlock &b : back) (void)hipFree(b.p);
+    give_back(back);
 }
 
 // ------------------------------------------------------------------ fills
@@ -349,7 +373,13 @@ extern "C" int gchi_memcpy(void *dst, const void *src, size_t bytes, void *strea
 extern "C" int gchi_malloc(void **d_ptr, size_t bytes) {
     GCHI_CHECK(d_ptr, GCHI_ERR_INVALID, "malloc: null pointer");
     *d_ptr = nullptr;
-    GCHI_HIP(hipMalloc(d_ptr, bytes ? bytes : 1));
+    GCHI_HIP(device_alloc(d_ptr, bytes ? bytes : 1));
+    return GCHI_OK;
+}
+
+extern "C" int gchi_pool_trim(size_t *h_bytes) {
+    const size_t bytes = pool_trim();
+    if (h_bytes) *h_bytes = bytes;
     return GCHI_OK;
 }
 

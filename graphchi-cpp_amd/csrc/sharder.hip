@@ -295,7 +295,7 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     zz.take<uint32_t>(E + 1);
     zz.take<uint32_t>(E + 1);
     zz.take<int32_t>(2 * (size_t)N);
-    if (hipMalloc(&sh->mem, zz.off) != hipSuccess) {
+    if (device_alloc(&sh->mem, zz.off) != hipSuccess) {
         delete sh;
         return fail(GCHI_ERR_HIP, "shard_build: hipMalloc failed");
     }

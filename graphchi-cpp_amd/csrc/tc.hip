@@ -1018,7 +1018,7 @@ extern "C" int gchi_relabel_edges(const uint32_t *d_src, const uint32_t *d_dst, 
     if (!nedges) return GCHI_OK;
     hipStream_t s = as_stream(stream);
     uint32_t *err = nullptr;
-    GCHI_HIP(hipMalloc(&err, 4));
+    GCHI_HIP(device_alloc(&err, 4));
     launch_fill_u32(err, 0u, 1, s);
     hipLaunchKernelGGL(relabel_kernel, dim3(grid_for(nedges, 256, 65536)), dim3(256), 0, s, d_src, d_dst, nedges,
                        nvertices, d_map, d_src_out, d_dst_out, err);

@@ -67,6 +67,7 @@ _SIGS = {
     "gchi_last_error": (c_i32, [ctypes.c_char_p, c_sz]),
     "gchi_device_open": (c_i32, [c_i32]),
     "gchi_device_info": (c_i32, [ctypes.POINTER(c_i32), ctypes.c_char_p, c_sz]),
+    "gchi_pool_trim": (c_i32, [ctypes.POINTER(c_sz)]),
     "gchi_memcpy": (c_i32, [c_vp, c_vp, c_sz, c_vp]),
     "gchi_rmat_generate": (c_i32, [c_vp, c_vp, c_u64, c_u64, c_i32, c_u64, ctypes.POINTER(ctypes.c_double), c_vp]),
     "gchi_rmat_generate_host": (c_i32, [c_vp, c_vp, c_u64, c_u64, c_i32, c_u64, ctypes.POINTER(ctypes.c_double), c_i32]),
@@ -198,14 +199,31 @@ def stream():
     return c_vp(torch.cuda.current_stream().cuda_stream)
 
 
-def empty_u32(n):
+def pool_trim():
+    """Gives the library's kept scratch memory back to the device; its bytes."""
+    n = c_sz()
+    check(lib().gchi_pool_trim(ctypes.byref(n)), "pool_trim")
+    return n.value
+
+
+def _empty(n, dtype):
+    """torch.empty on the GPU; out of memory, the library's kept scratch goes
+    back first."""
     torch = _torch()
-    return torch.empty(max(int(n), 1), dtype=torch.int32, device="cuda")
+    try:
+        return torch.empty(n, dtype=dtype, device="cuda")
+    except torch.cuda.OutOfMemoryError:
+        if not pool_trim():
+            raise
+    return torch.empty(n, dtype=dtype, device="cuda")
+
+
+def empty_u32(n):
+    return _empty(max(int(n), 1), _torch().int32)
 
 
 def workspace(nbytes):
-    torch = _torch()
-    return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device="cuda")
+    return _empty(max(int(nbytes), 256), _torch().uint8)
 
 
 def to_host_u32(t, n=None):
@@ -444,8 +462,8 @@ class PageRankExec:
         torch = _torch()
         N = plan.graph.N if plan.graph is not None else plan.N
         self.plan, self.nsweeps = plan, nsweeps
-        self.x = x if x is not None else [torch.empty(N, dtype=torch.float32, device="cuda") for _ in range(2)]
-        self.r = r if r is not None else [torch.empty(N, dtype=torch.float32, device="cuda") for _ in range(2)]
+        self.x = x if x is not None else [_empty(N, torch.float32) for _ in range(2)]
+        self.r = r if r is not None else [_empty(N, torch.float32) for _ in range(2)]
         self.stats = torch.zeros(max(2 * plan.ngraphs * nsweeps, 2), dtype=torch.float64, device="cuda")
         self.op = op
         self.handle = c_vp()
@@ -488,8 +506,8 @@ class PageRankBlocked:
         """init then nsweeps sweeps; returns (ranks, stats[nsweeps, 2])."""
         torch = _torch()
         n = self.graph.N
-        x = torch.empty(n, dtype=torch.float32, device="cuda")
-        r = [torch.empty(n, dtype=torch.float32, device="cuda") for _ in range(2)]
+        x = _empty(n, torch.float32)
+        r = [_empty(n, torch.float32) for _ in range(2)]
         stats = torch.zeros(max(2 * nsweeps, 2), dtype=torch.float64, device="cuda")
         check(lib().gchi_pr_blocked_init(self.handle, init, dptr(seed_bits), seed_value, dptr(x), dptr(r[0]),
                                          stream()), "pr_blocked_init")
@@ -784,8 +802,7 @@ class PprBatch:
         return {k: getattr(res, k) for k, _ in PprResult._fields_}, resid
 
     def ranks(self, q):
-        torch = _torch()
-        out = torch.empty(self.plan.graph.N, dtype=torch.float32, device="cuda")
+        out = _empty(self.plan.graph.N, _torch().float32)
         check(lib().gchi_ppr_batch_extract(self.handle, q, dptr(out), stream()), "ppr_batch_extract")
         return out
 
@@ -809,8 +826,8 @@ class PlainPpr:
         torch = _torch()
         self.plan, self.d = plan, damping
         N = plan.graph.N
-        self.x = [torch.empty(N, dtype=torch.float32, device="cuda") for _ in range(2)]
-        self.r = [torch.empty(N, dtype=torch.float32, device="cuda") for _ in range(2)]
+        self.x = [_empty(N, torch.float32) for _ in range(2)]
+        self.r = [_empty(N, torch.float32) for _ in range(2)]
         self.stats = torch.zeros(2, dtype=torch.float64, device="cuda")
 
     def run(self, seeds, tol=1e-6, max_sweeps=1000, check_every=4):

@@ -56,6 +56,12 @@ int gchi_device_info(int *num_cus, char *arch, size_t arch_len);
 /* Device memory for host-side callers (the engine's RAII buffers). */
 int gchi_malloc(void **d_ptr, size_t bytes);
 int gchi_free(void *d_ptr);
+/* Plan and shard builds keep the scratch memory of a finished call for the next
+ * one, up to 1 GiB per process.  It goes back by itself when an allocation of the
+ * library (gchi_malloc among them) fails; gchi_pool_trim gives it back at once, for
+ * callers whose own allocator needs it.  *h_bytes (may be NULL) = the bytes given
+ * back.  Any thread may call it; it may wait for the device. */
+int gchi_pool_trim(size_t *h_bytes);
 int gchi_synchronize(void *stream);
 /* Pinned (page-locked) host memory for the one-time shard upload: the engines
  * read shard files straight into it, so the upload runs at DMA speed.  Replaces
