@@ -1255,6 +1255,7 @@ struct TmpPool {
     std::vector<void *> ptrs;
     explicit TmpPool(hipStream_t stream) : s(stream) {}
     ~TmpPool() {
+        if (ptrs.empty()) return;  // a wait would end the capture that the allocation refused
         const hipError_t waited = hipStreamSynchronize(s);
         for (void *q : ptrs) pool_free(q, waited);
     }

@@ -732,6 +732,7 @@ struct SegTmp {
     std::vector<void *> ptrs;
     explicit SegTmp(hipStream_t stream) : s(stream) {}
     ~SegTmp() {
+        if (ptrs.empty()) return;  // a wait would end the capture that the allocation refused
         const hipError_t waited = hipStreamSynchronize(s);
         for (void *q : ptrs) pool_free(q, waited);
     }

@@ -1,7 +1,8 @@
 """CPU tests of the library's device memory: the scratch that builds keep between
-calls goes back when memory runs out, on request, and past its bound.  A small
-program stands in for the HIP runtime (its symbols come before libamdhip64's): device memory is host memory
-with a budget, kernels do nothing."""
+calls goes back when memory runs out, on request, and past its bound, and a build
+refused in a capture leaves the capturing stream alone.  A small program stands in
+for the HIP runtime (its symbols come before libamdhip64's): device memory is host
+memory with a budget, kernels do nothing."""
 import os
 import subprocess
 import tempfile
@@ -23,7 +24,7 @@ PROG = r'''
 struct Dim3 { unsigned x, y, z; };
 static std::map<void *, size_t> g_blocks;
 static size_t g_used = 0, g_budget = (size_t)1 << 40;
-static int g_error = 0;
+static int g_error = 0, g_capturing = 0, g_waits = 0;
 
 extern "C" {
 int hipMalloc(void **p, size_t n) {
@@ -49,9 +50,9 @@ int hipDeviceGetAttribute(int *v, int, int) { *v = 256; return 0; }
 int hipGetDevicePropertiesR0600(void *, int) { return 1; }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) { memcpy(d, s, n); return 0; }
-int hipStreamSynchronize(void *) { return 0; }
+int hipStreamSynchronize(void *) { g_waits++; return 0; }
 int hipDeviceSynchronize() { return 0; }
-int hipStreamIsCapturing(void *, int *st) { *st = 0; return 0; }
+int hipStreamIsCapturing(void *, int *st) { *st = g_capturing; return 0; }
 int hipLaunchKernel(const void *, Dim3, Dim3, void **, size_t, void *) { return 0; }
 int __hipPushCallConfiguration(Dim3, Dim3, size_t, void *) { return 0; }
 int __hipPopCallConfiguration(Dim3 *, Dim3 *, size_t *, void **) { return 0; }
@@ -67,6 +68,7 @@ int main(int, char **argv) {
     FN(gchi_free);
     FN(gchi_shard_build);
     FN(gchi_shard_destroy);
+    FN(gchi_pr_plan_create);
     const int what = atoi(argv[2]);
     const uint32_t top = (1u << 20) - 1;  // vertex ids: about 20 bytes each of scratch, 8 of the handle
     gchi_shards *sh = nullptr;
@@ -93,10 +95,27 @@ int main(int, char **argv) {
         CHECK(gchi_shard_build_(nullptr, nullptr, 0, top, 2, &sh, nullptr) == GCHI_OK);
         gchi_shard_destroy_(sh);
         CHECK(g_used == kept);
-    } else {  // past the bound of 1 GiB
+    } else if (what == 3) {  // past the bound of 1 GiB
         CHECK(gchi_shard_build_(nullptr, nullptr, 0, 80 * (top + 1) - 1, 2, &sh, nullptr) == GCHI_OK);
         gchi_shard_destroy_(sh);
         CHECK(g_used <= (size_t)1 << 30);
+    } else {  // refused while the stream captures, with no wait: that would end the capture
+        uint32_t off[2] = {0, 0}, deg[1] = {0};
+        gchi_dgraph g = {};
+        g.nvertices = 1;
+        g.in_off = off;
+        g.in_src = deg;
+        g.outdeg = deg;
+        g_capturing = 1;
+        g_waits = 0;
+        for (int form = 0; form <= 4; form++) {
+            gchi_pr_tune t = {form == 2 ? 256 : 0, 0, form, 0};
+            gchi_pr_plan *plan = nullptr;
+            CHECK(gchi_pr_plan_create_(&g, &t, &plan, nullptr) == GCHI_ERR_HIP);
+        }
+        CHECK(gchi_shard_build_(nullptr, nullptr, 0, top, 2, &sh, nullptr) == GCHI_ERR_HIP);
+        CHECK(g_waits == 0);
+        CHECK(g_used == kept);
     }
     puts("ok");
     return 0;
@@ -115,10 +134,10 @@ def prog():
         yield exe
 
 
-CASES = ["malloc", "handle", "trim", "bound"]
+CASES = ["malloc", "handle", "trim", "bound", "capture"]
 
 
 @pytest.mark.parametrize("what", range(len(CASES)), ids=CASES)
-def test_kept_scratch_goes_back(prog, what):
+def test_scratch_against_stand_in(prog, what):
     run = subprocess.run([prog, gchi.LIB_PATH, str(what)], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr
