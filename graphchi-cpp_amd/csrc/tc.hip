@@ -14,11 +14,14 @@
 //       w in N+(a) n N+(b) for b in N+(a).  One wavefront per vertex a.
 //       w among the 4096 highest ranks (the core; nearly all wedges of a skewed
 //       graph end there): tc_count_core_kernel, rows as bitmaps.
-//       The other w, |N+(a)| <= 512 of them (tc_count_tail_kernel): the
-//       (b, w in N+(b)) pairs of 64 consecutive b are flattened over the 64
-//       lanes, and each w passes a 4096-bit filter of N+(a) in LDS before it is
-//       searched there.  Longer N+(a) (tc_count_kernel): the same pairs, each
-//       lane binary-searching its w in N+(a).
+//       The other w by the length of N+(a) without its core entries.  Up to 512
+//       (tc_count_tail_kernel): the (b, w in N+(b)) pairs of 64 consecutive b are
+//       flattened over the 64 lanes, and each w passes a 4096-bit filter of N+(a)
+//       in LDS before it is searched there.  Up to 1024 (tc_count_hash_kernel):
+//       every w is looked up in an LDS hash table of N+(a).  Longer
+//       (tc_count_kernel): the tail's pairs, each lane binary-searching its w in
+//       N+(a).  gchi_tc_count_noalloc has no core (no scratch for its bitmaps): the
+//       tail kernel takes rows of up to 64 entries there, the hash kernel the rest.
 //       Counts: a, b and w each get +1 per triangle, gathered per wavefront or
 //       workgroup and converted to uint32 with an overflow flag.
 #include <mutex>
@@ -270,8 +273,8 @@ GCHI_DEV void tc_lds_sync() {
 // without tickets (which took 146 of 1105 us per wavefront in the core kernel).
 // Lane l holds the row bounds of the l-th of the next 64 vertices.
 
-// |N+(a)| in [2, kTcTailMax]: N+(a) in LDS with a bit filter of its ids, the
-// pairs of 64 b at a time in flattened order, kTcTailStep pairs per lane in
+// |N+(a)| in [2, max_da]: N+(a) in LDS with a bit filter of its ids, the pairs of
+// 64 b at a time in flattened order, kTcTailStep pairs per lane in
 // flight.  A pair's b comes from marks in LDS at the first pair of every b and a
 // maximum scan.  Bound: vector instructions (about 30 per 64 pairs) and, in
 // sparse graphs, the three dependent loads per vertex (row, b's bounds, w).
@@ -280,6 +283,7 @@ GCHI_DEV void tc_lds_sync() {
 // this one 172 us.
 constexpr int kTcTailWaves = 4;
 constexpr uint32_t kTcTailMax = 512;
+constexpr uint32_t kTcTailMaxWhole = 64;  // without a core (see tc_count_hash_kernel)
 constexpr int kTcTailStep = 4;
 
 GCHI_DEV uint32_t tc_filter(uint32_t x) { return (x ^ (x >> 12)) & 4095u; }
@@ -287,7 +291,8 @@ GCHI_DEV uint32_t tc_filter(uint32_t x) { return (x ^ (x >> 12)) & 4095u; }
 __global__ __launch_bounds__(kTcTailWaves *kWave) void tc_count_tail_kernel(const uint32_t *__restrict__ off,
                                                                             const uint32_t *__restrict__ end,
                                                                             const uint32_t *__restrict__ adj,
-                                                                            uint32_t n, unsigned long long *cnt,
+                                                                            uint32_t n, uint32_t max_da,
+                                                                            unsigned long long *cnt,
                                                                             unsigned long long *total) {
     __shared__ uint32_t s_a[kTcTailWaves][kTcTailMax];    // N+(a), ascending
     __shared__ uint32_t s_c[kTcTailWaves][kTcTailMax];    // credits of its entries
@@ -305,7 +310,7 @@ __global__ __launch_bounds__(kTcTailWaves *kWave) void tc_count_tail_kernel(cons
         const uint64_t mine = i0 + nw * lane;
         const uint32_t va = mine < n ? n - 1 - (uint32_t)mine : 0u;
         const uint32_t vb = mine < n ? off[va] : 0u, ve = mine < n ? end[va] : 0u;
-        uint64_t todo = __ballot(ve - vb >= 2 && ve - vb <= kTcTailMax);
+        uint64_t todo = __ballot(ve - vb >= 2 && ve - vb <= max_da);
         while (todo) {
             const int l = __builtin_ctzll(todo);
             todo &= todo - 1;
@@ -382,6 +387,170 @@ __global__ __launch_bounds__(kTcTailWaves *kWave) void tc_count_tail_kernel(cons
     if (lane == 0 && acc_total) atomicAdd(&s_total, acc_total);
     __syncthreads();
     if (threadIdx.x == 0 && s_total) atomicAdd(total, s_total);
+}
+
+// |N+(a)| in (min_da, kTcHashMax]: one wavefront puts N+(a) into an LDS hash table
+// (open addressing, linear probing, at most half full), then walks b in N+(a) one
+// at a time and looks up every w in N+(b) lane-wide, kTcInflight w per lane in
+// flight.  w's and b's credits go to their slots (16-bit halves of LDS words: at
+// most 2|N+(a)| per slot) and are added to the global counts once per a.
+// Bound: LDS probes, one or two per pair whether it closes a triangle or not; the
+// tail kernel pays about 30 instructions per 64 pairs and a binary search per
+// triangle.  So the line between them (min_da) lies where pairs close.  With the
+// core split off few do, and the tail kernel keeps what it holds (kTcTailMax; R-MAT
+// scale 21 with 14.9M edges: 2.5 ms, 3.0 with the line at 64).  Without a core:
+//   us at line           64      128     256     512
+//   clique of 150       190      280     201     198
+//   clique of 300       389      472     867     757
+//   clique of 600       924    1,011   1,404   3,114
+//   R-MAT scale 17    1,360    1,318   1,289   1,174
+//   R-MAT scale 19    5,741    5,255   5,378   5,707
+//   rows of 90, few  17,300    7,189   6,934   6,896
+// and 64 is the only one that is nowhere far slower than the hash table alone
+// (204, 395, 927, 1,409, 6,169 and 16,452 us).  Searched for every pair from 513
+// entries on, the clique of 600 took 225 ms and R-MAT scale 19 36.8.
+// More workgroups than fit, so that the hardware evens out rows of different
+// lengths (6 / 12 / 24 / 48 per CU: 12.3 / 12.5 / 11.2 / 12.0 ms for 40,000 rows of
+// about 300).
+constexpr int kTcHashWaves = 4;
+constexpr uint32_t kTcHashSlots = 2048;
+constexpr uint32_t kTcHashMax = kTcHashSlots / 2;
+constexpr uint32_t kTcEmpty = 0xffffffffu;
+constexpr unsigned kTcHashGrid = 24;  // workgroups per CU
+constexpr int kTcInflight = 8;  // w loads per lane in flight (one memory round trip per 512 w)
+
+GCHI_DEV uint32_t tc_slot(uint32_t w, int sh) { return (w * 2654435761u) >> sh; }
+
+GCHI_DEV int tc_find(const uint32_t *keys, uint32_t mask, int sh, uint32_t w) {
+    uint32_t h = tc_slot(w, sh);
+    for (;;) {
+        const uint32_t k = keys[h];
+        if (k == w) return (int)h;
+        if (k == kTcEmpty) return -1;
+        h = (h + 1) & mask;
+    }
+}
+
+GCHI_DEV void tc_credit(uint32_t *cw, uint32_t slot, uint32_t c) { atomicAdd(&cw[slot >> 1], c << ((slot & 1) * 16)); }
+
+// Entry `lane` of N+(b_j) (b_j, its start and length in lane j of b/bb/lb), or
+// kTcEmpty past the list; the load is issued at an in-bounds address either way.
+GCHI_DEV uint32_t tc_first_w(const uint32_t *adj, uint32_t bb, uint32_t lb, uint32_t j, int lane) {
+    const uint32_t bbj = (uint32_t)__builtin_amdgcn_readlane((int)bb, (int)j);
+    const uint32_t lbj = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j);
+    const uint32_t v = adj[lbj ? bbj + min((uint32_t)lane, lbj - 1) : 0u];
+    return (uint32_t)lane < lbj ? v : kTcEmpty;
+}
+
+// Triangles (a, b_j, w) for w in N+(b_j): w0 holds the list's first 64
+// entries, the rest are loaded here; each w found in the table is credited,
+// and b_j once with the wavefront's total.  Returns that total.
+GCHI_DEV uint32_t tc_count_b(const uint32_t *adj, const uint32_t *keys, uint32_t *cw, uint32_t mask, int sh,
+                             uint32_t b, uint32_t bb, uint32_t lb, uint32_t j, uint32_t w0, int lane) {
+    const uint32_t bj = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)j);
+    const uint32_t bbj = (uint32_t)__builtin_amdgcn_readlane((int)bb, (int)j);
+    const uint32_t lbj = (uint32_t)__builtin_amdgcn_readlane((int)lb, (int)j);
+    const uint32_t *B = adj + bbj;
+    uint32_t hits = 0;
+    if (w0 != kTcEmpty) {
+        const int h = tc_find(keys, mask, sh, w0);
+        if (h >= 0) {
+            tc_credit(cw, (uint32_t)h, 1u);
+            hits++;
+        }
+    }
+    for (uint32_t t = kWave + lane; t < lbj; t += kTcInflight * kWave) {
+        uint32_t w[kTcInflight];
+#pragma unroll
+        for (int q = 0; q < kTcInflight; q++) {
+            const uint32_t tq = t + q * kWave;
+            w[q] = tq < lbj ? B[tq] : kTcEmpty;
+        }
+#pragma unroll
+        for (int q = 0; q < kTcInflight; q++) {
+            if (w[q] == kTcEmpty) continue;
+            const int h = tc_find(keys, mask, sh, w[q]);
+            if (h >= 0) {
+                tc_credit(cw, (uint32_t)h, 1u);
+                hits++;
+            }
+        }
+    }
+    hits = wave_sum(hits);
+    if (hits && lane == 0) tc_credit(cw, (uint32_t)tc_find(keys, mask, sh, bj), hits);
+    return hits;
+}
+
+__global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(const uint32_t *__restrict__ off,
+                                                                            const uint32_t *__restrict__ end,
+                                                                            const uint32_t *__restrict__ adj,
+                                                                            uint32_t n, uint32_t min_da,
+                                                                            unsigned long long *cnt,
+                                                                            unsigned long long *total) {
+    __shared__ uint32_t sKey[kTcHashWaves][kTcHashSlots];
+    __shared__ uint32_t sCw[kTcHashWaves][kTcHashSlots / 2];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    uint32_t *keys = sKey[wave];
+    uint32_t *cw = sCw[wave];
+    unsigned long long acc_total = 0;
+    const uint64_t nw = (uint64_t)gridDim.x * kTcHashWaves;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * kTcHashWaves + wave; i0 < n; i0 += nw * kWave) {
+        const uint64_t mine = i0 + nw * lane;
+        const uint32_t va = mine < n ? n - 1 - (uint32_t)mine : 0u;
+        const uint32_t vb = mine < n ? off[va] : 0u, ve = mine < n ? end[va] : 0u;
+        uint64_t todo = __ballot(ve - vb > min_da && ve - vb <= kTcHashMax);
+        while (todo) {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)va, l);
+            const uint32_t ab = (uint32_t)__builtin_amdgcn_readlane((int)vb, l);
+            const uint32_t da = (uint32_t)__builtin_amdgcn_readlane((int)ve, l) - ab;
+            const uint32_t want = 4 * da;  // slots: pow2 >= 4 da, at most kTcHashSlots
+            const int lg = min(32 - __clz((int)(want - 1)), 11);
+            const uint32_t S = 1u << lg, mask = S - 1;
+            const int sh = 32 - lg;
+            for (uint32_t k = lane; k < S; k += kWave) keys[k] = kTcEmpty;
+            for (uint32_t k = lane; k < S / 2; k += kWave) cw[k] = 0u;
+            tc_lds_sync();
+            const uint32_t *A = adj + ab;
+            for (uint32_t k = lane; k < da; k += kWave) {
+                const uint32_t x = A[k];
+                uint32_t h = tc_slot(x, sh);
+                while (atomicCAS(&keys[h], kTcEmpty, x) != kTcEmpty) h = (h + 1) & mask;
+            }
+            tc_lds_sync();
+            uint32_t acc_a = 0;
+            // the last element of N+(a) closes no triangle here (no w above it)
+            for (uint32_t bc = 0; bc + 1 < da; bc += kWave) {
+                const uint32_t k = bc + lane;
+                const bool valid = k + 1 < da;
+                const uint32_t b = valid ? A[k] : 0u;
+                const uint32_t bb = valid ? off[b] : 0u;
+                const uint32_t lb = valid ? end[b] - bb : 0u;
+                const uint32_t nb = min((uint32_t)kWave, da - 1 - bc);
+                // The first 64 entries of N+(b_j) are loaded one b ahead (slots w2[0],
+                // w2[1] in turn), so that b_j's probes overlap b_{j+1}'s loads.
+                uint32_t w2[2];
+                w2[0] = tc_first_w(adj, bb, lb, 0, lane);
+                for (uint32_t j0 = 0; j0 < nb; j0 += 2) {  // loads unconditional (clamped j), uses not
+                    w2[1] = tc_first_w(adj, bb, lb, min(j0 + 1, nb - 1), lane);
+                    acc_a += tc_count_b(adj, keys, cw, mask, sh, b, bb, lb, j0, w2[0], lane);
+                    w2[0] = tc_first_w(adj, bb, lb, min(j0 + 2, nb - 1), lane);
+                    if (j0 + 1 < nb) acc_a += tc_count_b(adj, keys, cw, mask, sh, b, bb, lb, j0 + 1, w2[1], lane);
+                }
+            }
+            tc_lds_sync();
+            for (uint32_t k = lane; k < S; k += kWave) {
+                const uint32_t key = keys[k];
+                const uint32_t c = (cw[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+                if (key != kTcEmpty && c) atomicAdd(&cnt[key], (unsigned long long)c);
+            }
+            if (lane == 0 && acc_a) atomicAdd(&cnt[a], (unsigned long long)acc_a);
+            acc_total += acc_a;
+            tc_lds_sync();
+        }
+    }
+    if (lane == 0 && acc_total) atomicAdd(total, acc_total);
 }
 
 // ---- the core: triangles whose highest vertex w is among the kTcCore highest ranks ----
@@ -858,10 +1027,13 @@ static int tc_count_impl(const uint32_t *d_off, const uint32_t *d_adj, uint32_t 
         end = w.end;
     }
     if (!w.rows || n > kTcCore) {
+        const uint32_t tail_max = w.rows ? kTcTailMax : kTcTailMaxWhole;
         hipLaunchKernelGGL(tc_count_tail_kernel, dim3(ncu * 6), dim3(kTcTailWaves * kWave), 0, s, d_off, end, d_adj, n,
-                           w.cnt, w.tot);
+                           tail_max, w.cnt, w.tot);
+        hipLaunchKernelGGL(tc_count_hash_kernel, dim3(grid_for(n, kTcHashWaves, ncu * kTcHashGrid)),
+                           dim3(kTcHashWaves * kWave), 0, s, d_off, end, d_adj, n, tail_max, w.cnt, w.tot);
         hipLaunchKernelGGL(tc_count_kernel, dim3(ncu * 8), dim3(kTcWaves * kWave), 0, s, d_off, end, d_adj, n,
-                           kTcTailMax, w.cnt, w.tot);
+                           kTcHashMax, w.cnt, w.tot);
     }
     hipLaunchKernelGGL(tc_to_u32, dim3(grid_for(n, 256, 65536)), dim3(256), 0, s, w.cnt, n, d_per_vertex, d_overflow);
     GCHI_HIP(hipMemcpyAsync(d_total, w.tot, 8, hipMemcpyDeviceToDevice, s));

@@ -100,3 +100,17 @@ def test_tc_core_and_tail_vs_oracle(dev, n, hubs, p, extra):
                                               dev.dptr(o2), dev.stream()), "tc_count_noalloc")
     assert int(t2.item()) == otot
     np.testing.assert_array_equal(dev.to_host_u32(q, n), opv)
+
+
+def test_tc_rows_long_outside_the_core(dev):
+    """K_5150: 1,054 vertices below the 4,096 of the core, whose rows hold up to
+    1,053 entries outside it, so the tail, hash and search kernels all count
+    beside the core kernel."""
+    n, core = 5150, 4096
+    a, b = np.triu_indices(n, 1)
+    prep, pv, tot, ovf = run_tc(dev, a.astype(np.uint32), b.astype(np.uint32), n)
+    adj, off = dev.to_host_u32(prep.adj, prep.noriented), dev.to_host_u32(prep.off, n + 1).astype(np.int64)
+    outside = np.add.reduceat(adj < n - core, off[:-2])  # the last vertex has no row
+    assert (outside > 1024).any() and ((outside > 512) & (outside <= 1024)).any() and (outside[outside > 0] <= 512).any()
+    assert ovf == 0 and tot == n * (n - 1) * (n - 2) // 6
+    assert (pv == (n - 1) * (n - 2) // 2).all()

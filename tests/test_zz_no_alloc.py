@@ -52,6 +52,39 @@ def test_tc_count_noalloc_equals_workspace_form(dev):
     assert int(tot_n.item()) == int(tot_w.item())
 
 
+@pytest.mark.parametrize("n", [64, 65, 66, 512, 513, 514, 600, 1024, 1025, 1026, 1100])
+def test_tc_count_noalloc_complete_graphs(dev, n):
+    """K_n: rows of every length up to n - 1, around the lines between the tail
+    kernel (up to 64 entries here), the hash kernel (up to 1024) and the search
+    kernel, whose longer rows do not fit its LDS stage."""
+    a, b = np.triu_indices(n, 1)
+    prep = dev.TrianglePrep(dev.to_dev_u32(a.astype(np.uint32)), dev.to_dev_u32(b.astype(np.uint32)), n)
+    rows = np.diff(dev.to_host_u32(prep.off, n + 1).astype(np.int64))
+    assert rows.max() == n - 1
+    pv, tot, ovf = _noalloc(dev, prep, n)
+    assert int(tot.item()) == n * (n - 1) * (n - 2) // 6 and int(ovf.item()) == 0
+    assert (dev.to_host_u32(pv, n) == (n - 1) * (n - 2) // 2).all()
+
+
+def test_tc_count_noalloc_dense_rows_are_not_searched(dev):
+    """36M pairs in rows of up to 599 entries take about a millisecond through the
+    hash kernel; searched one by one they took 225."""
+    import time
+
+    import torch
+    n = 600
+    a, b = np.triu_indices(n, 1)
+    prep = dev.TrianglePrep(dev.to_dev_u32(a.astype(np.uint32)), dev.to_dev_u32(b.astype(np.uint32)), n)
+    best = 1.0
+    for _ in range(3):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        _noalloc(dev, prep, n)
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    assert best < 0.03
+
+
 def test_tc_count_noalloc_refuses_oversize(dev):
     L = dev.lib()
     one = ctypes.c_void_p(1)
