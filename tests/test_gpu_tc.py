@@ -102,6 +102,20 @@ def test_tc_core_and_tail_vs_oracle(dev, n, hubs, p, extra):
     np.testing.assert_array_equal(dev.to_host_u32(q, n), opv)
 
 
+@pytest.mark.parametrize("n", [31, 32, 63, 64, 65, 95, 96, 100, 127, 128])
+def test_tc_workgroups_of_small_graphs(dev, n):
+    """Vertex counts around one, two and three workgroups of the core kernel, whose
+    workspace holds a block of credits for each."""
+    import ctypes
+    a, b = np.triu_indices(n, 1)
+    prep, pv, tot, ovf = run_tc(dev, a.astype(np.uint32), b.astype(np.uint32), n)
+    assert ovf == 0 and tot == n * (n - 1) * (n - 2) // 6
+    assert (pv == (n - 1) * (n - 2) // 2).all()
+    nb = ctypes.c_size_t()
+    dev.check(dev.lib().gchi_tc_count_workspace(n, ctypes.byref(nb)))
+    assert nb.value >= max(1, n // 32) * 65536
+
+
 def test_tc_rows_long_outside_the_core(dev):
     """K_5150: 1,054 vertices below the 4,096 of the core, whose rows hold up to
     1,053 entries outside it, so the tail, hash and search kernels all count
