@@ -74,8 +74,9 @@ struct PpArgs {
 struct gchi_ppr_batch {
     gchi::PpArgs a{};
     uint32_t nq = 0, nqb = 0, N = 0;
-    void *r16[2] = {nullptr, nullptr};  // [nqb][N][64] bf16
-    float *r32[2] = {nullptr, nullptr};  // [nqb][N][64] fp32
+    size_t state = 0;              // values of one state buffer: [N][64] per query block, [N][2^lq] for the last
+    void *r16[2] = {nullptr, nullptr};   // bf16
+    float *r32[2] = {nullptr, nullptr};  // fp32
     double *res = nullptr;         // [nqb*64]
     uint32_t *seedk = nullptr;
     uint32_t *seed_v = nullptr;    // [nqb][64*64] sorted (vertex, query)
@@ -689,7 +690,8 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
     a.S = (uint32_t)std::min<uint64_t>(512, std::max<uint64_t>(1, lanes / slots / 64) * 64);
     a.nitems = (uint32_t)div_up(E, a.S);
     a.kwords = N / 32 + 1;
-    const size_t state = (size_t)nqb * N * kQ, epad = (size_t)E + 2 * a.S + 2 * kWave;
+    const size_t state = ((size_t)(nqb - 1) * kQ + ((size_t)1 << a.lq)) * N, epad = (size_t)E + 2 * a.S + 2 * kWave;
+    b->state = state;
     auto lay = [&](auto &c, auto get) {
         get(0, c.template take<uint32_t>(epad));              // src
         get(1, c.template take<float>(epad));                 // w
@@ -711,22 +713,28 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
         get(17, c.template take<uint16_t>(state));
         get(18, c.template take<float>(state));
         get(19, c.template take<float>(state));
-        // build scratch
-        get(20, c.template take<uint32_t>((size_t)N + 1));    // len
-        get(21, c.template take<uint32_t>((size_t)N + 1));    // some
-        get(22, c.template take<uint32_t>((size_t)N + 1));    // ord
-        get(23, c.template take<uint32_t>((size_t)N + 1));    // start
-        get(24, c.template take<char>(scan_workspace((size_t)N + 1)));
     };
-    SizerAdapter za;
+    auto lay_scratch = [&](auto &c, auto get) {  // of the build
+        for (int k = 0; k < 4; k++) get(k, c.template take<uint32_t>((size_t)N + 1));  // len, some, ord, start
+        get(4, c.template take<char>(scan_workspace((size_t)N + 1)));
+    };
+    SizerAdapter za, zs;
     lay(za, [](int, void *) {});
+    lay_scratch(zs, [](int, void *) {});
     if (device_alloc(&b->mem, za.z.off) != hipSuccess) {
         delete b;
         return fail(GCHI_ERR_HIP, "ppr_batch_create: hipMalloc failed (state " + std::to_string(za.z.off) + " bytes)");
     }
-    void *m[25];
-    Carver c(b->mem, za.z.off);
+    void *scratch = nullptr;
+    if (hipError_t e = pool_alloc(&scratch, zs.z.off, 0)) {
+        (void)hipFree(b->mem);
+        delete b;
+        return hip_fail(e, "ppr_batch_create: scratch", __FILE__, __LINE__);
+    }
+    void *m[20], *t[5];
+    Carver c(b->mem, za.z.off), sc(scratch, zs.z.off);
     lay(c, [&](int k, void *q) { m[k] = q; });
+    lay_scratch(sc, [&](int k, void *q) { t[k] = q; });
     auto u32 = [&](int k) { return static_cast<uint32_t *>(m[k]); };
     float *w = static_cast<float *>(m[1]);
     a.src = u32(0);
@@ -749,7 +757,9 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
     b->r16[1] = m[17];
     b->r32[0] = static_cast<float *>(m[18]);
     b->r32[1] = static_cast<float *>(m[19]);
-    uint32_t *len = u32(20), *some = u32(21), *ord = u32(22), *start = u32(23);
+    uint32_t *tmp[4];
+    for (int k = 0; k < 4; k++) tmp[k] = static_cast<uint32_t *>(t[k]);
+    uint32_t *len = tmp[0], *some = tmp[1], *ord = tmp[2], *start = tmp[3];
     const size_t swb = scan_workspace((size_t)N + 1);
     auto build = [&]() -> int {
         const dim3 gv(grid_for(N, 256, 65536)), blk(256);
@@ -758,8 +768,8 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
         launch_fill_u32(reinterpret_cast<uint32_t *>(w) + E, 0u, epad - E, 0);
         hipLaunchKernelGGL(pb_lengths, gv, blk, 0, 0, pv, len, some);
         if (pv.nhub) hipLaunchKernelGGL(pb_hub_lengths, dim3(grid_for(pv.nhub, 256, 65536)), blk, 0, 0, pv, len, some);
-        GCHI_TRY(exclusive_scan_u32(some, ord, N, m[24], swb, 0));
-        GCHI_TRY(exclusive_scan_u32(len, start, N, m[24], swb, 0));
+        GCHI_TRY(exclusive_scan_u32(some, ord, N, t[4], swb, 0));
+        GCHI_TRY(exclusive_scan_u32(len, start, N, t[4], swb, 0));
         hipLaunchKernelGGL(pb_rows, gv, blk, 0, 0, N, len, ord, start, u32(6), u32(7), u32(5), u32(2));
         hipLaunchKernelGGL(pb_regular, dim3(grid_for((uint64_t)N * 16, 256, 65536)), blk, 0, 0, pv, u32(6), start,
                            u32(0), w);
@@ -775,6 +785,7 @@ extern "C" int gchi_ppr_batch_create(const gchi_pr_plan *plan, uint32_t nqueries
         return GCHI_OK;
     };
     const int st = build();
+    pool_free(scratch, hipStreamSynchronize(0));
     if (st != GCHI_OK) {
         (void)hipFree(b->mem);
         delete b;
@@ -886,9 +897,8 @@ extern "C" int gchi_ppr_batch_run(gchi_ppr_batch *b, const uint32_t *h_seed_off,
             if (m <= cfg->bf16_switch_residual || m > 0.7 * prev) break;
             prev = m;
         }
-        const size_t state = (size_t)nqb * N * kQ;
         hipLaunchKernelGGL(ppr_widen_kernel, dim3(65536), dim3(256), 0, s, (const uint16_t *)b->r16[0], b->r32[0],
-                           state);
+                           b->state);
         b->fp32 = true;
     }
     // FP32 teleport values of the rows without in-edges in both buffers; of all

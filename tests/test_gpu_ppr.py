@@ -149,3 +149,30 @@ def test_batched_ppr_graph_without_edges(dev):
         want = np.zeros(40, np.float32)
         want[[q, q + 5]] = np.float32((1 - D) / 2)
         np.testing.assert_array_equal(b.ranks(q).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("nq,width", [(1, 4), (20, 32), (64, 64), (66, 68)])
+def test_batched_ppr_memory(dev, nq, width):
+    """A batch's device memory: its state is as wide as the queries need, and it
+    keeps the edges but no scratch of its creation.  Per vertex 12 bytes a value of
+    the blocks' width, 12 of tables and some bits; per edge 8 and up to 8 per block
+    for the rows that cross items (items of 64 edges), and allocations of 2 MiB."""
+    import torch
+    n, e = 1 << 19, 1 << 19
+    rng = np.random.default_rng(nq)
+    s, d = rng.integers(0, n, e).astype(np.uint32), rng.integers(0, n, e).astype(np.uint32)
+    plan = dev.PageRankPlan(dev.DeviceGraph(dev.to_dev_u32(s), dev.to_dev_u32(d), n), edges_per_block=2048)
+    torch.cuda.synchronize()
+    dev.pool_trim()
+    before = torch.cuda.mem_get_info()[0]
+    b = dev.PprBatch(plan, nq)
+    dev.pool_trim()
+    used = before - torch.cuda.mem_get_info()[0]
+    blocks = (nq + 63) // 64
+    assert used <= (12 * width + 13) * n + (9 + 8 * blocks) * e + (4 << 20)
+    queries = random_queries(n, nq, nq, 3)
+    info, _ = b.run(queries, D, TOL)
+    assert info["converged"] == 1
+    plain = dev.PlainPpr(plan, D)
+    rp, _ = plain.run(queries[-1], TOL)
+    assert (b.ranks(nq - 1) - rp).abs().sum().item() <= 2 * TOL
