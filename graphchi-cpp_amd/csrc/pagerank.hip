@@ -53,7 +53,6 @@ struct gchi_pr_plan {
     uint32_t nhub = 0;     // hub rows
     uint32_t nchunk = 0;   // hub chunks
     uint32_t nfin = 0;     // finalize workgroups (single-graph plans)
-    uint32_t npersist = 0; // workgroups of form 1 resident at once
     uint64_t e_reg = 0, e_hub = 0;
     const uint32_t *outdeg = nullptr;
     uint32_t *reg_off = nullptr;
@@ -327,11 +326,11 @@ GCHI_DEV void pr_tile(const PrArgs &a, const PrConsts &c, uint32_t tile, float *
 }
 
 // One workgroup per tile (hub chunks first, then regular blocks); the hardware
-// hands them out as earlier ones end.  Resident workgroups that pulled tiles from device counters instead took 668 us a sweep
-// where this launch takes 535 (300 R-MAT graphs of scales 10-17, 153M edges; 699
-// with a static tile list): the ticket and its two barriers stand in front of
-// every tile's chain of loads.
-// (The same kernel with a loop over tiles: 660 us.)
+// hands them out as earlier ones end.  300 R-MAT graphs of scales 10-17, 153M
+// edges: 535 us a sweep.  Resident workgroups that pulled tiles from device
+// counters took 668 (the ticket and its two barriers stand in front of every
+// tile's chain of loads), with a static tile list 699, with this launch and a loop
+// over tiles in the kernel 660.
 constexpr uint32_t kPrMaxGrid = 1u << 23;  // grid x threads stays below 2^32: more tiles take several launches
 
 __global__ __launch_bounds__(kPrThreads) void pr_sweep_kernel(PrArgs a, PrConsts c, uint32_t first) {
@@ -1566,7 +1565,6 @@ static int plan_create(const PlanInput &in, const gchi_pr_tune *tune, gchi_pr_pl
             lds_wg = prop.sharedMemPerBlock;
         }
         const uint32_t nhubt = (p->nchunk + kPrWaves - 1) / kPrWaves;
-        p->npersist = (uint32_t)std::min<uint64_t>((uint64_t)ncu * 8, (uint64_t)p->nblk + nhubt);
         if (p->persistent == 3) {
             // 256-thread workgroups, four per CU: each holds H cached values and
             // its 2W staging floats within a quarter of the CU's LDS
@@ -1783,10 +1781,7 @@ extern "C" int gchi_pr_plan_info_get(const gchi_pr_plan *p, gchi_pr_plan_info *i
     info->hub_edges = p->e_hub;
     info->ngraphs = p->G;
     info->persistent = p->persistent;
-    info->persistent_workgroups = p->persistent == 3   ? p->nhot_wg
-                                  : p->persistent == 2 ? p->nwave_wg
-                                  : p->persistent      ? p->npersist
-                                                       : 0u;
+    info->persistent_workgroups = p->persistent == 3 ? p->nhot_wg : p->persistent == 2 ? p->nwave_wg : 0u;
     info->hot_vertices = p->H;
     info->gather_sources = p->A;
     info->hot_threads = p->persistent == 2 ? (uint32_t)kWaveThreads : p->persistent == 3 ? (uint32_t)kPrThreads : 0u;

@@ -250,7 +250,7 @@ typedef struct gchi_pr_plan_info {
     uint64_t hub_edges;
     uint32_t ngraphs;
     uint32_t persistent;
-    uint32_t persistent_workgroups;
+    uint32_t persistent_workgroups;  /* of the launch forms 2, 3 and 4; 0: a workgroup per tile */
     uint32_t hot_vertices;     /* values cached in LDS per workgroup (0: none) */
     uint32_t gather_sources;   /* vertices in the gather layout (0: no layout) */
     uint32_t hot_threads;      /* workgroup size of the LDS-cached sweep */

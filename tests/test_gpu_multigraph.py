@@ -62,6 +62,16 @@ def test_persistent_single_graph_bitwise(dev):
     np.testing.assert_array_equal(a, b)
 
 
+def test_plan_info_names_the_workgroups_of_persistent_forms_only(dev):
+    """Forms 0 and 1 launch a workgroup per tile: none of them is persistent."""
+    s, d, n = make_graphs(1, 3)[0]
+    g = dev.DeviceGraph(dev.to_dev_u32(s), dev.to_dev_u32(d), n)
+    for form in range(5):
+        info = dev.PageRankPlan(g, persistent=form, edges_per_block=256 if form == 2 else 0).info()
+        assert info["persistent"] == form
+        assert (info["persistent_workgroups"] > 0) == (form >= 2), form
+
+
 def test_union_gather_layout_equals_individual_runs(dev):
     """A multi-graph plan in the gather layout with the LDS cache: every
     graph's ranks are still bit-identical to its solo vertex-id run."""
