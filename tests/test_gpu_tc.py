@@ -38,8 +38,10 @@ def test_tc_duplicates_and_reciprocal_edges(dev):
     assert pv[vm[3]] == 0
 
 
-def test_tc_long_lists_global_search(dev):
-    # K_1100: oriented lists longer than the 1024-entry LDS stage
+def test_tc_lists_of_the_core(dev):
+    # K_1100: oriented lists of up to 1,099 entries, all in the core (lists as long
+    # outside it: test_tc_rows_long_outside_the_core; without a core:
+    # test_tc_count_noalloc_complete_graphs)
     n = 1100
     a, b = np.triu_indices(n, 1)
     prep, pv, tot, ovf = run_tc(dev, a.astype(np.uint32), b.astype(np.uint32), n)
@@ -59,9 +61,9 @@ def test_tc_scale21_vs_oracle(dev):
     np.testing.assert_array_equal(pv, opv)
 
 
-@pytest.mark.parametrize("n", [3, 129, 131, 1500, 4097, 4200])
+@pytest.mark.parametrize("n", [3, 65, 66, 129, 131, 1500, 4097, 4200])
 def test_tc_complete_graphs(dev, n):
-    """K_n around the sizes of the counting kernels: rows of 128 and 129 core
+    """K_n around the sizes of the counting kernels: rows of 64 and 65 core
     entries (list / bitmap), a core smaller than, equal to and larger than the
     4096 highest ranks, more bitmaps per wavefront than its bit planes hold."""
     a, b = np.triu_indices(n, 1)
@@ -128,3 +130,33 @@ def test_tc_rows_long_outside_the_core(dev):
     assert (outside > 1024).any() and ((outside > 512) & (outside <= 1024)).any() and (outside[outside > 0] <= 512).any()
     assert ovf == 0 and tot == n * (n - 1) * (n - 2) // 6
     assert (pv == (n - 1) * (n - 2) // 2).all()
+
+
+def test_tc_long_core_rows_below_the_bitmaps(dev):
+    """40,000 vertices with 70 to 130 edges each into 4,000 hubs and some among
+    themselves: vertices below the 16,384 bitmapped ranks whose rows hold more than
+    64 core entries, walked entry by entry against a's bitmap."""
+    import torch
+    n, hubs, rows, core = 40000, 4000, 16384, 4096
+    rng = np.random.default_rng(40000)
+    low = np.arange(hubs, n)
+    deg = rng.integers(70, 131, len(low))
+    s = [np.repeat(low, deg), rng.integers(hubs, n, 80000)]
+    d = [rng.integers(0, hubs, int(deg.sum())), rng.integers(hubs, n, 80000)]
+    ids = rng.permutation(n)
+    src, dst = graphs.preprocess(ids[np.concatenate(s)], ids[np.concatenate(d)], simple=True)
+    prep, pv, tot, ovf = run_tc(dev, src, dst, n)
+    adj, off = dev.to_host_u32(prep.adj, prep.noriented), dev.to_host_u32(prep.off, n + 1).astype(np.int64)
+    entries = np.concatenate([[0], np.cumsum(adj >= n - core)])
+    long_rows = (entries[off[1:]] - entries[off[:-1]] > 64) & (np.arange(n) < n - rows)
+    assert long_rows[adj].sum() > 10000  # such a row is the b of a pair that often
+    vm, opv, otot = oracle.triangles(n, src, dst)
+    assert tot == otot and ovf == 0
+    np.testing.assert_array_equal(pv, opv)
+    q = dev.empty_u32(n)
+    t2 = torch.zeros(1, dtype=torch.int64, device="cuda")
+    o2 = torch.zeros(1, dtype=torch.int32, device="cuda")
+    dev.check(dev.lib().gchi_tc_count_noalloc(dev.dptr(prep.off), dev.dptr(prep.adj), n, dev.dptr(q), dev.dptr(t2),
+                                              dev.dptr(o2), dev.stream()), "tc_count_noalloc")
+    assert int(t2.item()) == otot
+    np.testing.assert_array_equal(dev.to_host_u32(q, n), opv)
