@@ -1,12 +1,11 @@
 // Autotuner for the PageRank sweep launch shape.
 //
 // Candidates: edges per regular block W (which also sets the hub threshold),
-// the one-lane-per-row threshold, the launch form (one workgroup per tile,
-// or persistent wavefronts), and (N < 2^30) the
-// out-degree gather layout with and without an LDS cache of the most
-// referenced source values, and the rank-space tiled sweep (form 4).  Each
-// candidate gets its own plan on the caller's graph and is
-// timed with HIP events over a few sweeps after a warm-up sweep; the fastest
+// the one-lane-per-row threshold, the launch form (one workgroup per tile, or
+// persistent wavefronts), and (N < 2^30) the out-degree gather layout with and
+// without an LDS cache of the most referenced source values, and the rank-space
+// tiled sweep (form 4).  Each candidate gets its own plan on the caller's graph and
+// is timed with HIP events over a few sweeps after a warm-up sweep; the fastest
 // wins.  Results are cached per (N, E) in the process (a plan depends on the
 // graph, a tune only on its shape and degree distribution).
 #include "common.hpp"

@@ -350,7 +350,8 @@ __global__ void cc_iota(uint32_t *l, uint32_t n) {
 // meets a 0, needs no further look at its neighbours: nothing is lower (vertex
 // 0's component; rows of others are read whole).  Round 0 still checks every
 // neighbour id.  Together with kCcsLanes lanes per short row, 16 flags per thread
-// in the compaction and the lists' own flags (no clearing passes) and two rounds per readback: 3317 -> 1421 us.
+// in the compaction, the lists' own flags (no clearing passes) and two rounds per
+// readback: 3317 -> 1421 us.
 constexpr uint32_t kCcsShort = 64;    // rows up to this length: kCcsLanes lanes each
 constexpr uint32_t kCcsChunk = 4096;  // longer rows: one wavefront per chunk
 constexpr int kCcsLanes = 4;  // 4 / 8 / 16: 445 / 488 / 579 us of short rows per call
@@ -514,7 +515,8 @@ __global__ void ccs_long_min(const uint32_t *__restrict__ off, const uint32_t *_
         const uint32_t lv = label[v];
         uint32_t m = 0xffffffffu;
         bool low = lv == 0;  // wavefront-uniform: the label is or becomes 0, the lowest there is
-        for (uint32_t k0 = b + lane; k0 - lane < e && (first || !low); k0 += 4 * kWave) {  // four gathers in flight per lane
+        // four gathers in flight per lane
+        for (uint32_t k0 = b + lane; k0 - lane < e && (first || !low); k0 += 4 * kWave) {
             uint32_t u[4], l[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) u[q] = adj[min(k0 + q * kWave, e - 1)];

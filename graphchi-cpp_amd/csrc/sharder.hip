@@ -104,8 +104,6 @@ __global__ void sh_interval_cut(const uint64_t *P, uint32_t n, uint32_t max_id, 
     *nshards_out = shardnum;
 }
 
-// (src << db) | dst, db = the id bits rounded up to a whole radix digit, so that
-// the first db/8 sort passes order the edges by dst alone.
 // (src << db | dst) -> (shard << 2*idb | src << idb | dst), shard = the first
 // interval whose end is >= dst (the last one for larger ids).
 __global__ void sh_rekey(uint64_t *keys, uint64_t e, int db, int idb, const uint32_t *ends, int ns) {
@@ -356,6 +354,8 @@ extern "C" int gchi_shard_build(const uint32_t *d_src, const uint32_t *d_dst, ui
     uint64_t *by_src_dst = keys;
     int st = GCHI_OK;
     if (E) {
+        // keys (src << db) | dst, db = the id bits rounded up to a whole radix digit, so
+        // that the first db/8 passes order the edges by dst alone
         PairIO io;
         io.lo_in = d_dst;
         io.hi_in = d_src;

@@ -559,7 +559,7 @@ __global__ __launch_bounds__(kTcHashWaves *kWave) void tc_count_hash_kernel(cons
 // kTcCore bits, 64 per lane: the w of (a, b) are one AND, their number one
 // popcount, and the credits of w vertical counters in registers (bit planes
 // summed with carry-save adders, flushed every 2^kTcPlanes bitmaps).  Bitmaps
-// are kept for the rows with more than kTcList core entries (one per lane: 762 us
+// are kept for the rows with more than kTcList core entries (one per lane: 752 us
 // at R-MAT scale 19, 811 with 128) of the highest ranks; the entries of other
 // rows are tested one by one against N+(a)'s bitmap in LDS.
 // Bound: vector instructions (about 25 per bitmap) and the L2 reads of the
